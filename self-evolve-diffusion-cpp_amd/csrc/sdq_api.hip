@@ -81,8 +81,8 @@ struct Workspace {
   size_t rinv_bytes = 0;
   char* grp = nullptr;  // sdq_qlinear_group's per-item scratch
   size_t grp_bytes = 0;
-  float* sdpa_part = nullptr;  // attention key splits' partial outputs and states
-  size_t sdpa_part_bytes = 0;
+  float* sdpa = nullptr;  // attention: packed K and V, shares' partial outputs
+  size_t sdpa_bytes = 0;
 };
 std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
 
@@ -1774,14 +1774,19 @@ int sdq_sdpa_batched(const float* q, int64_t ldq, const float* k, int64_t ldk, c
   if ((rc = ensure_device(dev))) return rc;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int cu_count = g_dev[dev].cu_count;
-  float* part = nullptr;
-  const int64_t pf = sdpa_part_floats(Lq, Lk, heads, batch, cu_count);
-  if (pf > 0 && (rc = ws_floats(dev, s, &Workspace::sdpa_part, &Workspace::sdpa_part_bytes,
-                                (size_t)pf * sizeof(float), &part)))
-    return rc;
+  // The packed form when its scratch can be had (at most 2 GiB, see
+  // sdpa_packed_bytes), else the form without scratch: an attention call is
+  // not refused for want of memory, under graph capture either.
+  float* scratch = nullptr;
+  const int64_t need = sdpa_packed_bytes(Lq, Lk, heads, batch, cu_count);
+  if (need > 0 && ws_floats(dev, s, &Workspace::sdpa, &Workspace::sdpa_bytes, (size_t)need,
+                            &scratch) != SDQ_OK)
+    scratch = nullptr;
   hipEvent_t p0 = t_prof ? prof_mark(s) : nullptr;
-  hipError_t e = launch_sdpa(q, ldq, k, ldk, v, ldv, out, ldo, Lq, Lk, heads, s, batch, part,
-                             cu_count);
+  const hipError_t e =
+      scratch ? launch_sdpa_packed(q, ldq, k, ldk, v, ldv, out, ldo, Lq, Lk, heads, s, batch,
+                                   scratch, cu_count)
+              : launch_sdpa(q, ldq, k, ldk, v, ldv, out, ldo, Lq, Lk, heads, s, batch);
   if (e != hipSuccess) {
     drop_events({p0});
     return hip_error(e, "sdpa launch");

@@ -1,0 +1,719 @@
+// Scaled dot-product attention over packed keys and values (gfx950), the
+// form of sdq_sdpa that has scratch memory (src/model/blocks.cpp:112-199,
+// non-causal, head_dim 128): every fp32 product as three fp16 MFMA products
+// of power-of-two-scaled parts (x = hi + lo; hi.hi + hi.lo + lo.hi, ~2^-22
+// relative), an online softmax, fp32 accumulation. Its error against float64
+// is below that of the form without scratch (sdq_glue.hip, whose P.V is split
+// into bf16 parts): 2.0e-6 against 4.8e-6 of the output's norm at 27280
+// tokens, 3.5e-7 against 3.8e-6 at 157 queries x 768 keys.
+//
+// What bounds it: the matrix cores, and with random operands their power
+// (12 Lq Lk 128 operations per head; a library bf16 GEMM reaches 1.37 PFLOP/s
+// on this card, a bare loop of these MFMAs with the same LDS reads 1.66). The
+// other form splits and transposes every K / V block again for each 256
+// queries, a third of its VALU work; here one pass does it once, in the order
+// the MFMAs read, so that LDS-DMAs move the blocks as they are and the loop
+// holds MFMAs, LDS reads and the softmax only. 27280^2, 24 heads: 30.2 ms
+// without, 19.3-19.7 ms with it (0.24 ms of that the packing); MFMAs 16x16x32:
+// 32x32x16 ones took 20.7 ms (fewer accumulator bits switch, a higher clock).
+#include "sdq_internal.h"
+#include "sdq_device.h"
+
+#include <cstdlib>
+
+#pragma clang fp contract(off)
+
+namespace sdq {
+namespace {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+constexpr int kHd = 128;             // head dim
+constexpr int kKB = 32;              // keys per block
+constexpr int kRec = 32768;          // bytes of a packed block: K parts, V parts
+constexpr int kRecV = 16384;         // V's offset in it
+constexpr int kPart = 8192;          // one part (hi or lo) of K or V
+constexpr int kWaves = 8;
+constexpr int kQ = 32 * kWaves;      // queries per workgroup
+constexpr int kRing = 4;             // blocks of K and of V in LDS
+// K and Q are scaled by powers of two so that the largest element of a key
+// block (of a query row) lies in [2^14, 2^15): their fp16 low parts then stay
+// normal numbers down to 2^-18 of it.
+constexpr int kTop = 15;
+constexpr int kZeroV = 1 << 20;      // "exponent" of a V block of zeros
+// V's exponents stop here (a V block all below 2^-95 then holds smaller
+// numbers) and the sums l are kept as l 2^-16: l ~ 2^(15 - e_v) stays a normal
+// float over all exponents.
+constexpr int kMinV = -110;
+constexpr int kSumExp = 16;
+
+// The exponent that scales a largest magnitude into [2^14, 2^15) (x = 0: any)
+__device__ __forceinline__ int top_exp(float x) {
+  return (x > 0.f ? __builtin_amdgcn_frexp_expf(x) : 0) - kTop;
+}
+// max(m, |x|) over finite x: an infinity or NaN reaches its own products only
+__device__ __forceinline__ float amax_finite(float m, float x) {
+  const float a = fabsf(x);
+  return a <= 3.402823466e38f ? fmaxf(m, a) : m;
+}
+
+// max / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 of a query, in all
+// of them
+template <class F>
+__device__ __forceinline__ float quad16(float v, F f) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float quad16_max(float v) {
+  return quad16(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float quad16_sum(float v) {
+  return quad16(v, [](float a, float b) { return a + b; });
+}
+
+// One workgroup per (key block, head, sequence): K scaled by the block's
+// power of two and split into fp16 parts, V split into bf16 parts, both in
+// the order the MFMA operands are read (16 bytes per lane):
+//   K [part][32-dim step d][16-key tile kt][lane]: key 16 kt + lane % 16,
+//     dims 32 d + 8 (lane / 16) + 0..7
+//   V [part][16-dim tile dt][lane]: dim 16 dt + lane % 16, keys
+//     16 (m / 4) + 4 (lane / 16) + m % 4, m = 0..7
+// Keys past Lk are zeros. HBM-bound: 8 bytes read and 8 written per (key,
+// dim) pair of K and V.
+__global__ void __launch_bounds__(256)
+sdpa_pack_kernel(const float* __restrict__ K, int64_t ldk, const float* __restrict__ V,
+                 int64_t ldv, int64_t Lk, int nkb, char* __restrict__ packed,
+                 int2* __restrict__ exps) {
+  __shared__ __attribute__((aligned(16))) char buf[kRec];
+  __shared__ float red[2][4];
+  const int t = threadIdx.x;
+  const int kb = blockIdx.x, head = blockIdx.y;
+  const int64_t seq = blockIdx.z;
+  const int64_t rec = (seq * gridDim.y + head) * nkb + kb;
+  const float* kp = K + seq * Lk * ldk + (int64_t)head * kHd;
+  const float* vp = V + seq * Lk * ldv + (int64_t)head * kHd;
+  // 4 dims (float4 q4 of a row) of 4 keys each: K's keys 8 i + r, V's 4 r + i
+  const int q4 = t & 31, r = t >> 5;
+  float4 a[4];
+  float v[4][4], mk = 0.f, mv = 0.f;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int64_t kr = (int64_t)kb * kKB + 8 * i + r, vr = (int64_t)kb * kKB + 4 * r + i;
+    a[i] = kr < Lk ? *reinterpret_cast<const float4*>(kp + kr * ldk + 4 * q4)
+                   : float4{0.f, 0.f, 0.f, 0.f};
+    const float4 x = vr < Lk ? *reinterpret_cast<const float4*>(vp + vr * ldv + 4 * q4)
+                             : float4{0.f, 0.f, 0.f, 0.f};
+    v[i][0] = x.x, v[i][1] = x.y, v[i][2] = x.z, v[i][3] = x.w;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    mk = amax_finite(amax_finite(mk, a[i].x), a[i].y);
+    mk = amax_finite(amax_finite(mk, a[i].z), a[i].w);
+#pragma unroll
+    for (int c = 0; c < 4; c++) mv = amax_finite(mv, v[i][c]);
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2)
+    mk = fmaxf(mk, __shfl_xor(mk, d)), mv = fmaxf(mv, __shfl_xor(mv, d));
+  if ((t & 63) == 0) red[0][t >> 6] = mk, red[1][t >> 6] = mv;
+  __syncthreads();
+  mk = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+  mv = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
+  const int ek = top_exp(mk), ev = top_exp(mv) < kMinV ? kMinV : top_exp(mv);
+  if (t == 0) exps[rec] = int2{ek, mv == 0.f ? kZeroV : ev};
+  auto put = [&](char* p, const float y0, const float y1, const float y2, const float y3) {
+    const v4h hi = {(_Float16)y0, (_Float16)y1, (_Float16)y2, (_Float16)y3};
+    const v4h lo = {(_Float16)(y0 - (float)hi.x), (_Float16)(y1 - (float)hi.y),
+                    (_Float16)(y2 - (float)hi.z), (_Float16)(y3 - (float)hi.w)};
+    *reinterpret_cast<v4h*>(p) = hi;
+    *reinterpret_cast<v4h*>(p + kPart) = lo;
+  };
+  // The record is put together in LDS and copied out whole. Its 16-byte
+  // lane slots are XORed within each 256 bytes (swz) so that the lanes of a
+  // wave, which hold different dims of one key, write to different banks.
+  auto swz = [](int chunk, int slot) {
+    return chunk * 1024 + (slot & 48) * 16 + ((slot & 15) ^ ((slot >> 4) * 4 + (chunk >> 1 & 3))) * 16;
+  };
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int key = 8 * i + r;
+    put(buf + swz((q4 >> 3) * 2 + (key >> 4), (q4 >> 1 & 3) * 16 + (key & 15)) + (q4 & 1) * 8,
+        ldexpf(a[i].x, -ek), ldexpf(a[i].y, -ek), ldexpf(a[i].z, -ek), ldexpf(a[i].w, -ek));
+  }
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    const int d = 4 * q4 + c;
+    put(buf + kRecV + swz(d >> 4, (r & 3) * 16 + (d & 15)) + (r >> 2) * 8, ldexpf(v[0][c], -ev),
+        ldexpf(v[1][c], -ev), ldexpf(v[2][c], -ev), ldexpf(v[3][c], -ev));
+  }
+  __syncthreads();
+  char* dst = packed + rec * kRec;
+#pragma unroll
+  for (int i = 0; i < kRec / 4096; i++) {
+    const int u = i * 256 + t;  // 16-byte slot of the record
+    *reinterpret_cast<uint4*>(dst + u * 16) = *reinterpret_cast<const uint4*>(
+        buf + (u >> 9) * kPart + swz(u >> 6 & 7, u & 63));
+  }
+}
+
+// How a sequence's items (256 queries of one head, all its key blocks) are
+// spread over workgroups. The first nfull items, whole rounds of the CUs, run
+// whole. The others, which would fill only part of a round, are cut by keys
+// into `splits` shares of kbs blocks (splits = 1: not cut); a share leaves its
+// unnormalized output and its (reference, sum) pair in slot (item - nfull) *
+// splits + share, and sdpa_combine_kernel adds up an item's shares.
+struct Plan {
+  int nkb;      // key blocks
+  int qgroups;  // items per head
+  int items;    // heads * qgroups
+  int nfull;
+  int splits;
+  int kbs;
+};
+struct Parts {
+  float* o;    // [seq][slots][256][128]
+  float2* ml;  // [seq][slots][256]: (reference, sum), base 2
+};
+
+// One MFMA operand of a lane as its high and low parts.
+struct Frag {
+  uint4 hi, lo;
+};
+__device__ __forceinline__ v4f mfma_h(const uint4& a, const v8h& b, const v4f& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), b, c, 0, 0, 0);
+}
+// o / l from a sum kept as l 2^-kSumExp, its exponent applied last (1 / l
+// itself may be subnormal)
+struct Inv {
+  float r;
+  int e;
+  __device__ __forceinline__ explicit Inv(float l)
+      : r(1.f / __builtin_amdgcn_frexp_mantf(l)), e(-__builtin_amdgcn_frexp_expf(l) - kSumExp) {}
+  __device__ __forceinline__ float operator()(float o) const { return ldexpf(o * r, e); }
+};
+
+// Keeps a value's computation where it is written (the compiler would sink it
+// past the barrier to its use).
+template <class T>
+__device__ __forceinline__ void pin(T& v) {
+  asm volatile("" : "+v"(v));
+}
+
+__global__ void __launch_bounds__(kWaves * 64)
+sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restrict__ packed,
+                   const int2* __restrict__ exps, float* __restrict__ O, int64_t ldo, int64_t Lq,
+                   int64_t Lk, Plan plan, float scale_log2e, Parts parts) {
+  constexpr int QT = 2;            // 16-query tiles per wave
+  constexpr int LD = 16 / kWaves;  // a wave's DMAs of one K or V block
+  __shared__ __attribute__((aligned(16))) char lds[kRing * kRec];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 15, h = lane >> 4;
+  const int64_t seq = blockIdx.y;
+  const float* Qs = Q + seq * Lq * ldq;
+  float* Os = O + seq * Lq * ldo;
+  const int nkb = plan.nkb;
+
+  // This workgroup's item and key range: consecutive items on one XCD
+  // (workgroup b runs on XCD b % 8), so its CUs walk the same head's blocks
+  // and share them in the XCD's L2.
+  int item, kb0 = 0, kb1 = nkb, slot = -1;
+  {
+    const bool whole = (int)blockIdx.x < plan.nfull;
+    const int c = whole ? blockIdx.x : blockIdx.x - plan.nfull;
+    const int total = whole ? plan.nfull : (plan.items - plan.nfull) * plan.splits;
+    const int x = c & 7, q8 = total >> 3, r8 = total & 7;
+    item = x * q8 + (x < r8 ? x : r8) + (c >> 3);
+    if (!whole) {
+      if (plan.splits > 1) slot = item;
+      kb0 = item % plan.splits * plan.kbs;
+      kb1 = kb0 + plan.kbs < nkb ? kb0 + plan.kbs : nkb;
+      item = plan.nfull + item / plan.splits;
+    }
+  }
+
+  const uint32_t lane16 = (uint32_t)lane * 16u;
+  const char* ldsp = lds + lane16;
+  const uint32_t ldsw =
+      __builtin_amdgcn_readfirstlane(dev::lds_addr32(lds)) + (uint32_t)(w * LD) * 1024u;
+  const uint32_t voff = lane16 + (uint32_t)(w * LD) * 1024u;
+  const int head = item / plan.qgroups, qg = item - head * plan.qgroups;
+  const int64_t q0 = (int64_t)qg * kQ + w * (16 * QT);
+  const int64_t col = (int64_t)head * kHd;
+  const int64_t rec0 = (seq * (plan.items / plan.qgroups) + head) * nkb;
+  const int2* ex = exps + rec0;
+
+  // This wave's DMAs: LD of the 16 KB-chunks of K(i) or V(i) (block kb0 + i)
+  // into ring slot i % kRing; blocks past the range repeat the last one
+  // (never used).
+  const dev::v4u rs = dev::raw_rsrc(packed + rec0 * kRec, (uint32_t)nkb * (uint32_t)kRec);
+  auto soff = [&](int i) { return (uint32_t)(kb0 + i < kb1 ? kb0 + i : kb1 - 1) * kRec; };
+  auto slot_k = [&](int i) { return ldsw + (uint32_t)(i & (kRing - 1)) * kRecV; };
+  auto slot_v = [&](int i) { return ldsw + (uint32_t)(kRing + (i & (kRing - 1))) * kRecV; };
+  auto issue_k = [&](int i) {
+#pragma unroll
+    for (int c = 0; c < LD; c++)
+      dev::dma16<0>(rs, voff, soff(i) + c * 1024u, slot_k(i) + c * 1024u);
+  };
+  auto issue_v = [&](int i) {
+#pragma unroll
+    for (int c = 0; c < LD; c++)
+      dev::dma16<0>(rs, voff, soff(i) + kRecV + c * 1024u, slot_v(i) + c * 1024u);
+  };
+  issue_k(0), issue_v(0), issue_k(1), issue_v(1), issue_k(2), issue_v(2), issue_k(3);
+  // The query rows, lane (j, h): dims 32 d + 8 h + 0..7 of query 16 t + j,
+  // scaled by 2^-eq and split into fp16 parts
+  v8h qh[QT][4], ql[QT][4];
+  int eq[QT];
+#pragma unroll
+  for (int t = 0; t < QT; t++) {
+    const int64_t qi = q0 + 16 * t + j;
+    const float* src = Qs + (qi < Lq ? qi : 0) * ldq + col + 8 * h;  // past Lq: not stored
+    float4 qr[8];
+    float mq = 0.f;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      qr[c] = *reinterpret_cast<const float4*>(src + 32 * (c >> 1) + 4 * (c & 1));
+      mq = amax_finite(amax_finite(mq, qr[c].x), qr[c].y);
+      mq = amax_finite(amax_finite(mq, qr[c].z), qr[c].w);
+    }
+    eq[t] = top_exp(quad16_max(mq));
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+      const float x[8] = {qr[2 * d].x,     qr[2 * d].y,     qr[2 * d].z,     qr[2 * d].w,
+                          qr[2 * d + 1].x, qr[2 * d + 1].y, qr[2 * d + 1].z, qr[2 * d + 1].w};
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const float y = ldexpf(x[e], -eq[t]);
+        qh[t][d][e] = (_Float16)y;
+        ql[t][d][e] = (_Float16)(y - (float)qh[t][d][e]);
+      }
+    }
+  }
+  // a V block of zeros takes the smallest exponent of the others
+  int vmin = kZeroV;
+  for (int k = lane; k < nkb; k += 64) vmin = min(vmin, ex[k].y);
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) vmin = min(vmin, __shfl_xor(vmin, d));
+  vmin = vmin == kZeroV ? 0 : vmin;
+  // exponents of 64 key blocks at a time, one block per lane
+  int2 ev;
+  auto load_ev = [&](int i) {
+    const int k = kb0 + i + lane;
+    ev = ex[k < nkb ? k : nkb - 1];
+    if (ev.y == kZeroV) ev.y = vmin;
+  };
+  load_ev(0);
+  auto kfrag = [&](int i, int c) {
+    const char* p = ldsp + (i & (kRing - 1)) * kRecV + c * 1024;
+    return Frag{*reinterpret_cast<const uint4*>(p), *reinterpret_cast<const uint4*>(p + kPart)};
+  };
+  auto vfrag = [&](int i, int c) {
+    const char* p = ldsp + (kRing + (i & (kRing - 1))) * kRecV + c * 1024;
+    return Frag{*reinterpret_cast<const uint4*>(p), *reinterpret_cast<const uint4*>(p + kPart)};
+  };
+  // scores of a block: S^T tile [kt][t], keys 16 kt + 4 h + r of query 16 t + j
+  struct Scores {
+    v4f s[2][QT];
+  };
+  v4f acc[8][QT];  // O^T tile [dt][t]: dims 16 dt + 4 h + r of query 16 t + j
+#pragma unroll
+  for (int d = 0; d < 8; d++)
+#pragma unroll
+    for (int t = 0; t < QT; t++) acc[d][t] = v4f{};
+  // R: the reference exponent of a query; P = 2^(s + e_v - R) with the base-2
+  // logit s and V's block exponent e_v, so that P V~ (V~ = V 2^-e_v) sums to
+  // 2^-R sum 2^s V, and l = 2^-R sum 2^s. R follows max(s + e_v), kept in
+  // [R + 7, R + 15]: P is then at most 2^15, its fp16 parts keep 22 bits down
+  // to 2^-10 of the largest P V~ so far (and an absolute 2^-32 of it below),
+  // and the accumulators are rarely rescaled.
+  float R[QT], lsum[QT], sq[QT], off[QT];
+#pragma unroll
+  for (int t = 0; t < QT; t++) R[t] = -INFINITY, lsum[t] = 0.f;
+  const int n = kb1 - kb0;
+  // the partial block, if this range ends with it (else never reached)
+  const int rem = (int)(Lk % kKB);
+  const int last = rem && kb1 == nkb ? n - 1 : -1;
+  auto mask = [&](Scores& sc) {
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (16 * kt + 4 * h + r >= rem)
+#pragma unroll
+          for (int t = 0; t < QT; t++) sc.s[kt][t][r] = -INFINITY;
+  };
+  auto max4 = [&](float x, const v4f& v) {
+    x = fmaxf(fmaxf(x, v[0]), v[1]);
+    return fmaxf(fmaxf(x, v[2]), v[3]);
+  };
+  auto raise = [&](const float* mb, float e) {
+#pragma unroll
+    for (int t = 0; t < QT; t++) {
+      const bool u = mb[t] > R[t] + 15.f;
+      const float rn = u ? mb[t] - 7.f : R[t];
+      const float alpha = u ? __builtin_amdgcn_exp2f(R[t] - rn) : 1.f;
+      R[t] = rn;
+      off[t] = e - rn;
+      lsum[t] *= alpha;
+#pragma unroll
+      for (int d = 0; d < 8; d++) acc[d][t] *= alpha;
+    }
+  };
+
+  // -1 the compiler does not know, so that x - hi stays a multiply-add that
+  // reads hi as fp16 and writes fp16 (one instruction per low part)
+  float neg1 = -1.f;
+  asm volatile("" : "+s"(neg1));
+  Frag fr[4];
+  // K(0) has landed (newer DMAs may be in flight), then V(0) and K(1)
+  __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(6 * LD));
+  asm volatile("s_barrier" ::: "memory");
+  Scores st, st2;
+#pragma unroll
+  for (int c = 0; c < 8; c++) {
+    const int d = c >> 1, kt = c & 1;
+    const Frag f = kfrag(0, c);
+#pragma unroll
+    for (int t = 0; t < QT; t++) st.s[kt][t] = mfma_h(f.hi, qh[t][d], d ? st.s[kt][t] : v4f{});
+#pragma unroll
+    for (int t = 0; t < QT; t++) st.s[kt][t] = mfma_h(f.hi, ql[t][d], st.s[kt][t]);
+#pragma unroll
+    for (int t = 0; t < QT; t++) st.s[kt][t] = mfma_h(f.lo, qh[t][d], st.s[kt][t]);
+  }
+  if (last == 0) mask(st);
+  {
+    float mb[QT];
+#pragma unroll
+    for (int t = 0; t < QT; t++) {
+      sq[t] = ldexpf(scale_log2e, eq[t] + __builtin_amdgcn_readlane(ev.x, 0));
+      mb[t] = fmaf(quad16_max(max4(max4(-INFINITY, st.s[0][t]), st.s[1][t])), sq[t],
+                   (float)__builtin_amdgcn_readlane(ev.y, 0));
+    }
+    raise(mb, (float)__builtin_amdgcn_readlane(ev.y, 0));
+  }
+  __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(4 * LD) & ~(15 << 8));
+  asm volatile("s_barrier" ::: "memory");
+  issue_k(4);
+  fr[0] = kfrag(1, 0);
+  fr[1] = kfrag(1, 1);
+
+  // Block i, whose scores sc, scale sq and offset off = e_v - R are known: the next
+  // block's scores on the matrix cores beside this block's exponentials,
+  // then P.V beside the next block's maximum. Every group of MFMAs is fenced
+  // with its share of the other work, and operands are read two steps
+  // ahead, so the MFMA pipe does not wait for either.
+  auto step = [&](int i, const Scores& sc, Scores& nx) {
+    v8h ph[QT], pl[QT];
+    uint32_t* phw = reinterpret_cast<uint32_t*>(ph);
+    uint32_t* plw = reinterpret_cast<uint32_t*>(pl);
+    float x0[QT / 2], x1[QT / 2], ps[QT];
+#pragma unroll
+    for (int t = 0; t < QT; t++) ps[t] = 0.f;
+    const int e_v = __builtin_amdgcn_readlane(ev.y, i & 63);
+    // pair u of step c: elements 2 e, 2 e + 1 (of 8) of query tile t
+    auto elem = [&](int c, int u, int k, int& t, int& e) {
+      const int pi = c * (QT / 2) + u;
+      t = pi >> 2, e = pi & 3;
+      return __builtin_amdgcn_exp2f(fmaf(sc.s[e >> 1][t][2 * (e & 1) + k], sq[t], off[t]));
+    };
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      const int d = c >> 1, kt = c & 1;
+      const Frag f = fr[c & 3];
+      fr[(c + 2) & 3] = c + 2 < 8 ? kfrag(i + 1, c + 2) : vfrag(i, c + 2 - 8);
+      int t0, e0;
+#pragma unroll
+      for (int t = 0; t < QT; t++)
+        nx.s[kt][t] = mfma_h(f.hi, qh[t][d], d ? nx.s[kt][t] : v4f{});
+#pragma unroll
+      for (int u = 0; u < QT / 2; u++) {
+        x0[u] = elem(c, u, 0, t0, e0);
+        pin(x0[u]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < QT; t++) nx.s[kt][t] = mfma_h(f.hi, ql[t][d], nx.s[kt][t]);
+#pragma unroll
+      for (int u = 0; u < QT / 2; u++) {
+        x1[u] = elem(c, u, 1, t0, e0);
+        ps[t0] += x0[u];
+        pin(x1[u]), pin(ps[t0]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < QT; t++) nx.s[kt][t] = mfma_h(f.lo, qh[t][d], nx.s[kt][t]);
+#pragma unroll
+      for (int u = 0; u < QT / 2; u++) {
+        const int pi = c * (QT / 2) + u;
+        ps[pi >> 2] += x1[u];
+        // P = fp16 hi + fp16 lo, two keys per dword
+        uint32_t hw = __builtin_bit_cast(uint32_t, v2h{(_Float16)x0[u], (_Float16)x1[u]});
+        pin(hw);  // the low parts then read its halves
+        const v2h hi = __builtin_bit_cast(v2h, hw);
+        const v2h lo = {(_Float16)__builtin_fmaf((float)hi.x, neg1, x0[u]),
+                        (_Float16)__builtin_fmaf((float)hi.y, neg1, x1[u])};
+        phw[pi] = hw;
+        plw[pi] = __builtin_bit_cast(uint32_t, lo);
+        pin(plw[pi]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // own DMAs of V(i+1) and K(i+2) have landed; after the barrier
+    // everyone's have, and K(i+1), V(i-1) have been read by all
+    __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(3 * LD));
+    asm volatile("s_barrier" ::: "memory");
+    if (i + 1 == last) mask(nx);
+    const int i1 = i + 1;
+    if ((i1 & 63) == 0) load_ev(i1);
+    const uint32_t sv = soff(i + 3) + kRecV, sk = soff(i + 5);
+    const uint32_t dv = slot_v(i + 3), dk = slot_k(i + 5);
+    float ml[QT], vx = 0.f;
+    int kx = 0;
+    bool up = false;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      const Frag f = fr[c & 3];
+      fr[(c + 2) & 3] = c + 2 < 8 ? vfrag(i, c + 2) : kfrag(i + 2, c + 2 - 8);
+      // O^T += V^T . P^T: V_hi.P_hi + V_hi.P_lo + V_lo.P_hi
+#pragma unroll
+      for (int t = 0; t < QT; t++) acc[c][t] = mfma_h(f.hi, ph[t], acc[c][t]);
+      // LD DMAs of V, then LD of K: LD / 2 of either per step
+      if (c < 4) {
+#pragma unroll
+        for (int u = 0; u < LD / 2; u++) {
+          const uint32_t o = (uint32_t)((c & 1) * (LD / 2) + u) * 1024u;
+          dev::dma16<0>(rs, voff, (c < 2 ? sv : sk) + o, (c < 2 ? dv : dk) + o);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < QT; t++) acc[c][t] = mfma_h(f.hi, pl[t], acc[c][t]);
+      if (c >= 2 && c < 4) {
+#pragma unroll
+        for (int t = 0; t < QT; t++) {
+          ml[t] = max4(c == 2 ? -INFINITY : ml[t], nx.s[c - 2][t]);
+          pin(ml[t]);
+        }
+      }
+      if (c == 1) {
+#pragma unroll
+        for (int t = 0; t < QT; t++) {
+          lsum[t] += ldexpf(ps[t], -kSumExp - e_v);
+          pin(lsum[t]);
+        }
+      }
+      if (c == 4) {
+        kx = __builtin_amdgcn_readlane(ev.x, i1 & 63);
+        vx = (float)__builtin_amdgcn_readlane(ev.y, i1 & 63);
+#pragma unroll
+        for (int t = 0; t < QT; t++) {
+          sq[t] = ldexpf(scale_log2e, eq[t] + kx);
+          pin(sq[t]);
+        }
+      }
+      if (c == 6) {
+#pragma unroll
+        for (int t = 0; t < QT; t++) {
+          up = up || ml[t] > R[t] + 15.f;
+          off[t] = vx - R[t];
+          pin(off[t]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < QT; t++) acc[c][t] = mfma_h(f.lo, ph[t], acc[c][t]);
+      if (c == 5) {
+#pragma unroll
+        for (int t = 0; t < QT; t++) {
+          ml[t] = fmaf(quad16_max(ml[t]), sq[t], vx);
+          pin(ml[t]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (i1 < n && __any(up)) raise(ml, vx);  // (past the end: a repeated block)
+  };
+  int i = 0;
+  for (; i + 1 < n; i += 2) {
+    step(i, st, st2);
+    step(i + 1, st2, st);
+  }
+  if (i < n) step(i, st, st2);
+
+  const int64_t nslots = (int64_t)(plan.items - plan.nfull) * plan.splits;
+#pragma unroll
+  for (int t = 0; t < QT; t++) {
+    const float ltot = quad16_sum(lsum[t]);
+    const int64_t qi = q0 + 16 * t + j;
+    if (slot >= 0) {
+      const int64_t row = (seq * nslots + slot) * kQ + w * (16 * QT) + 16 * t + j;
+      float* dst = parts.o + row * kHd + 4 * h;
+#pragma unroll
+      for (int d = 0; d < 8; d++) *reinterpret_cast<v4f*>(dst + 16 * d) = acc[d][t];
+      if (h == 0) parts.ml[row] = float2{R[t], ltot};
+    } else if (qi < Lq) {
+      const Inv inv(ltot);
+      float* dst = Os + qi * ldo + col + 4 * h;
+#pragma unroll
+      for (int d = 0; d < 8; d++)
+        *reinterpret_cast<v4f*>(dst + 16 * d) =
+            v4f{inv(acc[d][t][0]), inv(acc[d][t][1]), inv(acc[d][t][2]), inv(acc[d][t][3])};
+    }
+  }
+  // the repeated blocks' DMAs must land before the LDS is given back
+  __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(0));
+}
+
+// An item's shares combined: out = sum_s w_s o_s / sum_s w_s l_s, w_s =
+// 2^(R_s - max R). One thread per 4 dims of a query.
+__global__ void __launch_bounds__(256)
+sdpa_combine_kernel(Plan plan, Parts parts, int64_t Lq, float* __restrict__ O, int64_t ldo) {
+  const int it = blockIdx.x;  // item nfull + it
+  const int64_t seq = blockIdx.z;
+  const int q = blockIdx.y * 8 + (threadIdx.x >> 5), d = 4 * (threadIdx.x & 31);
+  const int item = plan.nfull + it;
+  const int head = item / plan.qgroups, qg = item - head * plan.qgroups;
+  const int64_t qi = (int64_t)qg * kQ + q;
+  if (qi >= Lq) return;
+  const int S = plan.splits;
+  const int64_t row = (seq * (plan.items - plan.nfull) + it) * S * kQ + q;
+  const float2* ml = parts.ml + row;
+  const float* op = parts.o + row * kHd + d;
+  float mx = -INFINITY;
+  for (int s = 0; s < S; s++) mx = fmaxf(mx, ml[s * kQ].x);
+  float lt = 0.f;
+  float4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < S; s++) {
+    const float2 m = ml[s * kQ];
+    const float wt = __builtin_amdgcn_exp2f(m.x - mx);
+    lt += wt * m.y;
+    const float4 v = *reinterpret_cast<const float4*>(op + (int64_t)s * kQ * kHd);
+    o.x += wt * v.x;
+    o.y += wt * v.y;
+    o.z += wt * v.z;
+    o.w += wt * v.w;
+  }
+  const Inv inv(lt);
+  *reinterpret_cast<float4*>(O + (seq * Lq + qi) * ldo + (int64_t)head * kHd + d) =
+      float4{inv(o.x), inv(o.y), inv(o.z), inv(o.w)};
+}
+
+// Depends on the sequence only, not on the batch, so stacked and separate
+// calls give the same bits.
+Plan make_plan(int64_t Lq, int64_t Lk, int heads, int cu_count) {
+  Plan p{};
+  p.nkb = (int)ceil_div(Lk, kKB);
+  p.qgroups = (int)ceil_div(Lq, kQ);
+  p.items = heads * p.qgroups;
+  p.splits = 1;
+  p.kbs = p.nkb;
+  const int cus = cu_count > 0 ? cu_count : 256;
+  p.nfull = p.items / cus * cus;
+  const int rest = p.items - p.nfull;
+  if (rest == 0 || std::getenv("SDQ_SDPA_SPLIT")) {  // the variable: comparisons without shares
+    p.nfull = p.items;
+    return p;
+  }
+  // The cut that ends first, in key-block times: rounds of shares, each with
+  // its own start and end (about 3 blocks), plus the second pass over the
+  // partial outputs.
+  double best = p.nkb + 3;
+  for (int S = 2; S <= 32 && 3 * S <= p.nkb; S++) {
+    const int kbs = (int)ceil_div(p.nkb, S);
+    if (ceil_div(p.nkb, kbs) != S) continue;  // no empty share
+    const double cost = (double)ceil_div((int64_t)rest * S, cus) * (kbs + 3) + 3;
+    if (cost < best) best = cost, p.splits = S, p.kbs = kbs;
+  }
+  return p;
+}
+
+int64_t pad256(int64_t n) { return (n + 255) / 256 * 256; }
+
+// Scratch of one launch over `heads` heads of `batch` sequences.
+struct Layout {
+  int64_t exps, o, ml, bytes;  // offsets of its parts (the records lie at 0)
+};
+Layout layout(const Plan& p, int64_t heads, int64_t batch) {
+  const int64_t recs = batch * heads * p.nkb;
+  const int64_t rows =
+      p.splits > 1 ? batch * (p.items - p.nfull) * p.splits * (int64_t)kQ : 0;
+  Layout l;
+  l.exps = recs * kRec;
+  l.o = l.exps + pad256(recs * 8);
+  l.ml = l.o + rows * kHd * 4;
+  l.bytes = l.ml + rows * 8;
+  return l;
+}
+
+// A call runs in launches of as many sequences, or of as many heads of one
+// sequence, as keep their records within kMaxRecs bytes, so the scratch a
+// stream holds is bounded (heads: a sequence's own share, so that it does
+// not depend on the batch).
+constexpr int64_t kMaxRecs = int64_t(1) << 31;
+struct Chunk {
+  int heads, seqs;
+};
+Chunk chunk(int64_t nkb, int heads, int batch) {
+  const int64_t per_head = nkb * kRec;
+  const int64_t h = kMaxRecs / per_head < 1 ? 1 : kMaxRecs / per_head;
+  if (h < heads) return {(int)h, 1};
+  const int64_t n = kMaxRecs / (per_head * heads);
+  return {heads, (int)(n < batch ? n : batch)};
+}
+
+}  // namespace
+
+int64_t sdpa_packed_bytes(int64_t Lq, int64_t Lk, int heads, int batch, int cu_count) {
+  // a head's records are addressed with 32-bit offsets; a grid holds 2^32 threads
+  if (Lk > kMaxRecs / kRec * kKB || heads > 65535 || ceil_div(Lq, kQ) * heads > (1 << 22))
+    return 0;
+  const Chunk c = chunk(ceil_div(Lk, kKB), heads, batch);
+  return layout(make_plan(Lq, Lk, c.heads, cu_count), c.heads, c.seqs).bytes;
+}
+
+hipError_t launch_sdpa_packed(const float* q, int64_t ldq, const float* k, int64_t ldk,
+                              const float* v, int64_t ldv, float* out, int64_t ldo, int64_t Lq,
+                              int64_t Lk, int heads, hipStream_t s, int batch, void* scratch,
+                              int cu_count) {
+  if (Lq <= 0 || batch <= 0) return hipSuccess;
+  if (Lk <= 0 || heads <= 0 || heads > 65535 || batch > 65535 || !scratch)
+    return hipErrorInvalidValue;
+  const float scale_log2e = (1.f / sqrtf((float)kHd)) * 1.4426950408889634f;
+  const Chunk ch = chunk(ceil_div(Lk, kKB), heads, batch);
+  char* packed = static_cast<char*>(scratch);
+  for (int b0 = 0; b0 < batch; b0 += ch.seqs)
+    for (int h0 = 0; h0 < heads; h0 += ch.heads) {
+      const int nb = batch - b0 < ch.seqs ? batch - b0 : ch.seqs;
+      const int nh = heads - h0 < ch.heads ? heads - h0 : ch.heads;
+      const Plan p = make_plan(Lq, Lk, nh, cu_count);
+      const Layout l = layout(p, nh, nb);
+      int2* exps = reinterpret_cast<int2*>(packed + l.exps);
+      const Parts parts{reinterpret_cast<float*>(packed + l.o),
+                        reinterpret_cast<float2*>(packed + l.ml)};
+      const int64_t col = (int64_t)h0 * kHd;
+      const float* qb = q + b0 * Lq * ldq + col;
+      float* ob = out + b0 * Lq * ldo + col;
+      hipLaunchKernelGGL(sdpa_pack_kernel, dim3((unsigned)p.nkb, (unsigned)nh, (unsigned)nb),
+                         dim3(256), 0, s, k + b0 * Lk * ldk + col, ldk, v + b0 * Lk * ldv + col,
+                         ldv, Lk, p.nkb, packed, exps);
+      const int64_t shares = (int64_t)(p.items - p.nfull) * p.splits;
+      hipLaunchKernelGGL(sdpa_packed_kernel, dim3((unsigned)(p.nfull + shares), (unsigned)nb),
+                         dim3(kWaves * 64), 0, s, qb, ldq, packed, exps, ob, ldo, Lq, Lk, p,
+                         scale_log2e, parts);
+      if (p.splits > 1)
+        hipLaunchKernelGGL(sdpa_combine_kernel,
+                           dim3((unsigned)(p.items - p.nfull), kQ / 8, (unsigned)nb), dim3(256),
+                           0, s, p, parts, Lq, ob, ldo);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
+  return hipSuccess;
+}
+
+}  // namespace sdq

@@ -1,0 +1,143 @@
+"""sdq_sdpa's packed form at the edges of its key blocks (32), query groups
+(256) and key shares, over V's element range, in chunks, and the form without
+scratch under graph capture. Bound: 2e-5 of the output scale (the parity bound
+of the attention against the oracle), or per output dimension where V's
+magnitudes differ."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(sdq_dev, q, kv, heads, batch=1):
+    import torch
+
+    import sdq
+
+    out = torch.full((q.shape[0], heads * 128), float("nan"), device=sdq_dev)
+    sdq.sdpa(q, kv, kv, out, heads, kcol=0, vcol=heads * 128, batch=batch)
+    torch.cuda.synchronize()
+    return out
+
+
+def _want64(q, kv, heads):
+    """softmax(q k^T / sqrt(128)) v in float64, head by head."""
+    import torch
+
+    C = heads * 128
+    out = torch.empty(q.shape[0], C, dtype=torch.float64, device=q.device)
+    for h in range(heads):
+        c = slice(128 * h, 128 * h + 128)
+        s = q[:, c].double() @ kv[:, c].double().t().contiguous() / 128.0 ** 0.5
+        out[:, c] = torch.softmax(s, 1) @ kv[:, C + 128 * h:C + 128 * h + 128].double().contiguous()
+    return out
+
+
+@pytest.mark.parametrize("Lq,Lk,heads", [
+    (1, 1, 1), (255, 31, 2), (256, 32, 1), (257, 33, 2), (33, 64, 3), (5, 65, 1),
+    (300, 191, 2), (300, 193, 2), (64, 1025, 5), (2900, 200, 24), (2816, 97, 24)])
+def test_edges(sdq_dev, oracle, Lq, Lk, heads):
+    """Partial last key blocks and query groups, ranges of one to many blocks,
+    whole rounds of items with and without a rest cut into shares."""
+    import torch
+
+    print(f"[sdpa-packed] Lq={Lq} Lk={Lk} heads={heads}", flush=True)
+    rng = np.random.default_rng(Lq + 31 * Lk)
+    C = heads * 128
+    q = (rng.standard_normal((Lq, C)) * 0.6).astype(np.float32)
+    kv = rng.standard_normal((Lk, 2 * C)).astype(np.float32)
+    got = _run(sdq_dev, torch.from_numpy(q).to(sdq_dev), torch.from_numpy(kv).to(sdq_dev), heads)
+    got = got.cpu().numpy().astype(np.float64)
+    want = oracle.sdpa(q, kv[:, :C], kv[:, C:], heads)
+    assert np.isfinite(got).all()
+    assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("case", ["rows", "tiny", "huge", "zero_blocks", "far_logits", "inf"])
+def test_value_range(sdq_dev, case):
+    """V rows of 2^-12..2^12 in one block, V near the ends of float's range,
+    blocks of zeros between blocks of small values, logits all far below 0
+    (the padding keys of a last block would win if they counted), and an
+    infinity, which reaches its own dimension only."""
+    import torch
+
+    print(f"[sdpa-packed] range {case}", flush=True)
+    g = torch.Generator(device=sdq_dev)
+    g.manual_seed(5)
+    Lq, Lk, heads = 70, 300, 2
+    C = heads * 128
+    q = torch.randn((Lq, C), generator=g, device=sdq_dev)
+    kv = torch.randn((Lk, 2 * C), generator=g, device=sdq_dev)
+    v = kv[:, C:]
+    bound = 2e-5
+    if case == "rows":
+        v *= torch.exp2(torch.randint(-12, 13, (Lk, 1), generator=g, device=sdq_dev).float())
+    elif case == "tiny":
+        v *= 2.0 ** -80
+    elif case == "huge":
+        v *= 2.0 ** 120
+    elif case == "zero_blocks":
+        v *= 2.0 ** -40
+        v[64:128] = 0.0
+        v[290:] = 0.0
+    elif case == "far_logits":
+        q.abs_()
+        kv[:, :C] = -kv[:, :C].abs() * 30.0
+        bound = 2e-4  # logits of ~-2000 carry 2^-24 of themselves: 1e-4 of a weight
+    want = _want64(q, kv, heads)
+    if case == "inf":
+        v[17, 5] = float("inf")
+    got = _run(sdq_dev, q, kv, heads).double()
+    if case == "inf":
+        assert not torch.isfinite(got[:, 5]).any()
+        got[:, 5] = want[:, 5]
+    scale = want.abs().max()
+    assert torch.isfinite(got).all()
+    err = float((got - want).abs().max() / scale)
+    print(f"  max err {err:.3e}", flush=True)
+    assert err <= bound
+
+
+def test_chunks(sdq_dev):
+    """More keys than one launch's scratch holds for two heads: one launch
+    per head; two stacked sequences give the bits of two separate calls."""
+    import torch
+
+    L, heads = 1_100_000, 2
+    print(f"[sdpa-packed] chunks Lk={L}", flush=True)
+    g = torch.Generator(device=sdq_dev)
+    g.manual_seed(6)
+    q = torch.randn((2 * 40, 256), generator=g, device=sdq_dev)
+    kv = torch.randn((2 * L, 512), generator=g, device=sdq_dev)
+    got = _run(sdq_dev, q, kv, heads, batch=2)
+    for b in range(2):
+        qs, ks = q[40 * b:40 * b + 40], kv[b * L:(b + 1) * L]
+        one = _run(sdq_dev, qs, ks, heads)
+        assert torch.equal(got[40 * b:40 * b + 40], one)
+        want = _want64(qs, ks, heads)
+        assert float((one.double() - want).abs().max() / want.abs().max()) <= 2e-5
+
+
+def test_capture_without_warm_up(sdq_dev):
+    """A capture on a stream whose workspace cannot grow any more takes the
+    form without scratch; replays see new inputs."""
+    import torch
+
+    import sdq
+
+    g = torch.Generator(device=sdq_dev)
+    g.manual_seed(7)
+    q = torch.randn((300, 256), generator=g, device=sdq_dev)
+    kv = torch.randn((500, 512), generator=g, device=sdq_dev)
+    out = torch.empty((300, 256), device=sdq_dev)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        sdq.sdpa(q, kv, kv, out, 2, kcol=0, vcol=256)
+    for _ in range(3):
+        q.copy_(torch.randn((300, 256), generator=g, device=sdq_dev))
+        graph.replay()
+        torch.cuda.synchronize()
+        want = _want64(q, kv, 2)
+        assert float((out.double() - want).abs().max() / want.abs().max()) <= 2e-5

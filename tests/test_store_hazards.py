@@ -126,7 +126,8 @@ def _scan_sgpr(asm_text):
 
 
 @pytest.mark.slow
-@pytest.mark.parametrize("src", ["sdq_gemm.hip", "sdq_quant.hip", "sdq_repack.hip", "sdq_api.hip"])
+@pytest.mark.parametrize("src", ["sdq_gemm.hip", "sdq_quant.hip", "sdq_repack.hip", "sdq_api.hip",
+                                 "sdq_sdpa.hip"])
 def test_no_wide_store_data_hazard(tmp_path, src):
     if not os.path.exists(HIPCC):
         pytest.skip("hipcc not available")
