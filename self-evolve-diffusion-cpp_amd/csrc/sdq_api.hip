@@ -422,7 +422,8 @@ int qlinear_device(const sdq_weight* w, const float* A, int64_t M, int64_t K,
     rmax_out->chunks = 0;
   }
   const bool premax = !lnmod && pre && pre->chunks > 0;
-  if (lnmod) {
+  const bool lnrows = lnmod && lnmod_rows_fits(A, K, w->KFp, lnmod->shift, lnmod->scale);
+  if (lnmod && !lnrows) {
     std::lock_guard<std::mutex> lk(g_mu);
     if ((rc = grow(s, reinterpret_cast<void**>(&ws->st), &ws->st_bytes,
                    (size_t)M * sizeof(float2))))
@@ -438,7 +439,9 @@ int qlinear_device(const sdq_weight* w, const float* A, int64_t M, int64_t K,
 
   hipEvent_t p0 = prof ? prof_mark(s) : nullptr;
   hipError_t e =
-      lnmod ? launch_act_quant_frags_lnmod(A, M, K, Mp, w->KFp, ws->at, ws->as, cc, lnmod->shift,
+      lnrows ? launch_act_quant_frags_lnmod_rows(A, M, K, Mp, w->KFp, ws->at, ws->as, cc,
+                                                 lnmod->shift, lnmod->scale, lnmod->eps, s)
+      : lnmod ? launch_act_quant_frags_lnmod(A, M, K, Mp, w->KFp, ws->at, ws->as, cc, lnmod->shift,
                                            lnmod->scale, lnmod->eps, ws->st, s)
       : premax ? launch_act_quant_frags_premax(A, M, K, Mp, w->KFp, ws->at, ws->as, cc, pre->p,
                                                pre->chunks, pre->stride, cu_count, s)
@@ -1683,8 +1686,9 @@ int sdq_layernorm(const float* x, int64_t M, int64_t K, const float* w, const fl
   if (rc) return rc;
   if ((rc = ensure_device(dev))) return rc;
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool rows = ln_rows_fits(x, M, K, w, b, y);
   float2* st = nullptr;
-  {
+  if (!rows) {
     std::lock_guard<std::mutex> lk(g_mu);
     Workspace& ws = g_ws[{dev, s}];
     if ((rc = grow(s, reinterpret_cast<void**>(&ws.st), &ws.st_bytes, (size_t)M * sizeof(float2))))
@@ -1692,8 +1696,9 @@ int sdq_layernorm(const float* x, int64_t M, int64_t K, const float* w, const fl
     st = ws.st;
   }
   hipEvent_t p0 = t_prof ? prof_mark(s) : nullptr;
-  hipError_t e = launch_ln_stats(x, M, K, eps, st, s);
-  if (e == hipSuccess) e = launch_ln_apply(x, M, K, st, w, b, y, s);
+  hipError_t e = rows ? launch_ln_rows(x, M, K, w, b, eps, y, s)
+                      : launch_ln_stats(x, M, K, eps, st, s);
+  if (e == hipSuccess && !rows) e = launch_ln_apply(x, M, K, st, w, b, y, s);
   if (e != hipSuccess) {
     drop_events({p0});
     return hip_error(e, "layernorm launch");

@@ -37,6 +37,23 @@ __device__ __forceinline__ int quant_one(float v, float inv) {
   return (int)c;
 }
 
+// quant_one of four values as the bytes of a dword, in five operations each
+// and three to join them: clamping first gives the same value (the bounds are
+// integers), NaN and products from 2^31 up fail the compare, those down to
+// -2^31 and below are -127 either way; adding 1.5 * 2^23 rounds to nearest
+// even and leaves the two's complement byte in the low bits.
+__device__ __forceinline__ uint32_t quant_pack4(float a, float b, float c, float d, float inv) {
+  auto q = [inv](float v) {
+    const float y = v * inv;
+    float t = __builtin_amdgcn_fmed3f(y, -127.f, 127.f);
+    t = y < 2147483648.f ? t : -127.f;
+    return __float_as_uint(t + 12582912.f);
+  };
+  const uint32_t lo = __builtin_amdgcn_perm(q(b), q(a), 0x0c0c0400);
+  const uint32_t hi = __builtin_amdgcn_perm(q(d), q(c), 0x04000c0c);
+  return lo | hi;
+}
+
 __device__ __forceinline__ float gelu_tanh(float v) {
   // nn.GELU(approximate='tanh'), src/model/ovi_dit.cpp:132-142:
   //   0.5 v (1 + tanh(u)) = v / (1 + e^(-2u)),  u = sqrt(2/pi) (v + 0.044715 v^3)

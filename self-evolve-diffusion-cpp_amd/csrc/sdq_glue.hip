@@ -13,6 +13,7 @@
 
 #include <cstdlib>
 #include <type_traits>
+#include "sdq_rowblock.h"
 #include "sdq_rowsum.h"
 
 #pragma clang fp contract(off)
@@ -132,6 +133,88 @@ rms_rope_apply_kernel(RmsSegs sg, int64_t C, int hd) {
   q[1] = y1;
 }
 
+// Both in one pass over the rows (C % 4 == 0, C <= rowblock::kMaxCols, head
+// width % 4 == 0, 16-byte aligned rows): workgroup b takes kRows rows of
+// the segment i with b in [blk0[i], blk0[i+1]).
+template <int NC>
+__global__ void __launch_bounds__(rowblock::kThreads, 4)
+rms_rope_rows_kernel(RmsSegs sg, int C, int hd, float eps) {
+  __shared__ rowblock::Lds lds;
+  const int l = threadIdx.x & 63;
+  const int w = rowblock::role();
+  const int i = seg_of(sg.blk0, sg.n, (int64_t)blockIdx.x);
+  const RmsSeg& g = sg.s[i];
+  if (w == rowblock::kWaves) {
+    rowblock::add_terms<NC>(lds);
+    return;
+  }
+  const int64_t row = ((int64_t)blockIdx.x - sg.blk0[i]) * rowblock::kRows + 2 * w;
+  const __amdgpu_buffer_rsrc_t r[2] = {
+      rowblock::row_rsrc(row < g.L ? g.x + row * g.ld : nullptr, C),
+      rowblock::row_rsrc(row + 1 < g.L ? g.x + (row + 1) * g.ld : nullptr, C)};
+  const __amdgpu_buffer_rsrc_t wr = rowblock::row_rsrc(g.w, C);
+  // the rows' (cos, sin) tables; none: empty, and no pair is rotated
+  const int nr = g.cs ? g.nr : 0;
+  const __amdgpu_buffer_rsrc_t cr[2] = {
+      rowblock::row_rsrc(nr && row < g.L ? g.cs + row * nr * 2 : nullptr, 2 * nr),
+      rowblock::row_rsrc(nr && row + 1 < g.L ? g.cs + (row + 1) * nr * 2 : nullptr, 2 * nr)};
+  rowblock::Rows<NC> x;
+  rowblock::load(x, r[0], r[1], l);
+  float ss[2];
+  const float none[2] = {0.f, 0.f};
+  // chunk k's weights and (cos, sin) pairs, read a chunk ahead of their use
+  struct Ops {
+    rowblock::v4f w;
+    float2 cs[2][2];
+  } ops;
+  auto fetch = [&](int k, int c) {
+    Ops& o = ops;
+    o.w = rowblock::get(wr, k, l);
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        o.cs[u][h] = __builtin_bit_cast(
+            float2, __builtin_amdgcn_raw_buffer_load_b64(cr[u], 4 * c + 8 * h, 0, 0));
+  };
+  const int step = rowblock::kChunk % hd;
+  auto next = [&](int c) { return c + step >= hd ? c + step - hd : c + step; };
+  int c = 4 * l % hd;  // column inside the head
+  rowblock::put_terms<NC, 2>(x, C, none, lds, w, ss);
+  fetch(0, c);
+  float inv[2];
+#pragma unroll
+  for (int u = 0; u < 2; u++) inv[u] = 1.f / sqrtf(ss[u] / (float)C + eps);
+#pragma unroll
+  for (int k = 0; k < NC; k++) {
+    const Ops o = ops;
+    if (k + 1 < NC) fetch(k + 1, next(c));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      rowblock::v4f y;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float a = x.v[u][k][e] * inv[u];
+        y[e] = a * o.w[e];
+      }
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const float2 t = o.cs[u][h];  // (cos, sin)
+        const float r1s = y[2 * h + 1] * t.y, r1c = y[2 * h + 1] * t.x;
+        const float n0 = __builtin_fmaf(y[2 * h], t.x, -r1s);
+        const float n1 = __builtin_fmaf(y[2 * h], t.y, r1c);
+        const bool rot = c / 2 + h < nr;  // the pair's index inside the head
+        y[2 * h] = rot ? n0 : y[2 * h];
+        y[2 * h + 1] = rot ? n1 : y[2 * h + 1];
+      }
+      rowblock::set(r[u], k, l, y);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    c = next(c);
+  }
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace
@@ -142,7 +225,7 @@ hipError_t launch_rmsnorm_rope_segs(const RmsSeg* segs, int nseg, int64_t C, int
     return hipErrorInvalidValue;
   RmsSegs st{};
   st.n = nseg;
-  bool vec = C % 4 == 0, few = true, any_w = false, full = C % 32 == 0;
+  bool vec = C % 4 == 0, few = true, any_w = false, all_w = true, full = C % 32 == 0;
   for (int i = 0; i < nseg; i++) {
     const RmsSeg& g = segs[i];
     if (g.L < 0 || g.ld < C || g.nr < 0 || g.nr > C / heads / 2 || (!g.w && !g.cs) ||
@@ -154,9 +237,22 @@ hipError_t launch_rmsnorm_rope_segs(const RmsSeg* segs, int nseg, int64_t C, int
     vec = vec && aligned16(g.x) && g.ld % 4 == 0;
     few = few && g.L <= 4096;
     any_w = any_w || (g.w && g.L > 0);
+    all_w = all_w && (g.w || g.L == 0);
     full = full && (g.L == 0 || seg_span_bytes(g, C) <= kFullMaxBytes);
   }
   full = full && vec;
+  bool rows = vec && all_w && C <= rowblock::kMaxCols && C / heads % 4 == 0;
+  for (int i = 0; i < nseg; i++) rows = rows && (segs[i].L == 0 || aligned16(segs[i].w));
+  if (rows) {
+    for (int i = 0; i < nseg; i++)
+      st.blk0[i + 1] = st.blk0[i] + ceil_div(segs[i].L, rowblock::kRows);
+    if (st.blk0[nseg] == 0) return hipSuccess;
+    return rowblock::for_cols(C, [&](auto nc) {
+      hipLaunchKernelGGL((rms_rope_rows_kernel<decltype(nc)::value>), dim3((unsigned)st.blk0[nseg]),
+                         dim3(rowblock::kThreads), 0, s, st, (int)C, (int)(C / heads), eps);
+      return hipGetLastError();
+    });
+  }
   // segments without a weight (rotation only) own no stats blocks
   if (any_w) {
     const dim3 g((unsigned)st.blk0[nseg]), b(64);
@@ -207,6 +303,62 @@ ln_apply_kernel(const float* x, int64_t M, int64_t K, const float2* __restrict__
   y[idx] = __builtin_fmaf(t, w ? w[k] : 1.f, b ? b[k] : 0.f);
 }
 
+// Statistics and normalization in one pass over the rows (K % 4 == 0, K <=
+// rowblock::kMaxCols, 16-byte aligned rows and weights); y may be x.
+template <int NC>
+__global__ void __launch_bounds__(rowblock::kThreads, 4)
+ln_rows_kernel(const float* x, int64_t M, int K, const float* __restrict__ w,
+               const float* __restrict__ b, float eps, float* y) {
+  __shared__ rowblock::Lds lds;
+  const int l = threadIdx.x & 63;
+  const int wv = rowblock::role();
+  if (wv == rowblock::kWaves) {
+    rowblock::add_terms<NC>(lds);
+    rowblock::add_terms<NC>(lds);
+    return;
+  }
+  const int64_t row = (int64_t)blockIdx.x * rowblock::kRows + 2 * wv;
+  const __amdgpu_buffer_rsrc_t yr[2] = {
+      rowblock::row_rsrc(row < M ? y + row * K : nullptr, K),
+      rowblock::row_rsrc(row + 1 < M ? y + (row + 1) * K : nullptr, K)};
+  const __amdgpu_buffer_rsrc_t wr = rowblock::row_rsrc(w, K), br = rowblock::row_rsrc(b, K);
+  rowblock::Rows<NC> r;
+  rowblock::load(r, rowblock::row_rsrc(row < M ? x + row * K : nullptr, K),
+                 rowblock::row_rsrc(row + 1 < M ? x + (row + 1) * K : nullptr, K), l);
+  // chunk i's weights, read a chunk ahead of their use
+  rowblock::v4f wt, bt;
+  auto fetch = [&](int i) {
+    wt = rowblock::get(wr, i, l);
+    bt = rowblock::get(br, i, l);
+  };
+  float mu[2] = {0.f, 0.f}, var[2];
+  rowblock::put_terms<NC, 0>(r, K, mu, lds, wv, mu);
+#pragma unroll
+  for (int u = 0; u < 2; u++) mu[u] = mu[u] / (float)K;
+  rowblock::put_terms<NC, 1>(r, K, mu, lds, wv, var);
+  fetch(0);
+  float inv[2];
+#pragma unroll
+  for (int u = 0; u < 2; u++) inv[u] = 1.f / sqrtf(var[u] / (float)K + eps);
+#pragma unroll
+  for (int i = 0; i < NC; i++) {
+    const rowblock::v4f wi = w ? wt : rowblock::v4f{1.f, 1.f, 1.f, 1.f}, bi = bt;
+    if (i + 1 < NC) fetch(i + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      rowblock::v4f o;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float t = r.v[u][i][e] * inv[u];
+        o[e] = __builtin_fmaf(t, wi[e], bi[e]);
+      }
+      rowblock::set(yr[u], i, l, o);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
 __global__ void __launch_bounds__(256)
 add_kernel(float* x, const float* y, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -242,6 +394,23 @@ resid2_kernel(float* __restrict__ x, int64_t n4, int64_t N4, ResidStep a, ResidS
 }
 
 }  // namespace
+
+bool ln_rows_fits(const float* x, int64_t M, int64_t K, const float* w, const float* b,
+                  const float* y) {
+  return K % 4 == 0 && K <= rowblock::kMaxCols && M <= (int64_t)1 << 30 && aligned16(x) &&
+         aligned16(y) && aligned16(w) && aligned16(b);
+}
+
+hipError_t launch_ln_rows(const float* x, int64_t M, int64_t K, const float* w, const float* b,
+                          float eps, float* y, hipStream_t s) {
+  if (M <= 0 || K <= 0) return hipSuccess;
+  return rowblock::for_cols(K, [&](auto nc) {
+    hipLaunchKernelGGL((ln_rows_kernel<decltype(nc)::value>),
+                       dim3((unsigned)ceil_div(M, rowblock::kRows)), dim3(rowblock::kThreads), 0, s,
+                       x, M, (int)K, w, b, eps, y);
+    return hipGetLastError();
+  });
+}
 
 hipError_t launch_ln_apply(const float* x, int64_t M, int64_t K, const float2* st, const float* w,
                            const float* b, float* y, hipStream_t s) {

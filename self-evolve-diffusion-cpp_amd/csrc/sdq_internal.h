@@ -113,6 +113,14 @@ hipError_t launch_act_quant_frags_lnmod(const float* A, int64_t M, int64_t K, in
                                         int64_t KFp, int8_t* at, float* as, const ColCopy& cc,
                                         const float* shift, const float* scale, float eps,
                                         float2* st, hipStream_t s);
+// The same in one pass over the rows, without scratch, for what
+// lnmod_rows_fits accepts (up to 3072 columns, 16-byte aligned arrays).
+bool lnmod_rows_fits(const float* A, int64_t K, int64_t KFp, const float* shift,
+                     const float* scale);
+hipError_t launch_act_quant_frags_lnmod_rows(const float* A, int64_t M, int64_t K, int64_t Mp,
+                                             int64_t KFp, int8_t* at, float* as,
+                                             const ColCopy& cc, const float* shift,
+                                             const float* scale, float eps, hipStream_t s);
 // In place on L rows of stride ld (C columns): rmsnorm with weight w (w ==
 // nullptr: none), then RoPE of each head's first nr pairs with the (cos, sin)
 // table cs [L][nr] (cs == nullptr: no RoPE). inv: [L] scratch.
@@ -141,6 +149,12 @@ hipError_t launch_ln_stats(const float* A, int64_t M, int64_t K, float eps, floa
 // nullable: 1, 0). x, y: [M, K] contiguous (may alias).
 hipError_t launch_ln_apply(const float* x, int64_t M, int64_t K, const float2* st, const float* w,
                            const float* b, float* y, hipStream_t s);
+// Both in one pass over the rows, without scratch, for what ln_rows_fits
+// accepts (up to 3072 columns, 16-byte aligned arrays); x, y may be the same.
+bool ln_rows_fits(const float* x, int64_t M, int64_t K, const float* w, const float* b,
+                  const float* y);
+hipError_t launch_ln_rows(const float* x, int64_t M, int64_t K, const float* w, const float* b,
+                          float eps, float* y, hipStream_t s);
 // x[i] += y[i], i < n.
 hipError_t launch_add(float* x, const float* y, int64_t n, hipStream_t s);
 // One residual epilogue of a Linear applied to x from the Linear's plain

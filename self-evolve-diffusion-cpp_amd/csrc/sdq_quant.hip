@@ -20,6 +20,7 @@
 
 #include "sdq_internal.h"
 #include "sdq_device.h"
+#include "sdq_rowblock.h"
 #include "sdq_rowsum.h"
 
 #pragma clang fp contract(off)
@@ -27,7 +28,6 @@
 namespace sdq {
 namespace {
 
-using dev::quant_one;
 
 constexpr int kQuantWaves = 16;
 constexpr int kQuantCache = 6;  // 16 waves x 6 frags x 32 = K <= 3072 in one pass
@@ -72,12 +72,8 @@ __device__ __forceinline__ float amax16(const float v[16], float mx) {
 __device__ __forceinline__ uint4 pack16(const float v[16], float inv) {
   uint32_t w[4];
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    uint32_t x = 0;
-#pragma unroll
-    for (int b = 0; b < 4; b++) x |= (uint32_t)(uint8_t)(int8_t)quant_one(v[4 * i + b], inv) << (8 * b);
-    w[i] = x;
-  }
+  for (int i = 0; i < 4; i++)
+    w[i] = dev::quant_pack4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3], inv);
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
@@ -497,6 +493,109 @@ act_quant_emit_kernel(const float* __restrict__ A, int64_t M, int64_t K, int64_t
   }
 }
 
+// Norm, modulation and quantization in one pass over the rows (the values of
+// act_quant_unit<..., XF>; rows of up to 3072 columns): workgroup b takes rows
+// kRows b .. of the Mp padded ones; they stay in registers across their sums
+// (sdq_rowblock.h), the int8 rows are put together in LDS and leave as runs of
+// 16 kRows bytes. Workgroups past M (tile padding) write zeros.
+template <int NC>
+__global__ void __launch_bounds__(rowblock::kThreads, 4)
+lnmod_quant_rows_kernel(const float* __restrict__ A, int64_t M, int64_t Mp, int K, int KFp,
+                        const float* __restrict__ shift, const float* __restrict__ scale,
+                        float eps, int8_t* __restrict__ out, float* __restrict__ as, ColCopy cc) {
+  using rowblock::v4f;
+  constexpr int kRun = 16 * rowblock::kRows;
+  constexpr int kPitch = 2 * kRun + 16;  // a fragment's piece, then on to other banks
+  union Shared {
+    rowblock::Lds sums;
+    char q[NC * 8 * kPitch];
+  };
+  __shared__ __attribute__((aligned(16))) Shared lds;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cc.CP;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    if (cc.bias_pad) cc.bias_pad[i] = i < cc.N ? cc.bias[i] : 0.f;
+    if (cc.gate_pad) cc.gate_pad[i] = i < cc.N ? cc.gate[i] : 0.f;
+  }
+  const int l = threadIdx.x & 63;
+  const int w = rowblock::role();
+  const int64_t row0 = (int64_t)blockIdx.x * rowblock::kRows, row = row0 + 2 * w;
+  if (row0 >= M) {
+    for (int i = threadIdx.x; i < NC * 8 * kPitch / 4; i += rowblock::kThreads)
+      reinterpret_cast<uint32_t*>(lds.q)[i] = 0;
+  } else if (w == rowblock::kWaves) {
+    rowblock::add_terms<NC>(lds.sums);
+    rowblock::add_terms<NC>(lds.sums);
+    rowblock::sync();
+  } else {
+    rowblock::Rows<NC> r;
+    rowblock::load(r, rowblock::row_rsrc(row < M ? A + row * K : nullptr, K),
+                   rowblock::row_rsrc(row + 1 < M ? A + (row + 1) * K : nullptr, K), l);
+    const __amdgpu_buffer_rsrc_t shr = rowblock::row_rsrc(shift, K),
+                                 scr = rowblock::row_rsrc(scale, K);
+    float mu[2] = {0.f, 0.f}, var[2], inv[2];
+    rowblock::put_terms<NC, 0>(r, K, mu, lds.sums, w, mu);
+#pragma unroll
+    for (int u = 0; u < 2; u++) mu[u] = mu[u] / (float)K;
+    rowblock::put_terms<NC, 1>(r, K, mu, lds.sums, w, var);
+#pragma unroll
+    for (int u = 0; u < 2; u++) inv[u] = 1.f / sqrtf(var[u] / (float)K + eps);
+    float mx[2] = {0.f, 0.f};
+    v4f sh = rowblock::get(shr, 0, l), sc = rowblock::get(scr, 0, l);
+#pragma unroll
+    for (int i = 0; i < NC; i++) {
+      const v4f shi = sh, sci = sc;
+      // a chunk's modulation is read a chunk ahead of its use
+      if (i + 1 < NC) sh = rowblock::get(shr, i + 1, l), sc = rowblock::get(scr, i + 1, l);
+      __builtin_amdgcn_sched_barrier(0);
+      const bool in = i * rowblock::kChunk + 4 * l < K;
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const float t = r.v[u][i][e] * inv[u];
+          const float o = t + 0.f;
+          const float a = 1.f + sci[e];
+          r.v[u][i][e] = in ? __builtin_fmaf(o, a, shi[e]) : 0.f;
+        }
+        rowblock::keep(r.v[u][i]);
+#pragma unroll
+        for (int e = 0; e < 4; e++) mx[u] = fmaxf(mx[u], fabsf(r.v[u][i][e]));  // NaN never wins
+        rowblock::keep(mx[u]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    rowblock::sync();  // every wave has read its sums: the LDS turns into the int8 rows
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+#pragma unroll
+      for (int d = 1; d < 64; d *= 2) mx[u] = fmaxf(mx[u], __shfl_xor(mx[u], d));
+      float s = mx[u] / 127.f;
+      if (s == 0.f) s = 1.f;
+      const float qi = 1.f / s;
+      if (l == 0 && row + u < M) as[row + u] = s;
+#pragma unroll
+      for (int i = 0; i < NC; i++) {
+        const v4f v = r.v[u][i];
+        *reinterpret_cast<uint32_t*>(lds.q + (8 * i + (l >> 3)) * kPitch + (l >> 2 & 1) * kRun +
+                                     (2 * w + u) * 16 + (l & 3) * 4) =
+            dev::quant_pack4(v[0], v[1], v[2], v[3], qi);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  rowblock::sync();
+  // 16-byte slots: fragment kb, half, row
+  for (int n = threadIdx.x; n < KFp * 2 * rowblock::kRows; n += rowblock::kThreads) {
+    const int half = n / rowblock::kRows, r = n - half * rowblock::kRows;
+    const int kb = half >> 1;
+    const int64_t m = row0 + r;
+    if (m < Mp)
+      *reinterpret_cast<uint4*>(out + ((m >> 5) * KFp + kb) * 1024 + (half & 1) * 512 +
+                                (m & 31) * 16) =
+          *reinterpret_cast<const uint4*>(lds.q + kb * kPitch + (half & 1) * kRun + r * 16);
+  }
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // Fragment groups per split item: 4 from 64 units up (measured at K=14336:
@@ -598,6 +697,25 @@ hipError_t launch_act_quant_frags_lnmod(const float* A, int64_t M, int64_t K, in
                      dim3((unsigned)units), dim3(kQuantUnitWaves * 64), 0, s, A, M, K, KFp, vec,
                      at, as, cc, nullptr, 0, 0, lm);
   return hipGetLastError();
+}
+
+bool lnmod_rows_fits(const float* A, int64_t K, int64_t KFp, const float* shift,
+                     const float* scale) {
+  return K % 4 == 0 && KFp * 32 <= rowblock::kMaxCols && aligned16(A) && aligned16(shift) &&
+         aligned16(scale);
+}
+
+hipError_t launch_act_quant_frags_lnmod_rows(const float* A, int64_t M, int64_t K, int64_t Mp,
+                                             int64_t KFp, int8_t* at, float* as,
+                                             const ColCopy& cc, const float* shift,
+                                             const float* scale, float eps, hipStream_t s) {
+  if (!shift || !scale || K <= 0) return hipErrorInvalidValue;
+  return rowblock::for_cols(KFp * 32, [&](auto nc) {
+    hipLaunchKernelGGL((lnmod_quant_rows_kernel<decltype(nc)::value>),
+                       dim3((unsigned)ceil_div(Mp, rowblock::kRows)), dim3(rowblock::kThreads), 0,
+                       s, A, M, Mp, (int)K, (int)KFp, shift, scale, eps, at, as, cc);
+    return hipGetLastError();
+  });
 }
 
 hipError_t launch_act_quant_frags_premax(const float* A, int64_t M, int64_t K, int64_t Mp,
