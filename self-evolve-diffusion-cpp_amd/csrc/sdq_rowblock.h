@@ -3,8 +3,8 @@
 // at 256 i + 4 l of chunk i), so a row norm reads its rows once and writes its
 // result once. The sums keep the reference's column order (bit-exact, see
 // sdq_rowsum.h): chunk by chunk those waves put their terms into a ring in
-// LDS, and the eighth, its lane l on row l % 14, runs the dependent adds of
-// all rows (a wave of its own: its operand tiles and the rows would not fit
+// LDS, and the eighth, its lane l on row l % 14, runs the dependent adds of all
+// rows (a wave of its own: its operand tiles and the rows would not fit
 // one wave's registers at two workgroups per CU; five-wave workgroups of eight
 // rows, which place two waves on one SIMD, ran one or two per CU).
 //
@@ -144,7 +144,10 @@ template <int NC>
 __device__ __forceinline__ void add_terms(Lds& s) {
   const int l = threadIdx.x & 63;
   const int mine = l % kRows;
-  constexpr int kTiles = kChunk / 32;  // 32-column tiles, the next one read while this one is added
+  // 32-column tiles, the next one read while this one is added, with one wait
+  // per tile: an add takes ~5 cycles (the chain's latency) and every other
+  // instruction of this wave as long, so a row costs ~1.3 x its columns.
+  constexpr int kTiles = kChunk / 32;
   v4f a[2][8];
   auto read = [&](int i, int t, v4f (&d)[8]) {
     const v4f* row = reinterpret_cast<const v4f*>(s.t[i % 3][mine]) + 8 * t;
@@ -160,6 +163,7 @@ __device__ __forceinline__ void add_terms(Lds& s) {
     for (int t = 0; t < kTiles; t++) {
       // (the tile after the last: of a chunk written before, not added)
       read(t + 1 < kTiles ? i : i + 1, (t + 1) % kTiles, a[(t + 1) & 1]);
+      __builtin_amdgcn_s_waitcnt(15 | 3 << 14 | 7 << 4 | 8 << 8);  // the tile's own reads
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int q = 0; q < 8; q++)

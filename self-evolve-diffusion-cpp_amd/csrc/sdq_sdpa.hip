@@ -204,6 +204,18 @@ __device__ __forceinline__ void pin(T& v) {
   asm volatile("" : "+v"(v));
 }
 
+// a, b as fp16 hi + lo, each part's pair in a dword. neg1 = -1 unknown to the
+// compiler: x - hi then stays a multiply-add that reads hi as fp16 and writes
+// fp16 (one instruction per low part).
+__device__ __forceinline__ void split_pair(float a, float b, float neg1, uint32_t& hi,
+                                           uint32_t& lo) {
+  hi = __builtin_bit_cast(uint32_t, v2h{(_Float16)a, (_Float16)b});
+  pin(hi);  // the low parts read its halves
+  const v2h h = __builtin_bit_cast(v2h, hi);
+  lo = __builtin_bit_cast(uint32_t, v2h{(_Float16)__builtin_fmaf((float)h.x, neg1, a),
+                                        (_Float16)__builtin_fmaf((float)h.y, neg1, b)});
+}
+
 __global__ void __launch_bounds__(kWaves * 64)
 sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restrict__ packed,
                    const int2* __restrict__ exps, float* __restrict__ O, int64_t ldo, int64_t Lq,
@@ -265,50 +277,62 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
     for (int c = 0; c < LD; c++)
       dev::dma16<0>(rs, voff, soff(i) + kRecV + c * 1024u, slot_v(i) + c * 1024u);
   };
-  issue_k(0), issue_v(0), issue_k(1), issue_v(1), issue_k(2), issue_v(2), issue_k(3);
+  float neg1 = -1.f;  // for split_pair
+  asm volatile("" : "+s"(neg1));
+  // Everything the first scores need is asked for at once: block exponents
+  // (64 blocks from kb0, one per lane, and the first 64 of all), query rows,
+  // and the first DMAs; the other DMAs follow the queries' conversion, whose
+  // wait would cover them too.
+  int2 ev = ex[kb0 + lane < nkb ? kb0 + lane : nkb - 1];
+  int vmin = ex[lane < nkb ? lane : nkb - 1].y;
   // The query rows, lane (j, h): dims 32 d + 8 h + 0..7 of query 16 t + j,
   // scaled by 2^-eq and split into fp16 parts
   v8h qh[QT][4], ql[QT][4];
   int eq[QT];
+  float4 qrow[QT][8];
 #pragma unroll
   for (int t = 0; t < QT; t++) {
     const int64_t qi = q0 + 16 * t + j;
     const float* src = Qs + (qi < Lq ? qi : 0) * ldq + col + 8 * h;  // past Lq: not stored
-    float4 qr[8];
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+      qrow[t][c] = *reinterpret_cast<const float4*>(src + 32 * (c >> 1) + 4 * (c & 1));
+  }
+  issue_k(0), issue_v(0), issue_k(1);
+#pragma unroll
+  for (int t = 0; t < QT; t++) {
+    const float4(&qr)[8] = qrow[t];
     float mq = 0.f;
 #pragma unroll
     for (int c = 0; c < 8; c++) {
-      qr[c] = *reinterpret_cast<const float4*>(src + 32 * (c >> 1) + 4 * (c & 1));
-      mq = amax_finite(amax_finite(mq, qr[c].x), qr[c].y);
-      mq = amax_finite(amax_finite(mq, qr[c].z), qr[c].w);
+      mq = fmaxf(fmaxf(mq, fabsf(qr[c].x)), fabsf(qr[c].y));
+      mq = fmaxf(fmaxf(mq, fabsf(qr[c].z)), fabsf(qr[c].w));
     }
     eq[t] = top_exp(quad16_max(mq));
 #pragma unroll
     for (int d = 0; d < 4; d++) {
-      const float x[8] = {qr[2 * d].x,     qr[2 * d].y,     qr[2 * d].z,     qr[2 * d].w,
-                          qr[2 * d + 1].x, qr[2 * d + 1].y, qr[2 * d + 1].z, qr[2 * d + 1].w};
+      uint32_t* hw = reinterpret_cast<uint32_t*>(&qh[t][d]);
+      uint32_t* lw = reinterpret_cast<uint32_t*>(&ql[t][d]);
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const float y = ldexpf(x[e], -eq[t]);
-        qh[t][d][e] = (_Float16)y;
-        ql[t][d][e] = (_Float16)(y - (float)qh[t][d][e]);
+      for (int e = 0; e < 4; e++) {
+        const float4& v = qr[2 * d + (e >> 1)];
+        split_pair(ldexpf(e & 1 ? v.z : v.x, -eq[t]), ldexpf(e & 1 ? v.w : v.y, -eq[t]), neg1,
+                   hw[e], lw[e]);
       }
     }
   }
+  issue_v(1), issue_k(2), issue_v(2), issue_k(3);
   // a V block of zeros takes the smallest exponent of the others
-  int vmin = kZeroV;
-  for (int k = lane; k < nkb; k += 64) vmin = min(vmin, ex[k].y);
+  for (int k = lane + 64; k < nkb; k += 64) vmin = min(vmin, ex[k].y);
 #pragma unroll
   for (int d = 1; d < 64; d *= 2) vmin = min(vmin, __shfl_xor(vmin, d));
   vmin = vmin == kZeroV ? 0 : vmin;
-  // exponents of 64 key blocks at a time, one block per lane
-  int2 ev;
+  if (ev.y == kZeroV) ev.y = vmin;
   auto load_ev = [&](int i) {
     const int k = kb0 + i + lane;
     ev = ex[k < nkb ? k : nkb - 1];
     if (ev.y == kZeroV) ev.y = vmin;
   };
-  load_ev(0);
   auto kfrag = [&](int i, int c) {
     const char* p = ldsp + (i & (kRing - 1)) * kRecV + c * 1024;
     return Frag{*reinterpret_cast<const uint4*>(p), *reinterpret_cast<const uint4*>(p + kPart)};
@@ -366,10 +390,6 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
     }
   };
 
-  // -1 the compiler does not know, so that x - hi stays a multiply-add that
-  // reads hi as fp16 and writes fp16 (one instruction per low part)
-  float neg1 = -1.f;
-  asm volatile("" : "+s"(neg1));
   Frag fr[4];
   // K(0) has landed (newer DMAs may be in flight), then V(0) and K(1)
   __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(6 * LD));
@@ -453,13 +473,7 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
         const int pi = c * (QT / 2) + u;
         ps[pi >> 2] += x1[u];
         // P = fp16 hi + fp16 lo, two keys per dword
-        uint32_t hw = __builtin_bit_cast(uint32_t, v2h{(_Float16)x0[u], (_Float16)x1[u]});
-        pin(hw);  // the low parts then read its halves
-        const v2h hi = __builtin_bit_cast(v2h, hw);
-        const v2h lo = {(_Float16)__builtin_fmaf((float)hi.x, neg1, x0[u]),
-                        (_Float16)__builtin_fmaf((float)hi.y, neg1, x1[u])};
-        phw[pi] = hw;
-        plw[pi] = __builtin_bit_cast(uint32_t, lo);
+        split_pair(x0[u], x1[u], neg1, phw[pi], plw[pi]);
         pin(plw[pi]);
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -539,12 +553,12 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
     }
     if (i1 < n && __any(up)) raise(ml, vx);  // (past the end: a repeated block)
   };
-  int i = 0;
-  for (; i + 1 < n; i += 2) {
+  for (int i = 0;;) {
     step(i, st, st2);
-    step(i + 1, st2, st);
+    if (++i == n) break;
+    step(i, st2, st);
+    if (++i == n) break;
   }
-  if (i < n) step(i, st, st2);
 
   const int64_t nslots = (int64_t)(plan.items - plan.nfull) * plan.splits;
 #pragma unroll
