@@ -308,11 +308,14 @@ int hip_error(hipError_t e, const char* what) {
 }
 
 // Row maxima handed from a GELU GEMM's epilogue to the next quantizer:
-// p[row * stride + c], c < chunks (chunks = 0: not written).
+// p[row * stride + c], c < chunks, or tail_chunks from row tail_row on (chunks
+// = 0: not written).
 struct RowMax {
   float* p = nullptr;
   int stride = 0;
   int chunks = 0;
+  int64_t tail_row = 0;
+  int tail_chunks = 0;
 };
 
 // Norm + modulation folded into the activation quantizer: the GEMM's rows
@@ -444,7 +447,8 @@ int qlinear_device(const sdq_weight* w, const float* A, int64_t M, int64_t K,
       : lnmod ? launch_act_quant_frags_lnmod(A, M, K, Mp, w->KFp, ws->at, ws->as, cc, lnmod->shift,
                                            lnmod->scale, lnmod->eps, ws->st, s)
       : premax ? launch_act_quant_frags_premax(A, M, K, Mp, w->KFp, ws->at, ws->as, cc, pre->p,
-                                               pre->chunks, pre->stride, cu_count, s)
+                                               pre->chunks, pre->stride, pre->tail_row,
+                                               pre->tail_chunks, cu_count, s)
                : launch_act_quant_frags(A, M, K, Mp, w->KFp, ws->at, ws->as, cc,
                                         pmax_bytes ? ws->pmax : nullptr, cu_count, s);
   if (e != hipSuccess) {
@@ -459,9 +463,25 @@ int qlinear_device(const sdq_weight* w, const float* A, int64_t M, int64_t K,
   int tail = 0;
   hipEvent_t pmid = nullptr;
   if (prof && hipEventCreate(&pmid) != hipSuccess) pmid = nullptr;
+  // The 128x128 launch of a 256x256 one's last rows: its own split-K where it
+  // is few tiles, if the partial sums' buffer can be had (not in the no-alloc
+  // mode, whose scratch the shapes it takes were sized without).
+  int tail_splitk = 1;
+  int* tail_part = nullptr;
+  if (const int64_t Ma = cfg == kCfg256x256 && !fixed ? tail_split_rows(M, N, cu_count) : 0) {
+    // row maxima come from the unsplit launch only
+    tail_splitk = rmax_out ? 1 : choose_splitk(kCfg128x128, M - Ma, N, w->KFp, cu_count);
+    if (tail_splitk > 1) {
+      std::lock_guard<std::mutex> lk(g_mu);
+      if (grow(s, reinterpret_cast<void**>(&ws->part), &ws->part_bytes,
+               (size_t)tail_splitk * (size_t)(M - Ma) * (size_t)N * 4) == SDQ_OK)
+        tail_part = ws->part;
+    }
+  }
   GemmAux aux{cc.bias_pad, cc.gate_pad, ws->sink, g_dev[w->device].cu_count, splitk,
-              splitk > 1 ? ws->part : nullptr, rmax_out ? &rmax_out->chunks : nullptr, &tail,
-              pmid};
+              splitk > 1 ? ws->part : nullptr, rmax_out ? &rmax_out->chunks : nullptr,
+              rmax_out ? &rmax_out->tail_row : nullptr,
+              rmax_out ? &rmax_out->tail_chunks : nullptr, &tail, pmid, tail_splitk, tail_part};
   e = launch_qgemm(cfg, w->frags, w->scale, ws->at, ws->as, M, N, w->KFp, ea, Y, vec, aux, s);
   if (e != hipSuccess) {
     drop_events({p0, p1, pmid});
@@ -1544,8 +1564,8 @@ int sdq_qlinear_stack(const sdq_group_item* items, int n, int ngroup, const sdq_
     if (cv[i].seg < 0 || (fold_g >= 0 && i == fold_s)) continue;
     const QuantSeg& q = qs.s[cv[i].seg];
     const EpiArgs ea = make_epi(&it.epi, it.w->K);
-    const GemmAux aux{q.cc.bias_pad, q.cc.gate_pad, sink, cu_count, 1, nullptr, nullptr, &tail,
-                      nullptr};
+    const GemmAux aux{q.cc.bias_pad, q.cc.gate_pad, sink, cu_count, 1, nullptr, nullptr, nullptr,
+                      nullptr, &tail, nullptr, 1, nullptr};
     e = launch_qgemm(cfgs[i], it.w->frags, it.w->scale, q.at, q.as, it.M, it.w->N, it.w->KFp, ea,
                      it.Y, 1, aux, s);
     if (e != hipSuccess) return hip_error(e, "stack qgemm launch");
@@ -1565,8 +1585,8 @@ int sdq_qlinear_stack(const sdq_group_item* items, int n, int ngroup, const sdq_
     ea.rmax = rm.p;
     ea.rmax_stride = rm.stride;
     const QuantSeg& q = qs.s[cv[n].seg];
-    const GemmAux aux{q.cc.bias_pad, nullptr, sink, cu_count, 1, nullptr, &rm.chunks, &tail,
-                      nullptr};
+    const GemmAux aux{q.cc.bias_pad, nullptr, sink, cu_count, 1, nullptr, &rm.chunks,
+                      &rm.tail_row, &rm.tail_chunks, &tail, nullptr, 1, nullptr};
     e = launch_qgemm(cfg1, fc1->frags, fc1->scale, q.at, q.as, ffn->M, fc1->N, fc1->KFp, ea,
                      ffn->hid, 1, aux, s);
     if (e != hipSuccess) return hip_error(e, "stack fc1 launch");

@@ -58,10 +58,14 @@ __device__ __forceinline__ float gelu_tanh(float v) {
   // nn.GELU(approximate='tanh'), src/model/ovi_dit.cpp:132-142:
   //   0.5 v (1 + tanh(u)) = v / (1 + e^(-2u)),  u = sqrt(2/pi) (v + 0.044715 v^3)
   // (1 + tanh(u) = 2 / (1 + e^(-2u))), with the hardware exp2 and reciprocal
-  // (~1 ulp each): a few instructions and no branch. Saturation matches the
-  // tanh form: e^(-2u) -> inf gives v * 0 (a signed zero), -> 0 gives v.
-  const float u = 0.7978845608028654f * (v + 0.044715f * v * v * v);
-  const float e = __builtin_amdgcn_exp2f(-2.8853900817779268f * u);  // e^(-2u) = 2^(-2u log2 e)
+  // (~1 ulp each): a few instructions and no branch. -2 u log2(e) as v (k1 +
+  // k2 v^2): three roundings instead of six (error over [-12, 12]: mean 1.8e-7
+  // of the value against 2.3e-7, largest 8.8e-6 against 1.5e-5 in the far
+  // tail) and three operations fewer per value of the FFN's hidden state.
+  // Saturation matches the tanh form: e^(-2u) -> inf gives v * 0 (a signed
+  // zero), -> 0 gives v.
+  const float e =
+      __builtin_amdgcn_exp2f(v * __builtin_fmaf(v * v, -0.1029432395800235f, -2.302208198144325f));
   return v * __builtin_amdgcn_rcpf(1.f + e);
 }
 

@@ -828,9 +828,10 @@ qgemm_persist(const int8_t* __restrict__ wt, ColOps cols, const int8_t* __restri
               if constexpr (EPI == SDQ_EPI_GELU) {
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
+                  // columns past N are 0 or NaN (zero scale and bias), rows
+                  // past M are not written: neither needs a mask
                   v[r] = gelu_tanh(v[r]);
-                  const float av = ok ? fabsf(v[r]) : 0.f;
-                  rm[b][i] = rm[b][i] < av ? av : rm[b][i];
+                  rm[b][i] = fmaxf(rm[b][i], fabsf(v[r]));  // NaN never wins
                 }
               } else if constexpr (EPI == SDQ_EPI_GATED || EPI == SDQ_EPI_RESID) {
                 const v4f x = xa[b][i];
@@ -1454,7 +1455,10 @@ hipError_t launch_qgemm(int cfg, const int8_t* wt, const float* bs, const int8_t
                        N * 4 * 256 <= 0x7FFFFFF0;
   // Row maxima of a GELU output: written by the persistent kernels only
   // (not under split-K), one column chunk per wave column of each tile.
-  if (aux.rmax_chunks) *aux.rmax_chunks = 0;
+  if (aux.rmax_chunks) {
+    *aux.rmax_chunks = *aux.rmax_tail_chunks = 0;
+    *aux.rmax_tail_row = M;
+  }
   if (aux.tail) *aux.tail = 0;
   const bool rmax = epi.rmax && epi.kind == SDQ_EPI_GELU && persist && aux.splitk <= 1 &&
                     (cfg == kCfg128x128 || cfg == kCfg256x256) &&
@@ -1484,9 +1488,12 @@ hipError_t launch_qgemm(int cfg, const int8_t* wt, const float* bs, const int8_t
       if (persist) {
         // A last round of 256x256 tiles under half full: the rows of the
         // full rounds (whole m-tiles) run here, the rest as 128x128 tiles (a
-        // quarter of the work each, two per CU) right after. Not with row
-        // maxima (the two tile widths write different column chunks).
-        const int64_t Ma = epi_r.rmax ? 0 : tail_split_rows(M, N, aux.cu_count);
+        // quarter of the work each, two per CU) right after; its row maxima
+        // are over chunks of its own tiles' width (27280 rows, K = 3072, N =
+        // 14336 with row maxima: a round of 104 tiles, ~50 us, becomes 448
+        // narrow ones in 32 us).
+        int64_t Ma = tail_split_rows(M, N, aux.cu_count);
+        if (epi_r.rmax && gemm_rmax_chunks(kCfg128x128, N) > epi_r.rmax_stride) Ma = 0;
         if (Ma > 0) {
           hipError_t e = run_persist<256, 256, 2, 4, 2, 4, 1>(wt, cols, at, as, Ma, N, KFp, epi_r,
                                                               Y, aux.cu_count, s);
@@ -1495,9 +1502,27 @@ hipError_t launch_qgemm(int cfg, const int8_t* wt, const float* bs, const int8_t
           if (aux.mid && (e = hipEventRecord(aux.mid, s)) != hipSuccess) return e;
           EpiArgs et = epi_r;
           if (et.resid) et.resid += Ma * N;
-          return run_persist<128, 128, 2, 2, 2, 4, 2>(
-              wt, cols, at + (Ma / kFragRows) * KFp * kFragBytes, as + Ma, M - Ma, N, KFp, et,
-              static_cast<char*>(Y) + Ma * N * 4, 2 * aux.cu_count, s);
+          if (et.rmax) {
+            et.rmax += Ma * et.rmax_stride;
+            *aux.rmax_tail_row = Ma;
+            *aux.rmax_tail_chunks = gemm_rmax_chunks(kCfg128x128, N);
+          }
+          const int8_t* att = at + (Ma / kFragRows) * KFp * kFragBytes;
+          void* Yt = static_cast<char*>(Y) + Ma * N * 4;
+          if (aux.tail_splitk > 1 && aux.tail_part) {
+            // few tiles with long K (27280 rows, K = 14336, N = 3072: 48 tiles,
+            // 62 us on 48 CUs, 24 us as four k-ranges and their sum)
+            EpiArgs acc_epi = et;
+            acc_epi.kind = SDQ_EPI_ACC;
+            e = run_persist<128, 128, 2, 2, 2, 4, 2>(wt, cols, att, as + Ma, M - Ma, N, KFp,
+                                                     acc_epi, aux.tail_part, 2 * aux.cu_count, s,
+                                                     aux.tail_splitk);
+            if (e != hipSuccess) return e;
+            return run_splitk_reduce(aux.tail_part, aux.tail_splitk, M - Ma, N, as + Ma, bs, et,
+                                     Yt, s);
+          }
+          return run_persist<128, 128, 2, 2, 2, 4, 2>(wt, cols, att, as + Ma, M - Ma, N, KFp, et,
+                                                      Yt, 2 * aux.cu_count, s);
         }
         return run_persist<256, 256, 2, 4, 2, 4, 1>(wt, cols, at, as, M, N, KFp, epi_r, Y,
                                                     aux.cu_count, s);

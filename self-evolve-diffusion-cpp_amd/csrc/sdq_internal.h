@@ -193,12 +193,14 @@ hipError_t launch_sdpa_packed(const float* q, int64_t ldq, const float* k, int64
                               int64_t Lk, int heads, hipStream_t s, int batch, void* scratch,
                               int cu_count);
 // Same output, with the row maxima already known: max_c rmax[row*rstride + c]
-// over c < rchunks (e.g. written by the producing GEMM's epilogue), so A is
+// over c < rchunks, from row tail_row on over c < tail_chunks (written by the
+// producing GEMM's epilogue, whose last rows may be narrower tiles), so A is
 // read once.
 hipError_t launch_act_quant_frags_premax(const float* A, int64_t M, int64_t K, int64_t Mp,
                                          int64_t KFp, int8_t* at, float* as, const ColCopy& cc,
                                          const float* rmax, int rchunks, int rstride,
-                                         int cu_count, hipStream_t s);
+                                         int64_t tail_row, int tail_chunks, int cu_count,
+                                         hipStream_t s);
 // Same quantizer, row-major int8 output [M,K] (parity API).
 hipError_t launch_act_quant_rowmajor(const float* A, int64_t M, int64_t K, int8_t* aq, float* as,
                                      hipStream_t s);
@@ -248,9 +250,15 @@ struct GemmAux {
   int splitk;  // choose_splitk's factor (1 = none)
   int* part;   // splitk x M x N int32 partial sums (splitk > 1)
   int* rmax_chunks;  // out (nullable): column chunks written to epi.rmax, 0 = none
+  // out (with rmax_chunks): from this row on there are rmax_tail_chunks
+  int64_t* rmax_tail_row;
+  int* rmax_tail_chunks;
   int* tail;         // out (nullable): 1 when a 256x256 launch handed its last rows to a
                      // second, 128x128 launch (two kernels ran), else 0
   hipEvent_t mid;    // nullable: recorded between those two launches (per-kernel timing)
+  // The second launch's split-K (1: none) and its partial sums.
+  int tail_splitk;
+  int* tail_part;
 };
 // Grouped persistent GEMM: up to kMaxGemmGroup independent problems with
 // the same K (KFp) in one launch of the 128x128 persistent kernel (each with

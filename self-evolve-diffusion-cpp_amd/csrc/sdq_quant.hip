@@ -293,8 +293,8 @@ template <int R, int NW, int CACHE, bool PRE, bool XF>
 __device__ __forceinline__ void
 act_quant_unit(const float* __restrict__ A, int64_t M, int64_t K, int64_t KFp, int vec,
                int8_t* __restrict__ out, float* __restrict__ as,
-               const float* __restrict__ pre, int pc, int pstride, LnModArgs lm,
-               const int64_t unit) {
+               const float* __restrict__ pre, int pc, int pstride, int64_t tail_row, int tail_pc,
+               LnModArgs lm, const int64_t unit) {
   static_assert(R == 8 || R == 16, "unit height");
   static_assert(!(PRE && XF), "given maxima are for the plain rows");
   constexpr int F = 32 / R;  // fragments per lane group
@@ -329,7 +329,7 @@ act_quant_unit(const float* __restrict__ A, int64_t M, int64_t K, int64_t KFp, i
   }
   if constexpr (PRE) {
     static_assert(!PRE || R == 8, "given maxima are read by the 8 lanes of a row");
-    mx = premax_row(pre + (row_ok ? row : 0) * pstride, pc, row_ok, l);
+    mx = premax_row(pre + (row_ok ? row : 0) * pstride, row < tail_row ? pc : tail_pc, row_ok, l);
   } else {
     // (loading several groups per iteration here measured slower at large
     // M: the extra VGPRs cost occupancy, 5 -> 3 waves per SIMD)
@@ -379,14 +379,15 @@ template <int R, int NW, int CACHE, bool PRE, bool XF>
 __global__ void __launch_bounds__(NW * 64)
 act_quant_units_kernel(const float* __restrict__ A, int64_t M, int64_t K, int64_t KFp, int vec,
                        int8_t* __restrict__ out, float* __restrict__ as, ColCopy cc,
-                       const float* __restrict__ pre, int pc, int pstride, LnModArgs lm) {
+                       const float* __restrict__ pre, int pc, int pstride, int64_t tail_row,
+                       int tail_pc, LnModArgs lm) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cc.CP;
        i += (int64_t)gridDim.x * blockDim.x) {
     if (cc.bias_pad) cc.bias_pad[i] = i < cc.N ? cc.bias[i] : 0.f;
     if (cc.gate_pad) cc.gate_pad[i] = i < cc.N ? cc.gate[i] : 0.f;
   }
-  act_quant_unit<R, NW, CACHE, PRE, XF>(A, M, K, KFp, vec, out, as, pre, pc, pstride, lm,
-                                        blockIdx.x);
+  act_quant_unit<R, NW, CACHE, PRE, XF>(A, M, K, KFp, vec, out, as, pre, pc, pstride, tail_row,
+                                        tail_pc, lm, blockIdx.x);
 }
 
 // Several independent quantizations in one launch (the inputs of Linears
@@ -408,7 +409,7 @@ act_quant_segs_kernel(QuantSegs segs) {
     if (cc.gate_pad) cc.gate_pad[c] = c < cc.N ? cc.gate[c] : 0.f;
   }
   act_quant_unit<kQuantRows, kQuantUnitWaves, kQuantUnitCache, false, false>(
-      g.A, g.M, g.K, g.KFp, g.vec, g.at, g.as, nullptr, 0, 0, LnModArgs{}, unit);
+      g.A, g.M, g.K, g.KFp, g.vec, g.at, g.as, nullptr, 0, 0, 0, 0, LnModArgs{}, unit);
 }
 
 // Split form of the fragment-layout quantizer for few rows, where one
@@ -457,7 +458,8 @@ template <int GPW>
 __global__ void __launch_bounds__(256)
 act_quant_emit_kernel(const float* __restrict__ A, int64_t M, int64_t K, int64_t KFp, int vec,
                       int C, int64_t items, const float* __restrict__ pmax, int pc, int pstride,
-                      int8_t* __restrict__ out, float* __restrict__ as, ColCopy cc) {
+                      int64_t tail_row, int tail_pc, int8_t* __restrict__ out,
+                      float* __restrict__ as, ColCopy cc) {
   constexpr int R = 8, F = 32 / R;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cc.CP;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -480,7 +482,8 @@ act_quant_emit_kernel(const float* __restrict__ A, int64_t M, int64_t K, int64_t
     const int64_t g = (int64_t)c * GPW + i;
     if (g < ng) load16(rowp, (g * F + sub) * 32 + kg, K, row_ok, vec != 0, v[i]);
   }
-  const float mx = premax_row(pmax + (row_ok ? row : 0) * pstride, pc, row_ok, l);
+  const float mx =
+      premax_row(pmax + (row_ok ? row : 0) * pstride, row < tail_row ? pc : tail_pc, row_ok, l);
   float sc = mx / 127.f;
   if (sc == 0.f) sc = 1.f;
   const float inv = 1.f / sc;
@@ -640,18 +643,18 @@ hipError_t launch_act_quant_frags(const float* A, int64_t M, int64_t K, int64_t 
       hipLaunchKernelGGL((act_quant_pmax_kernel<4>), dim3(blocks), dim3(256), 0, s, A, M, K, KFp,
                          vec, C, items, pmax);
       hipLaunchKernelGGL((act_quant_emit_kernel<4>), dim3(blocks), dim3(256), 0, s, A, M, K, KFp,
-                         vec, C, items, pmax, C, Cp, at, as, cc);
+                         vec, C, items, pmax, C, Cp, M, C, at, as, cc);
     } else {
       hipLaunchKernelGGL((act_quant_pmax_kernel<2>), dim3(blocks), dim3(256), 0, s, A, M, K, KFp,
                          vec, C, items, pmax);
       hipLaunchKernelGGL((act_quant_emit_kernel<2>), dim3(blocks), dim3(256), 0, s, A, M, K, KFp,
-                         vec, C, items, pmax, C, Cp, at, as, cc);
+                         vec, C, items, pmax, C, Cp, M, C, at, as, cc);
     }
     return hipGetLastError();
   }
   hipLaunchKernelGGL((act_quant_units_kernel<kQuantRows, kQuantUnitWaves, kQuantUnitCache, false, false>),
                      dim3((unsigned)units), dim3(kQuantUnitWaves * 64), 0, s, A, M, K, KFp, vec,
-                     at, as, cc, nullptr, 0, 0, LnModArgs{});
+                     at, as, cc, nullptr, 0, 0, 0, 0, LnModArgs{});
   return hipGetLastError();
 }
 
@@ -695,7 +698,7 @@ hipError_t launch_act_quant_frags_lnmod(const float* A, int64_t M, int64_t K, in
   LnModArgs lm{st, shift, scale};
   hipLaunchKernelGGL((act_quant_units_kernel<kQuantRows, kQuantUnitWaves, kQuantUnitCache, false, true>),
                      dim3((unsigned)units), dim3(kQuantUnitWaves * 64), 0, s, A, M, K, KFp, vec,
-                     at, as, cc, nullptr, 0, 0, lm);
+                     at, as, cc, nullptr, 0, 0, 0, 0, lm);
   return hipGetLastError();
 }
 
@@ -721,8 +724,10 @@ hipError_t launch_act_quant_frags_lnmod_rows(const float* A, int64_t M, int64_t 
 hipError_t launch_act_quant_frags_premax(const float* A, int64_t M, int64_t K, int64_t Mp,
                                          int64_t KFp, int8_t* at, float* as, const ColCopy& cc,
                                          const float* rmax, int rchunks, int rstride,
-                                         int cu_count, hipStream_t s) {
-  if (!rmax || rchunks < 1 || rstride < rchunks || (rstride & 3) || !aligned16(rmax))
+                                         int64_t tail_row, int tail_chunks, int cu_count,
+                                         hipStream_t s) {
+  if (!rmax || rchunks < 1 || rstride < rchunks || rstride < tail_chunks ||
+      (tail_row < M && tail_chunks < 1) || (rstride & 3) || !aligned16(rmax))
     return hipErrorInvalidValue;
   const int vec = (aligned16(A) && (K % 4) == 0) ? 1 : 0;
   const int64_t units = Mp / kQuantRows;
@@ -733,15 +738,15 @@ hipError_t launch_act_quant_frags_premax(const float* A, int64_t M, int64_t K, i
     const unsigned blocks = (unsigned)ceil_div(items, 4);
     if (split_gpw(Mp) == 4)
       hipLaunchKernelGGL((act_quant_emit_kernel<4>), dim3(blocks), dim3(256), 0, s, A, M, K, KFp,
-                         vec, C, items, rmax, rchunks, rstride, at, as, cc);
+                         vec, C, items, rmax, rchunks, rstride, tail_row, tail_chunks, at, as, cc);
     else
       hipLaunchKernelGGL((act_quant_emit_kernel<2>), dim3(blocks), dim3(256), 0, s, A, M, K, KFp,
-                         vec, C, items, rmax, rchunks, rstride, at, as, cc);
+                         vec, C, items, rmax, rchunks, rstride, tail_row, tail_chunks, at, as, cc);
     return hipGetLastError();
   }
   hipLaunchKernelGGL((act_quant_units_kernel<kQuantRows, kQuantUnitWaves, kQuantUnitCache, true, false>),
                      dim3((unsigned)units), dim3(kQuantUnitWaves * 64), 0, s, A, M, K, KFp, vec,
-                     at, as, cc, rmax, rchunks, rstride, LnModArgs{});
+                     at, as, cc, rmax, rchunks, rstride, tail_row, tail_chunks, LnModArgs{});
   return hipGetLastError();
 }
 
