@@ -774,21 +774,28 @@ bool read_spans(int fd, const std::vector<ReadSpan>& spans, int threads) {
 namespace {
 
 // sdq_qlinear_host's staging, per host thread and device, grown and never
-// shrunk (held until the process ends): a device block for the call's
-// arrays, a stream of its own, and two pinned host buffers through which
-// host arrays move in chunks (the copy of one chunk into pinned memory
-// overlaps the DMA of the previous one).
-constexpr size_t kHostBounce = size_t(16) << 20;  // bytes per pinned buffer
-struct HostStage {
+// shrunk (held until the process ends): slots of a stream, a device block and
+// a pinned host buffer each. A call goes through them in pieces of rows, a
+// slot's piece from the host copy into its pinned buffer to the one out of it,
+// so one piece's copies overlap the other pieces' DMAs, both directions of the
+// bus and the kernels.
+constexpr int kHostSlots = 4;
+constexpr size_t kHostBounce = size_t(8) << 20;  // bytes per pinned buffer
+struct HostSlot {
   hipStream_t stream = nullptr;
   char* dbuf = nullptr;
   size_t dbytes = 0;
-  char* pin[2] = {nullptr, nullptr};
-  hipEvent_t done[2] = {nullptr, nullptr};
+  char* pin = nullptr;
+  char* dpin = nullptr;  // its device address
+  hipEvent_t done = nullptr;
+};
+struct HostStage {
+  HostSlot slot[kHostSlots];
 };
 thread_local HostStage t_host_stage[kMaxDev];
 
-int host_stage_ready(HostStage& hs) {
+// The slot's stream, event, pinned buffer and `bytes` of device memory.
+int host_slot_ready(HostSlot& hs, size_t bytes) {
   hipError_t e = hipSuccess;
   if (!hs.stream) {
     e = hipStreamCreateWithFlags(&hs.stream, hipStreamNonBlocking);
@@ -797,52 +804,88 @@ int host_stage_ready(HostStage& hs) {
       return hip_error(e, "hipStreamCreate (host calls)");
     }
   }
-  for (int i = 0; i < 2; i++) {
-    if (!hs.pin[i]) {
-      void* p = nullptr;
-      e = hipHostMalloc(&p, kHostBounce, hipHostMallocDefault);
-      if (e != hipSuccess) return hip_error(e, "hipHostMalloc (host-call bounce)");
-      hs.pin[i] = static_cast<char*>(p);
+  if (!hs.pin) {
+    void* p = nullptr;
+    e = hipHostMalloc(&p, kHostBounce, hipHostMallocDefault);
+    if (e != hipSuccess) return hip_error(e, "hipHostMalloc (host-call bounce)");
+    void* d = nullptr;
+    e = hipHostGetDevicePointer(&d, p, 0);
+    if (e != hipSuccess) {
+      (void)hipHostFree(p);
+      return hip_error(e, "hipHostGetDevicePointer (host-call bounce)");
     }
-    if (!hs.done[i]) {
-      e = hipEventCreateWithFlags(&hs.done[i], hipEventDisableTiming);
-      if (e != hipSuccess) {
-        hs.done[i] = nullptr;
-        return hip_error(e, "hipEventCreate (host calls)");
-      }
+    hs.pin = static_cast<char*>(p);
+    hs.dpin = static_cast<char*>(d);
+  }
+  if (!hs.done) {
+    e = hipEventCreateWithFlags(&hs.done, hipEventDisableTiming);
+    if (e != hipSuccess) {
+      hs.done = nullptr;
+      return hip_error(e, "hipEventCreate (host calls)");
     }
+  }
+  if (bytes > hs.dbytes) {
+    // the slot's stream is idle here (every call ends synchronized)
+    if (hs.dbuf) (void)hipFree(hs.dbuf);
+    hs.dbuf = nullptr;
+    hs.dbytes = 0;
+    e = hipMalloc(&hs.dbuf, bytes);
+    if (e != hipSuccess) {
+      hs.dbuf = nullptr;
+      return hip_error(e, "hipMalloc (host-call buffers)");
+    }
+    hs.dbytes = bytes;
   }
   return SDQ_OK;
 }
 
-// Host -> device through the pinned buffers. A buffer is refilled only
+// Rows per piece: a quarter of the call's bytes, 1 MiB at least (a piece costs
+// ~12 us of launches), 3 MiB at most (the first piece's way in and the last
+// one's way out overlap nothing), 16 rows at least. Median of 41 calls, K = N =
+// 3072, in pieces of 384 KiB / by this rule / whole: 64 rows 109 / 86 / 91 us,
+// 256 rows 219 / 219 / 294; in pieces of 1.5 MiB / by this rule / whole: 1024
+// rows 838 / 730 / 1042.
+int64_t host_piece_rows(int64_t M, size_t row_bytes) {
+  const size_t bytes =
+      std::min(size_t(3) << 20, std::max(size_t(1) << 20, (size_t)M * row_bytes / 4));
+  const int64_t r = std::max<int64_t>(16, (int64_t)(bytes / row_bytes));
+  return std::min(M, round_up(ceil_div(M, ceil_div(M, r)), 16));
+}
+
+bool bytes_overlap(const void* a, size_t na, const void* b, size_t nb) {
+  const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return a && b && na && nb && x < y + nb && y < x + na;
+}
+
+// Host -> device through the first two slots' pinned buffers, on the first
+// one's stream. A buffer is refilled only
 // after the DMA that read it finished.
-int host_stage_h2d(HostStage& hs, char* dst, const void* src, size_t bytes) {
+int host_stage_h2d(HostSlot* hs, char* dst, const void* src, size_t bytes) {
   const char* p = static_cast<const char*>(src);
   for (size_t off = 0, c = 0; off < bytes; off += kHostBounce, c++) {
     const size_t len = bytes - off < kHostBounce ? bytes - off : kHostBounce;
     const int b = (int)(c & 1);
-    hipError_t e = hipEventSynchronize(hs.done[b]);
+    hipError_t e = hipEventSynchronize(hs[b].done);
     if (e == hipSuccess) {
-      std::memcpy(hs.pin[b], p + off, len);
-      e = hipMemcpyAsync(dst + off, hs.pin[b], len, hipMemcpyHostToDevice, hs.stream);
+      std::memcpy(hs[b].pin, p + off, len);
+      e = hipMemcpyAsync(dst + off, hs[b].pin, len, hipMemcpyHostToDevice, hs[0].stream);
     }
-    if (e == hipSuccess) e = hipEventRecord(hs.done[b], hs.stream);
+    if (e == hipSuccess) e = hipEventRecord(hs[b].done, hs[0].stream);
     if (e != hipSuccess) return hip_error(e, "host-call H2D");
   }
   return SDQ_OK;
 }
 
-// Device -> host through the pinned buffers: chunk c's DMA is queued before
+// Device -> host the same way: chunk c's DMA is queued before
 // chunk c-1 is copied out of its pinned buffer.
-int host_stage_d2h(HostStage& hs, void* dst, const char* src, size_t bytes) {
+int host_stage_d2h(HostSlot* hs, void* dst, const char* src, size_t bytes) {
   char* q = static_cast<char*>(dst);
   size_t prev_off = 0, prev_len = 0;
   int prev_b = -1;
   auto drain = [&]() {
     if (prev_b < 0) return hipSuccess;
-    hipError_t e = hipEventSynchronize(hs.done[prev_b]);
-    if (e == hipSuccess) std::memcpy(q + prev_off, hs.pin[prev_b], prev_len);
+    hipError_t e = hipEventSynchronize(hs[prev_b].done);
+    if (e == hipSuccess) std::memcpy(q + prev_off, hs[prev_b].pin, prev_len);
     prev_b = -1;
     return e;
   };
@@ -850,8 +893,8 @@ int host_stage_d2h(HostStage& hs, void* dst, const char* src, size_t bytes) {
     const size_t len = bytes - off < kHostBounce ? bytes - off : kHostBounce;
     const int b = (int)(c & 1);
     // buffer b last held chunk c-2, copied out when chunk c-1 was queued
-    hipError_t e = hipMemcpyAsync(hs.pin[b], src + off, len, hipMemcpyDeviceToHost, hs.stream);
-    if (e == hipSuccess) e = hipEventRecord(hs.done[b], hs.stream);
+    hipError_t e = hipMemcpyAsync(hs[b].pin, src + off, len, hipMemcpyDeviceToHost, hs[0].stream);
+    if (e == hipSuccess) e = hipEventRecord(hs[b].done, hs[0].stream);
     if (e == hipSuccess) e = drain();
     if (e != hipSuccess) return hip_error(e, "host-call D2H");
     prev_off = off;
@@ -1844,48 +1887,101 @@ int sdq_qlinear_host(const sdq_weight* w, const float* A, int64_t M, int64_t K,
   int dev = -1;
   if ((rc = current_device(&dev))) return rc;
   if ((rc = ensure_device(dev))) return rc;
-  HostStage& hs = t_host_stage[dev];
-  if ((rc = host_stage_ready(hs))) return rc;
-  const size_t abytes = (size_t)(M * K) * 4, ybytes = (size_t)(M * N) * 4;
-  // one device block: A | Y | resid | bias | gate, each 256-byte aligned
+  HostSlot* hs = t_host_stage[dev].slot;
   auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
-  const bool has_resid = epi && epi->resid;
-  const size_t o_y = al(abytes), o_r = o_y + al(ybytes), o_b = o_r + (has_resid ? al(ybytes) : 0);
-  const size_t o_g = o_b + al((size_t)N * 4), total = o_g + al((size_t)N * 4);
-  if (total > hs.dbytes) {
-    // the stage's stream is idle here (every call ends synchronized)
-    if (hs.dbuf) (void)hipFree(hs.dbuf);
-    hs.dbuf = nullptr;
-    hs.dbytes = 0;
-    hipError_t e = hipMalloc(&hs.dbuf, total);
-    if (e != hipSuccess) {
-      hs.dbuf = nullptr;
-      return hip_error(e, "hipMalloc (host-call buffers)");
-    }
-    hs.dbytes = total;
-  }
-  char* buf = hs.dbuf;
+  const bool has_resid = epi && epi->resid, has_bias = epi && epi->bias, has_gate = epi && epi->gate;
   sdq_epilogue de{};
   if (epi) de = *epi;
+
+  // By pieces of rows, where one fits a pinned buffer and no output row lands
+  // on an input that a later piece still reads (a residual updated in place
+  // does not).
+  const size_t arow = (size_t)K * 4, yrow = (size_t)N * 4, row = arow + yrow * (has_resid ? 2 : 1);
+  const int64_t R = host_piece_rows(M, row);
+  // a slot's pinned and device layout: bias | gate | A | resid | Y
+  const size_t o_gate = has_bias ? al(yrow) : 0, o_a = o_gate + (has_gate ? al(yrow) : 0);
+  const size_t o_res = o_a + al((size_t)R * arow), o_y = o_res + (has_resid ? al((size_t)R * yrow) : 0);
+  const size_t slot_bytes = o_y + al((size_t)R * yrow);
+  const size_t abytes = (size_t)M * arow, ybytes = (size_t)M * yrow;
+  const bool pieces =
+      slot_bytes <= kHostBounce && !bytes_overlap(Y, ybytes, A, abytes) &&
+      !(has_bias && bytes_overlap(Y, ybytes, epi->bias, yrow)) &&
+      !(has_gate && bytes_overlap(Y, ybytes, epi->gate, yrow)) &&
+      !(has_resid && epi->resid != Y && bytes_overlap(Y, ybytes, epi->resid, ybytes));
+  if (pieces) {
+    const int n = (int)ceil_div(M, R), used = std::min(n, kHostSlots);
+    for (int i = 0; i < used; i++)
+      if ((rc = host_slot_ready(hs[i], slot_bytes))) return rc;
+    auto drain = [&](int i) {
+      HostSlot& h = hs[i % kHostSlots];
+      const int64_t r0 = i * R;
+      const hipError_t e = hipEventSynchronize(h.done);
+      if (e != hipSuccess) return hip_error(e, "host-call D2H");
+      std::memcpy(static_cast<char*>(Y) + r0 * yrow, h.pin + o_y, std::min(R, M - r0) * yrow);
+      return (int)SDQ_OK;
+    };
+    int i = 0, out = 0;  // pieces queued, pieces copied out
+    for (; i < n && !rc; i++) {
+      if (i >= kHostSlots && (rc = drain(out++))) break;
+      HostSlot& h = hs[i % kHostSlots];
+      const int64_t r0 = i * R, m = std::min(R, M - r0);
+      size_t lo = o_a;
+      if (i < kHostSlots && o_a) {  // the slot's first piece of the call
+        lo = 0;
+        if (has_bias) std::memcpy(h.pin, epi->bias, yrow);
+        if (has_gate) std::memcpy(h.pin + o_gate, epi->gate, yrow);
+      }
+      std::memcpy(h.pin + o_a, reinterpret_cast<const char*>(A) + r0 * arow, m * arow);
+      if (has_resid)
+        std::memcpy(h.pin + o_res, reinterpret_cast<const char*>(epi->resid) + r0 * yrow, m * yrow);
+      const size_t hi = has_resid ? o_res + m * yrow : o_a + m * arow;
+      hipError_t e = launch_bus_copy(h.dbuf + lo, h.dpin + lo, hi - lo, h.stream);
+      if (e != hipSuccess) {
+        rc = hip_error(e, "host-call H2D");
+        break;
+      }
+      if (has_bias) de.bias = reinterpret_cast<float*>(h.dbuf);
+      if (has_gate) de.gate = reinterpret_cast<float*>(h.dbuf + o_gate);
+      if (has_resid) de.resid = reinterpret_cast<float*>(h.dbuf + o_res);
+      if ((rc = qlinear_device(w, reinterpret_cast<float*>(h.dbuf + o_a), m, K,
+                               epi ? &de : nullptr, h.dbuf + o_y, h.stream)))
+        break;
+      e = launch_bus_copy(h.dpin + o_y, h.dbuf + o_y, m * yrow, h.stream);
+      if (e == hipSuccess) e = hipEventRecord(h.done, h.stream);
+      if (e != hipSuccess) rc = hip_error(e, "host-call D2H");
+    }
+    while (!rc && out < n) rc = drain(out++);
+    if (!rc) return SDQ_OK;  // every slot drained: idle
+    // leave the stage idle whatever happened
+    for (int k = 0; k < used; k++) (void)hipStreamSynchronize(hs[k].stream);
+    return rc;
+  }
+
+  // Whole: every input is on the device before the first output row is written.
+  // One device block: A | Y | resid | bias | gate, each 256-byte aligned.
+  const size_t w_y = al(abytes), w_r = w_y + al(ybytes), w_b = w_r + (has_resid ? al(ybytes) : 0);
+  const size_t w_g = w_b + al(yrow), total = w_g + al(yrow);
+  if ((rc = host_slot_ready(hs[0], total)) || (rc = host_slot_ready(hs[1], 0))) return rc;
+  char* buf = hs[0].dbuf;
   rc = host_stage_h2d(hs, buf, A, abytes);
   if (!rc && has_resid) {
-    rc = host_stage_h2d(hs, buf + o_r, epi->resid, ybytes);
-    de.resid = reinterpret_cast<float*>(buf + o_r);
+    rc = host_stage_h2d(hs, buf + w_r, epi->resid, ybytes);
+    de.resid = reinterpret_cast<float*>(buf + w_r);
   }
-  if (!rc && epi && epi->bias) {
-    rc = host_stage_h2d(hs, buf + o_b, epi->bias, (size_t)N * 4);
-    de.bias = reinterpret_cast<float*>(buf + o_b);
+  if (!rc && has_bias) {
+    rc = host_stage_h2d(hs, buf + w_b, epi->bias, yrow);
+    de.bias = reinterpret_cast<float*>(buf + w_b);
   }
-  if (!rc && epi && epi->gate) {
-    rc = host_stage_h2d(hs, buf + o_g, epi->gate, (size_t)N * 4);
-    de.gate = reinterpret_cast<float*>(buf + o_g);
+  if (!rc && has_gate) {
+    rc = host_stage_h2d(hs, buf + w_g, epi->gate, yrow);
+    de.gate = reinterpret_cast<float*>(buf + w_g);
   }
   if (!rc)
-    rc = qlinear_device(w, reinterpret_cast<float*>(buf), M, K, epi ? &de : nullptr, buf + o_y,
-                        hs.stream);
-  if (!rc) rc = host_stage_d2h(hs, Y, buf + o_y, ybytes);
+    rc = qlinear_device(w, reinterpret_cast<float*>(buf), M, K, epi ? &de : nullptr, buf + w_y,
+                        hs[0].stream);
+  if (!rc) rc = host_stage_d2h(hs, Y, buf + w_y, ybytes);
   // leave the stage idle whatever happened
-  const hipError_t e = hipStreamSynchronize(hs.stream);
+  const hipError_t e = hipStreamSynchronize(hs[0].stream);
   if (!rc && e != hipSuccess) rc = hip_error(e, "hipStreamSynchronize (host call)");
   return rc;
 }

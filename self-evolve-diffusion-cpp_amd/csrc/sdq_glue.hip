@@ -393,6 +393,18 @@ resid2_kernel(float* __restrict__ x, int64_t n4, int64_t N4, ResidStep a, ResidS
   reinterpret_cast<v4f_t*>(x)[i] = v;
 }
 
+
+// A piece of a host call's arrays over the bus, read or written by the compute
+// units: bound by the bus, 3.1 MB alone 68 us either way (46 GB/s; a DMA
+// engine's 63), but ~6 us a copy less than an engine's start and signal, which
+// the small pieces that overlap feel: 256 rows of 3072 in and out 250 -> 220
+// us, 16 rows 61 -> 44. 64 workgroups keep the bus busy (16: 226, 256: 229)
+// and leave the other pieces' kernels their compute units.
+__global__ void __launch_bounds__(256)
+bus_copy_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, uint32_t n) {
+  for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
+}
+
 }  // namespace
 
 bool ln_rows_fits(const float* x, int64_t M, int64_t K, const float* w, const float* b,
@@ -424,6 +436,15 @@ hipError_t launch_ln_apply(const float* x, int64_t M, int64_t K, const float2* s
 hipError_t launch_add(float* x, const float* y, int64_t n, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(add_kernel, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, s, x, y, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_bus_copy(void* dst, const void* src, size_t bytes, hipStream_t s) {
+  if (!bytes) return hipSuccess;
+  if (!aligned16(dst) || !aligned16(src) || bytes > (size_t(1) << 32)) return hipErrorInvalidValue;
+  const uint32_t n = (uint32_t)((bytes + 15) / 16);
+  hipLaunchKernelGGL(bus_copy_kernel, dim3(std::min(64u, (n + 255) / 256)), dim3(256), 0, s,
+                     static_cast<const uint4*>(src), static_cast<uint4*>(dst), n);
   return hipGetLastError();
 }
 

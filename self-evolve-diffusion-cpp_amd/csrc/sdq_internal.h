@@ -201,6 +201,9 @@ hipError_t launch_act_quant_frags_premax(const float* A, int64_t M, int64_t K, i
                                          const float* rmax, int rchunks, int rstride,
                                          int64_t tail_row, int tail_chunks, int cu_count,
                                          hipStream_t s);
+// Copies bytes, rounded up to 16, between device memory and a pinned host
+// buffer (its device address), both 16-byte aligned.
+hipError_t launch_bus_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
 // Same quantizer, row-major int8 output [M,K] (parity API).
 hipError_t launch_act_quant_rowmajor(const float* A, int64_t M, int64_t K, int8_t* aq, float* as,
                                      hipStream_t s);
