@@ -774,12 +774,16 @@ bool read_spans(int fd, const std::vector<ReadSpan>& spans, int threads) {
 namespace {
 
 // sdq_qlinear_host's staging, per host thread and device, grown and never
-// shrunk (held until the process ends): slots of a stream, a device block and
-// a pinned host buffer each. A call goes through them in pieces of rows, a
-// slot's piece from the host copy into its pinned buffer to the one out of it,
-// so one piece's copies overlap the other pieces' DMAs, both directions of the
-// bus and the kernels.
+// shrunk (held until the process ends): slots of a device block and a pinned
+// host buffer each, on two streams in turn. A call goes through them in pieces
+// of rows, a slot's piece from the host copy into its pinned buffer to the one
+// out of it, so one piece's copies overlap the other pieces' DMAs, both
+// directions of the bus and the kernels. Two streams carry all of that (256
+// rows of 3072 in and out: 216 us, with a stream per slot 222) and leave two of
+// the process's four hardware queues: with a stream per slot, a program's own
+// two streams shared one (a twin layer's stack 297 -> 326 us).
 constexpr int kHostSlots = 4;
+constexpr int kHostStreams = 2;
 constexpr size_t kHostBounce = size_t(8) << 20;  // bytes per pinned buffer
 struct HostSlot {
   hipStream_t stream = nullptr;
@@ -794,9 +798,12 @@ struct HostStage {
 };
 thread_local HostStage t_host_stage[kMaxDev];
 
-// The slot's stream, event, pinned buffer and `bytes` of device memory.
-int host_slot_ready(HostSlot& hs, size_t bytes) {
+// Slot i's stream, event, pinned buffer and `bytes` of device memory.
+int host_slot_ready(HostSlot* slots, int i, size_t bytes) {
+  HostSlot& hs = slots[i];
   hipError_t e = hipSuccess;
+  // (slots are made ready in order)
+  if (!hs.stream && i >= kHostStreams) hs.stream = slots[i % kHostStreams].stream;
   if (!hs.stream) {
     e = hipStreamCreateWithFlags(&hs.stream, hipStreamNonBlocking);
     if (e != hipSuccess) {
@@ -825,7 +832,7 @@ int host_slot_ready(HostSlot& hs, size_t bytes) {
     }
   }
   if (bytes > hs.dbytes) {
-    // the slot's stream is idle here (every call ends synchronized)
+    // the slot is idle here (every call ends synchronized)
     if (hs.dbuf) (void)hipFree(hs.dbuf);
     hs.dbuf = nullptr;
     hs.dbytes = 0;
@@ -1911,7 +1918,7 @@ int sdq_qlinear_host(const sdq_weight* w, const float* A, int64_t M, int64_t K,
   if (pieces) {
     const int n = (int)ceil_div(M, R), used = std::min(n, kHostSlots);
     for (int i = 0; i < used; i++)
-      if ((rc = host_slot_ready(hs[i], slot_bytes))) return rc;
+      if ((rc = host_slot_ready(hs, i, slot_bytes))) return rc;
     auto drain = [&](int i) {
       HostSlot& h = hs[i % kHostSlots];
       const int64_t r0 = i * R;
@@ -1961,7 +1968,7 @@ int sdq_qlinear_host(const sdq_weight* w, const float* A, int64_t M, int64_t K,
   // One device block: A | Y | resid | bias | gate, each 256-byte aligned.
   const size_t w_y = al(abytes), w_r = w_y + al(ybytes), w_b = w_r + (has_resid ? al(ybytes) : 0);
   const size_t w_g = w_b + al(yrow), total = w_g + al(yrow);
-  if ((rc = host_slot_ready(hs[0], total)) || (rc = host_slot_ready(hs[1], 0))) return rc;
+  if ((rc = host_slot_ready(hs, 0, total)) || (rc = host_slot_ready(hs, 1, 0))) return rc;
   char* buf = hs[0].dbuf;
   rc = host_stage_h2d(hs, buf, A, abytes);
   if (!rc && has_resid) {
