@@ -1,6 +1,6 @@
 """Row norms whose rows stay in registers (up to 3072 columns): layernorm,
 rmsnorm + RoPE and the norm + modulation quantizer at the edges of their
-workgroups (14 rows), chunks (256 columns; 4, 8 or 12 held) and limit,
+workgroups (14 rows), chunks (256 columns; 2, 4, 6, .. 12 held) and limit,
 bit-exact against the oracle, with the first shapes past the limit beside
 them."""
 import numpy as np
@@ -19,7 +19,8 @@ def _x(oracle, M, K, seed):
 
 @pytest.mark.parametrize("M,K", [(1, 4), (13, 256), (14, 260), (15, 1024), (29, 1028), (3, 2044),
                                  (28, 2048), (16, 2052), (14, 3068), (43, 3072), (15, 3076),
-                                 (14, 3074)])
+                                 (14, 3074), (29, 508), (14, 512), (1, 516), (15, 1536),
+                                 (14, 1540), (43, 2560), (15, 2564)])
 def test_rows_bitexact(sdq_dev, oracle, M, K):
     import torch
 
