@@ -13,9 +13,9 @@
 // 3072-column chain is ~7 us). It replaces, for rows of up to 3072 columns, a
 // statistics kernel that reads the rows once per sum and an apply kernel. us
 // before and after, 3072 columns: rmsnorm + RoPE of q and k at 27280 rows 531,
-// 280 (4.8 TB/s), at 768 rows 26, 19.5; layernorm at 27280 rows 354, 180, at
-// 157 rows 29, 24; norm + modulation + quantizer at 27280 rows 196, 150-170,
-// at 4099 rows 60, 41, at 768 rows 35, 28.
+// 280 (4.8 TB/s), at 768 rows 26, 18.3; layernorm at 27280 rows 354, 180, at
+// 157 rows 29, 22.5; norm + modulation + quantizer at 27280 rows 196, 150-170,
+// at 4099 rows 60, 41, at 768 rows 35, 26.7.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -77,7 +77,7 @@ __device__ __forceinline__ float quad16_sum(float v) {
 }
 
 // One workgroup per (key block, head, sequence): K scaled by the block's
-// power of two and split into fp16 parts, V split into bf16 parts, both in
+// power of two and split into fp16 parts, V the same, both in
 // the order the MFMA operands are read (16 bytes per lane):
 //   K [part][32-dim step d][16-key tile kt][lane]: key 16 kt + lane % 16,
 //     dims 32 d + 8 (lane / 16) + 0..7
