@@ -1860,7 +1860,7 @@ int sdq_sdpa_batched(const float* q, int64_t ldq, const float* k, int64_t ldk, c
   hipEvent_t p0 = t_prof ? prof_mark(s) : nullptr;
   const hipError_t e =
       scratch ? launch_sdpa_packed(q, ldq, k, ldk, v, ldv, out, ldo, Lq, Lk, heads, s, batch,
-                                   scratch, cu_count)
+                                   scratch, need, cu_count)
               : launch_sdpa(q, ldq, k, ldk, v, ldv, out, ldo, Lq, Lk, heads, s, batch);
   if (e != hipSuccess) {
     drop_events({p0});

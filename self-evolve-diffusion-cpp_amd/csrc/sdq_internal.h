@@ -191,7 +191,7 @@ int64_t sdpa_packed_bytes(int64_t Lq, int64_t Lk, int heads, int batch, int cu_c
 hipError_t launch_sdpa_packed(const float* q, int64_t ldq, const float* k, int64_t ldk,
                               const float* v, int64_t ldv, float* out, int64_t ldo, int64_t Lq,
                               int64_t Lk, int heads, hipStream_t s, int batch, void* scratch,
-                              int cu_count);
+                              int64_t scratch_bytes, int cu_count);
 // Same output, with the row maxima already known: max_c rmax[row*rstride + c]
 // over c < rchunks, from row tail_row on over c < tail_chunks (written by the
 // producing GEMM's epilogue, whose last rows may be narrower tiles), so A is

@@ -18,8 +18,7 @@
 // 32x32x16 ones took 20.7 ms (fewer accumulator bits switch, a higher clock).
 #include "sdq_internal.h"
 #include "sdq_device.h"
-
-#include <cstdlib>
+#include "sdq_sdpa_plan.h"
 
 #pragma clang fp contract(off)
 
@@ -31,13 +30,15 @@ typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
-constexpr int kHd = 128;             // head dim
-constexpr int kKB = 32;              // keys per block
-constexpr int kRec = 32768;          // bytes of a packed block: K parts, V parts
+using sdpa::kHd;
+using sdpa::kKB;
+using sdpa::kQ;
+using sdpa::kRec;
+using sdpa::Plan;
 constexpr int kRecV = 16384;         // V's offset in it
 constexpr int kPart = 8192;          // one part (hi or lo) of K or V
 constexpr int kWaves = 8;
-constexpr int kQ = 32 * kWaves;      // queries per workgroup
+static_assert(kQ == 32 * kWaves);
 constexpr int kRing = 4;             // blocks of K and of V in LDS
 // K and Q are scaled by powers of two so that the largest element of a key
 // block (of a query row) lies in [2^14, 2^15): their fp16 low parts then stay
@@ -161,20 +162,6 @@ sdpa_pack_kernel(const float* __restrict__ K, int64_t ldk, const float* __restri
   }
 }
 
-// How a sequence's items (256 queries of one head, all its key blocks) are
-// spread over workgroups. The first nfull items, whole rounds of the CUs, run
-// whole. The others, which would fill only part of a round, are cut by keys
-// into `splits` shares of kbs blocks (splits = 1: not cut); a share leaves its
-// unnormalized output and its (reference, sum) pair in slot (item - nfull) *
-// splits + share, and sdpa_combine_kernel adds up an item's shares.
-struct Plan {
-  int nkb;      // key blocks
-  int qgroups;  // items per head
-  int items;    // heads * qgroups
-  int nfull;
-  int splits;
-  int kbs;
-};
 struct Parts {
   float* o;    // [seq][slots][256][128]
   float2* ml;  // [seq][slots][256]: (reference, sum), base 2
@@ -618,95 +605,29 @@ sdpa_combine_kernel(Plan plan, Parts parts, int64_t Lq, float* __restrict__ O, i
       float4{inv(o.x), inv(o.y), inv(o.z), inv(o.w)};
 }
 
-// Depends on the sequence only, not on the batch, so stacked and separate
-// calls give the same bits.
-Plan make_plan(int64_t Lq, int64_t Lk, int heads, int cu_count) {
-  Plan p{};
-  p.nkb = (int)ceil_div(Lk, kKB);
-  p.qgroups = (int)ceil_div(Lq, kQ);
-  p.items = heads * p.qgroups;
-  p.splits = 1;
-  p.kbs = p.nkb;
-  const int cus = cu_count > 0 ? cu_count : 256;
-  p.nfull = p.items / cus * cus;
-  const int rest = p.items - p.nfull;
-  if (rest == 0 || std::getenv("SDQ_SDPA_SPLIT")) {  // the variable: comparisons without shares
-    p.nfull = p.items;
-    return p;
-  }
-  // The cut that ends first, in key-block times: rounds of shares, each with
-  // its own start and end (about 3 blocks), plus the second pass over the
-  // partial outputs.
-  double best = p.nkb + 3;
-  for (int S = 2; S <= 32 && 3 * S <= p.nkb; S++) {
-    const int kbs = (int)ceil_div(p.nkb, S);
-    if (ceil_div(p.nkb, kbs) != S) continue;  // no empty share
-    const double cost = (double)ceil_div((int64_t)rest * S, cus) * (kbs + 3) + 3;
-    if (cost < best) best = cost, p.splits = S, p.kbs = kbs;
-  }
-  return p;
-}
-
-int64_t pad256(int64_t n) { return (n + 255) / 256 * 256; }
-
-// Scratch of one launch over `heads` heads of `batch` sequences.
-struct Layout {
-  int64_t exps, o, ml, bytes;  // offsets of its parts (the records lie at 0)
-};
-Layout layout(const Plan& p, int64_t heads, int64_t batch) {
-  const int64_t recs = batch * heads * p.nkb;
-  const int64_t rows =
-      p.splits > 1 ? batch * (p.items - p.nfull) * p.splits * (int64_t)kQ : 0;
-  Layout l;
-  l.exps = recs * kRec;
-  l.o = l.exps + pad256(recs * 8);
-  l.ml = l.o + rows * kHd * 4;
-  l.bytes = l.ml + rows * 8;
-  return l;
-}
-
-// A call runs in launches of as many sequences, or of as many heads of one
-// sequence, as keep their records within kMaxRecs bytes, so the scratch a
-// stream holds is bounded (heads: a sequence's own share, so that it does
-// not depend on the batch).
-constexpr int64_t kMaxRecs = int64_t(1) << 31;
-struct Chunk {
-  int heads, seqs;
-};
-Chunk chunk(int64_t nkb, int heads, int batch) {
-  const int64_t per_head = nkb * kRec;
-  const int64_t h = kMaxRecs / per_head < 1 ? 1 : kMaxRecs / per_head;
-  if (h < heads) return {(int)h, 1};
-  const int64_t n = kMaxRecs / (per_head * heads);
-  return {heads, (int)(n < batch ? n : batch)};
-}
-
 }  // namespace
 
 int64_t sdpa_packed_bytes(int64_t Lq, int64_t Lk, int heads, int batch, int cu_count) {
-  // a head's records are addressed with 32-bit offsets; a grid holds 2^32 threads
-  if (Lk > kMaxRecs / kRec * kKB || heads > 65535 || ceil_div(Lq, kQ) * heads > (1 << 22))
-    return 0;
-  const Chunk c = chunk(ceil_div(Lk, kKB), heads, batch);
-  return layout(make_plan(Lq, Lk, c.heads, cu_count), c.heads, c.seqs).bytes;
+  return sdpa::scratch_bytes(Lq, Lk, heads, batch, cu_count);
 }
 
 hipError_t launch_sdpa_packed(const float* q, int64_t ldq, const float* k, int64_t ldk,
                               const float* v, int64_t ldv, float* out, int64_t ldo, int64_t Lq,
                               int64_t Lk, int heads, hipStream_t s, int batch, void* scratch,
-                              int cu_count) {
+                              int64_t scratch_bytes, int cu_count) {
   if (Lq <= 0 || batch <= 0) return hipSuccess;
   if (Lk <= 0 || heads <= 0 || heads > 65535 || batch > 65535 || !scratch)
     return hipErrorInvalidValue;
   const float scale_log2e = (1.f / sqrtf((float)kHd)) * 1.4426950408889634f;
-  const Chunk ch = chunk(ceil_div(Lk, kKB), heads, batch);
+  const sdpa::Chunk ch = sdpa::chunk(ceil_div(Lk, kKB), heads, batch);
   char* packed = static_cast<char*>(scratch);
   for (int b0 = 0; b0 < batch; b0 += ch.seqs)
     for (int h0 = 0; h0 < heads; h0 += ch.heads) {
       const int nb = batch - b0 < ch.seqs ? batch - b0 : ch.seqs;
       const int nh = heads - h0 < ch.heads ? heads - h0 : ch.heads;
-      const Plan p = make_plan(Lq, Lk, nh, cu_count);
-      const Layout l = layout(p, nh, nb);
+      const Plan p = sdpa::make_plan(Lq, Lk, nh, cu_count);
+      const sdpa::Layout l = sdpa::layout(p, nh, nb);
+      if (l.bytes > scratch_bytes) return hipErrorInvalidValue;
       int2* exps = reinterpret_cast<int2*>(packed + l.exps);
       const Parts parts{reinterpret_cast<float*>(packed + l.o),
                         reinterpret_cast<float2*>(packed + l.ml)};

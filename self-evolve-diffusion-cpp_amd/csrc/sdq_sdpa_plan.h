@@ -1,0 +1,111 @@
+// Host side of the packed attention (sdq_sdpa.hip): how a call is spread over
+// workgroups and what scratch that takes. Plain C++, so that it is checked
+// without a GPU.
+#pragma once
+
+#include <cstdint>
+#include <cstdlib>
+
+namespace sdq {
+namespace sdpa {
+
+constexpr int kHd = 128;     // head dim
+constexpr int kKB = 32;      // keys per block
+constexpr int kQ = 256;      // queries per workgroup
+constexpr int kRec = 32768;  // bytes of a packed block: K parts, V parts
+
+inline int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+inline int64_t pad256(int64_t n) { return div_up(n, 256) * 256; }
+
+// How a sequence's items (256 queries of one head, all its key blocks) are
+// spread over workgroups. The first nfull items, whole rounds of the CUs, run
+// whole. The others, which would fill only part of a round, are cut by keys
+// into `splits` shares of kbs blocks (splits = 1: not cut); a share leaves its
+// unnormalized output and its (reference, sum) pair in slot (item - nfull) *
+// splits + share, and sdpa_combine_kernel adds up an item's shares.
+struct Plan {
+  int nkb;      // key blocks
+  int qgroups;  // items per head
+  int items;    // heads * qgroups
+  int nfull;
+  int splits;
+  int kbs;
+};
+// Depends on the sequence only, not on the batch, so stacked and separate
+// calls give the same bits.
+inline Plan make_plan(int64_t Lq, int64_t Lk, int heads, int cu_count) {
+  Plan p{};
+  p.nkb = (int)div_up(Lk, kKB);
+  p.qgroups = (int)div_up(Lq, kQ);
+  p.items = heads * p.qgroups;
+  p.splits = 1;
+  p.kbs = p.nkb;
+  const int cus = cu_count > 0 ? cu_count : 256;
+  p.nfull = p.items / cus * cus;
+  const int rest = p.items - p.nfull;
+  if (rest == 0 || std::getenv("SDQ_SDPA_SPLIT")) {  // the variable: comparisons without shares
+    p.nfull = p.items;
+    return p;
+  }
+  // The cut that ends first, in key-block times: rounds of shares, each with
+  // its own start and end (about 3 blocks), plus the second pass over the
+  // partial outputs.
+  double best = p.nkb + 3;
+  for (int S = 2; S <= 32 && 3 * S <= p.nkb; S++) {
+    const int kbs = (int)div_up(p.nkb, S);
+    if (div_up(p.nkb, kbs) != S) continue;  // no empty share
+    const double cost = (double)div_up((int64_t)rest * S, cus) * (kbs + 3) + 3;
+    if (cost < best) best = cost, p.splits = S, p.kbs = kbs;
+  }
+  return p;
+}
+
+// Scratch of one launch over `heads` heads of `batch` sequences.
+struct Layout {
+  int64_t exps, o, ml, bytes;  // offsets of its parts (the records lie at 0)
+};
+inline Layout layout(const Plan& p, int64_t heads, int64_t batch) {
+  const int64_t recs = batch * heads * p.nkb;
+  const int64_t rows =
+      p.splits > 1 ? batch * (p.items - p.nfull) * p.splits * (int64_t)kQ : 0;
+  Layout l;
+  l.exps = recs * kRec;
+  l.o = l.exps + pad256(recs * 8);
+  l.ml = l.o + rows * kHd * 4;
+  l.bytes = l.ml + rows * 8;
+  return l;
+}
+
+// A call runs in launches of as many sequences, or of as many heads of one
+// sequence, as keep their records within kMaxRecs bytes, so the scratch a
+// stream holds is bounded (heads: a sequence's own share, so that it does
+// not depend on the batch).
+constexpr int64_t kMaxRecs = int64_t(1) << 31;
+struct Chunk {
+  int heads, seqs;
+};
+inline Chunk chunk(int64_t nkb, int heads, int batch) {
+  const int64_t per_head = nkb * kRec;
+  const int64_t h = kMaxRecs / per_head < 1 ? 1 : kMaxRecs / per_head;
+  if (h < heads) return {(int)h, 1};
+  const int64_t n = kMaxRecs / (per_head * heads);
+  return {heads, (int)(n < batch ? n : batch)};
+}
+
+// Bytes that every launch of a call fits in; 0: the packed form does not take
+// it. A last chunk of fewer heads has a plan of its own, whose shares' outputs
+// can outweigh the records that the missing heads leave free.
+inline int64_t scratch_bytes(int64_t Lq, int64_t Lk, int heads, int batch, int cu_count) {
+  // a head's records are addressed with 32-bit offsets; a grid holds 2^32 threads
+  if (Lk > kMaxRecs / kRec * kKB || heads > 65535 || div_up(Lq, kQ) * heads > (1 << 22)) return 0;
+  const Chunk c = chunk(div_up(Lk, kKB), heads, batch);
+  int64_t most = 0;
+  for (const int h : {c.heads, heads % c.heads}) {
+    const int64_t b = h ? layout(make_plan(Lq, Lk, h, cu_count), h, c.seqs).bytes : 0;
+    most = b > most ? b : most;
+  }
+  return most;
+}
+
+}  // namespace sdpa
+}  // namespace sdq

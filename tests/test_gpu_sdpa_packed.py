@@ -118,6 +118,22 @@ def test_chunks(sdq_dev):
         assert float((one.double() - want).abs().max() / want.abs().max()) <= 2e-5
 
 
+def test_ragged_head_chunks(sdq_dev):
+    """Heads that the launches' scratch does not divide: the last launch has
+    fewer, and its own plan."""
+    import torch
+
+    Lq, Lk, heads = 70, 600_000, 5
+    print(f"[sdpa-packed] head chunks Lk={Lk} heads={heads}", flush=True)
+    g = torch.Generator(device=sdq_dev)
+    g.manual_seed(8)
+    q = torch.randn((Lq, 128 * heads), generator=g, device=sdq_dev)
+    kv = torch.randn((Lk, 256 * heads), generator=g, device=sdq_dev)
+    got = _run(sdq_dev, q, kv, heads)
+    want = _want64(q, kv, heads)
+    assert float((got.double() - want).abs().max() / want.abs().max()) <= 2e-5
+
+
 def test_capture_without_warm_up(sdq_dev):
     """A capture on a stream whose workspace cannot grow any more takes the
     form without scratch; replays see new inputs."""
