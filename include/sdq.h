@@ -320,7 +320,7 @@ int sdq_add(float* x, const float* y, int64_t n, void* stream);
  * three split fp16 MFMA products of power-of-two-scaled parts (taken back out
  * exactly), an online softmax: within 2e-5 of the reference's output scale
  * (its serial sums are not reproduced). K and V are packed once into scratch
- * of the stream's workspace (at most ~2 GiB, grown and kept like the others);
+ * of the stream's workspace (at most 2 GiB and 1 MiB, grown and kept like the others);
  * where that cannot be had (a stream capturing a graph before it has grown,
  * no device memory) a slower form without scratch runs, to the same bound.
  * 16-byte aligned rows. Stream-ordered. */

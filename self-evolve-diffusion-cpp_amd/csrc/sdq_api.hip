@@ -1849,8 +1849,8 @@ int sdq_sdpa_batched(const float* q, int64_t ldq, const float* k, int64_t ldk, c
   if ((rc = ensure_device(dev))) return rc;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   const int cu_count = g_dev[dev].cu_count;
-  // The packed form when its scratch can be had (at most 2 GiB, see
-  // sdpa_packed_bytes), else the form without scratch: an attention call is
+  // The packed form when its scratch can be had (at most
+  // sdpa::kMaxScratch bytes), else the form without scratch: an attention call is
   // not refused for want of memory, under graph capture either.
   float* scratch = nullptr;
   const int64_t need = sdpa_packed_bytes(Lq, Lk, heads, batch, cu_count);

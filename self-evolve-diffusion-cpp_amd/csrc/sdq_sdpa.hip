@@ -619,13 +619,13 @@ hipError_t launch_sdpa_packed(const float* q, int64_t ldq, const float* k, int64
   if (Lk <= 0 || heads <= 0 || heads > 65535 || batch > 65535 || !scratch)
     return hipErrorInvalidValue;
   const float scale_log2e = (1.f / sqrtf((float)kHd)) * 1.4426950408889634f;
-  const sdpa::Chunk ch = sdpa::chunk(ceil_div(Lk, kKB), heads, batch);
+  const sdpa::Chunk ch = sdpa::chunk(Lq, Lk, heads, batch, cu_count);
   char* packed = static_cast<char*>(scratch);
   for (int b0 = 0; b0 < batch; b0 += ch.seqs)
     for (int h0 = 0; h0 < heads; h0 += ch.heads) {
       const int nb = batch - b0 < ch.seqs ? batch - b0 : ch.seqs;
       const int nh = heads - h0 < ch.heads ? heads - h0 : ch.heads;
-      const Plan p = sdpa::make_plan(Lq, Lk, nh, cu_count);
+      const Plan p = sdpa::launch_plan(Lq, Lk, nh, cu_count);
       const sdpa::Layout l = sdpa::layout(p, nh, nb);
       if (l.bytes > scratch_bytes) return hipErrorInvalidValue;
       int2* exps = reinterpret_cast<int2*>(packed + l.exps);

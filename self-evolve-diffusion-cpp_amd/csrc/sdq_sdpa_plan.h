@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <cstdlib>
+#include <initializer_list>
 
 namespace sdq {
 namespace sdpa {
@@ -31,9 +32,16 @@ struct Plan {
   int splits;
   int kbs;
 };
-// Depends on the sequence only, not on the batch, so stacked and separate
-// calls give the same bits.
-inline Plan make_plan(int64_t Lq, int64_t Lk, int heads, int cu_count) {
+// Scratch of a launch: at most this, whatever the call (a head's 2^21 keys are
+// 2 GiB of records; their exponents come on top).
+constexpr int64_t kMaxRecs = int64_t(1) << 31;
+constexpr int64_t kMaxScratch = kMaxRecs + (1 << 20);
+constexpr int64_t kShareBytes = kQ * (kHd * 4 + 8);  // a share's partial output
+
+// `most`: bytes that the partial outputs of one sequence may take. Depends on
+// the sequence only, not on the batch, so stacked and separate calls give the
+// same bits.
+inline Plan make_plan(int64_t Lq, int64_t Lk, int heads, int cu_count, int64_t most) {
   Plan p{};
   p.nkb = (int)div_up(Lk, kKB);
   p.qgroups = (int)div_up(Lq, kQ);
@@ -51,10 +59,10 @@ inline Plan make_plan(int64_t Lq, int64_t Lk, int heads, int cu_count) {
   // its own start and end (about 3 blocks), plus the second pass over the
   // partial outputs.
   double best = p.nkb + 3;
-  for (int S = 2; S <= 32 && 3 * S <= p.nkb; S++) {
-    const int kbs = (int)div_up(p.nkb, S);
-    if (div_up(p.nkb, kbs) != S) continue;  // no empty share
-    const double cost = (double)div_up((int64_t)rest * S, cus) * (kbs + 3) + 3;
+  for (int S = 2; S <= 32 && 3 * S <= p.nkb && rest * S * kShareBytes <= most; S++) {
+    const int kbs = (p.nkb + S - 1) / S;
+    if ((p.nkb + kbs - 1) / kbs != S) continue;  // no empty share
+    const double cost = (double)((rest * S + cus - 1) / cus) * (kbs + 3) + 3;
     if (cost < best) best = cost, p.splits = S, p.kbs = kbs;
   }
   return p;
@@ -76,20 +84,35 @@ inline Layout layout(const Plan& p, int64_t heads, int64_t batch) {
   return l;
 }
 
-// A call runs in launches of as many sequences, or of as many heads of one
-// sequence, as keep their records within kMaxRecs bytes, so the scratch a
-// stream holds is bounded (heads: a sequence's own share, so that it does
-// not depend on the batch).
-constexpr int64_t kMaxRecs = int64_t(1) << 31;
+// The plan of a launch over `heads` heads, its partial outputs within what the
+// records leave of kMaxScratch.
+inline Plan launch_plan(int64_t Lq, int64_t Lk, int heads, int cu_count) {
+  const int64_t recs = heads * div_up(Lk, kKB);
+  return make_plan(Lq, Lk, heads, cu_count, kMaxScratch - recs * kRec - pad256(recs * 8));
+}
+
+// A call runs in launches of as many sequences, or of equal numbers of heads
+// of one sequence, as fit kMaxScratch with the plan they would have without
+// that limit (heads: a sequence's own share, so that it does not depend on the
+// batch); a single head takes fewer shares instead.
 struct Chunk {
   int heads, seqs;
 };
-inline Chunk chunk(int64_t nkb, int heads, int batch) {
-  const int64_t per_head = nkb * kRec;
-  const int64_t h = kMaxRecs / per_head < 1 ? 1 : kMaxRecs / per_head;
-  if (h < heads) return {(int)h, 1};
-  const int64_t n = kMaxRecs / (per_head * heads);
-  return {heads, (int)(n < batch ? n : batch)};
+inline Chunk chunk(int64_t Lq, int64_t Lk, int heads, int batch, int cu_count) {
+  auto bytes = [&](int h) {
+    return layout(make_plan(Lq, Lk, h, cu_count, INT64_MAX), h, 1).bytes;
+  };
+  if (const int64_t b = bytes(heads); b <= kMaxScratch) {
+    const int64_t n = kMaxScratch / b;
+    return {heads, (int)(n < batch ? n : batch)};
+  }
+  // (from the fewest launches that the records allow)
+  for (int64_t c = div_up(heads * div_up(Lk, kKB) * kRec, kMaxRecs); c < heads; c++) {
+    const int h = (int)div_up(heads, c);
+    if (bytes(h) <= kMaxScratch && (heads % h == 0 || bytes(heads % h) <= kMaxScratch))
+      return {h, 1};
+  }
+  return {1, 1};
 }
 
 // Bytes that every launch of a call fits in; 0: the packed form does not take
@@ -98,10 +121,10 @@ inline Chunk chunk(int64_t nkb, int heads, int batch) {
 inline int64_t scratch_bytes(int64_t Lq, int64_t Lk, int heads, int batch, int cu_count) {
   // a head's records are addressed with 32-bit offsets; a grid holds 2^32 threads
   if (Lk > kMaxRecs / kRec * kKB || heads > 65535 || div_up(Lq, kQ) * heads > (1 << 22)) return 0;
-  const Chunk c = chunk(div_up(Lk, kKB), heads, batch);
+  const Chunk c = chunk(Lq, Lk, heads, batch, cu_count);
   int64_t most = 0;
   for (const int h : {c.heads, heads % c.heads}) {
-    const int64_t b = h ? layout(make_plan(Lq, Lk, h, cu_count), h, c.seqs).bytes : 0;
+    const int64_t b = h ? layout(launch_plan(Lq, Lk, h, cu_count), h, c.seqs).bytes : 0;
     most = b > most ? b : most;
   }
   return most;

@@ -1,6 +1,7 @@
 // Sweeps the packed attention's host plan (csrc/sdq_sdpa_plan.h): every launch
-// of a call must lie inside the scratch that is asked for the call, and every
-// item's keys must be covered once. Prints the first call that breaks a rule.
+// of a call must lie inside the scratch that is asked for the call, that
+// scratch inside 2 GiB (and its records' exponents), and every item's keys must
+// be covered once. Prints the first call that breaks a rule.
 #include <cmath>
 #include <cstdio>
 #include <random>
@@ -19,13 +20,14 @@ bool check(int64_t Lq, int64_t Lk, int heads, int batch, int cus) {
                 (long long)Lk, heads, batch, cus, what, (long long)a, (long long)b);
     return false;
   };
-  const sd::Chunk c = sd::chunk(sd::div_up(Lk, sd::kKB), heads, batch);
+  const sd::Chunk c = sd::chunk(Lq, Lk, heads, batch, cus);
+  if (have > (int64_t(1) << 31) + (1 << 20)) return bad("more than 2 GiB", have, c.seqs);
   if (c.heads < 1 || c.seqs < 1) return bad("empty chunk", c.heads, c.seqs);
   if (c.heads < heads && c.seqs != 1) return bad("chunk of heads and sequences", c.heads, c.seqs);
   for (int h : {c.heads, heads % c.heads})
     for (int n : {c.seqs, batch % c.seqs}) {
       if (h == 0 || n == 0) continue;
-      const sd::Plan p = sd::make_plan(Lq, Lk, h, cus);
+      const sd::Plan p = sd::launch_plan(Lq, Lk, h, cus);
       const int64_t need = sd::layout(p, h, n).bytes;
       if (need > have) return bad("launch past the scratch (needs, has)", need, have);
       if (p.items != h * p.qgroups || p.nfull < 0 || p.nfull > p.items)
@@ -39,8 +41,11 @@ bool check(int64_t Lq, int64_t Lk, int heads, int batch, int cus) {
 }  // namespace
 
 int main() {
-  // ragged last chunks of heads
-  bool ok = check(151584, 151584, 24, 1, 256) && check(38688, 262244, 12, 1, 256) &&
+  // shares' outputs beyond the records: 2.7, 3.0 and 49 GiB without a bound of
+  // their own; then ragged last chunks of heads
+  bool ok = check(27280, 1 << 20, 1, 1, 256) && check(1024, 1024, 24, 64, 256) &&
+            check(27280, 4099, 1, 512, 256) && check(1, 1 << 21, 1, 1, 256) &&
+            check(9000, 1 << 21, 3, 1, 256) && check(151584, 151584, 24, 1, 256) && check(38688, 262244, 12, 1, 256) &&
             check(278008, 349526, 24, 1, 256) && check(1, 1, 1, 1, 256) &&
             check(40, 1100000, 2, 2, 256);
   std::mt19937_64 g(7);
