@@ -26,6 +26,7 @@ namespace sdq {
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef short v2s __attribute__((ext_vector_type(2)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -40,11 +41,24 @@ constexpr int kPart = 8192;          // one part (hi or lo) of K or V
 constexpr int kWaves = 8;
 static_assert(kQ == 32 * kWaves);
 constexpr int kRing = 4;             // blocks of K and of V in LDS
-// K and Q are scaled by powers of two so that the largest element of a key
-// block (of a query row) lies in [2^14, 2^15): their fp16 low parts then stay
-// normal numbers down to 2^-18 of it.
+// Operands are scaled by powers of two so that the largest element of a key
+// block's K, of its V, and of a query row lies in [2^14, 2^15). hi + lo then
+// hold 22 bits of an element down to 2^-18 of that largest one and an absolute
+// 2^-40 of it below: a key 2^18 smaller than the largest of its 32 loses low
+// bits of its logits, a V element those of its own dimension.
 constexpr int kTop = 15;
+// A V row whose largest element lies 2^kShift or more below its block's is
+// scaled up by 2^(a multiple of kShift), its P down by the same, so that no
+// key's P v is lost beside another's: a block with such rows is uneven. (Of the
+// output's scale, before and with it: weights of 2^-20 on V 2^20 larger 1e-3,
+// 6e-6; V of 2^40 and 2^-90 130%, 4e-6. Ordinary blocks keep their values; 27280
+// tokens 0.9% longer, 157 x 768 34.6 -> 35.4 us.)
+constexpr int kShift = 8;
+// Blocks whose V lies this far below the head's largest are treated like
+// uneven ones (their P may be 0 where their weights are not).
+constexpr int kFar = 60;
 constexpr int kZeroV = 1 << 20;      // "exponent" of a V block of zeros
+constexpr int kMinLogit = -100;      // scales of q.k below 2^this: all logits 0 either way
 // V's exponents stop here (a V block all below 2^-95 then holds smaller
 // numbers) and the sums l are kept as l 2^-16: l ~ 2^(15 - e_v) stays a normal
 // float over all exponents.
@@ -84,14 +98,16 @@ __device__ __forceinline__ float quad16_sum(float v) {
 //     dims 32 d + 8 (lane / 16) + 0..7
 //   V [part][16-dim tile dt][lane]: dim 16 dt + lane % 16, keys
 //     16 (m / 4) + 4 (lane / 16) + m % 4, m = 0..7
-// Keys past Lk are zeros. HBM-bound: 8 bytes read and 8 written per (key,
-// dim) pair of K and V.
+// Keys past Lk are zeros. exps: K's exponent e and 2 e + (uneven) of V (kZeroV:
+// zeros); shifts: the keys' of V, a byte each. HBM-bound: 8 bytes read and 8
+// written per (key, dim) pair of K and V.
 __global__ void __launch_bounds__(256)
 sdpa_pack_kernel(const float* __restrict__ K, int64_t ldk, const float* __restrict__ V,
                  int64_t ldv, int64_t Lk, int nkb, char* __restrict__ packed,
-                 int2* __restrict__ exps) {
+                 int2* __restrict__ exps, uint32_t* __restrict__ shifts) {
   __shared__ __attribute__((aligned(16))) char buf[kRec];
-  __shared__ float red[2][4];
+  __shared__ float red[4];
+  __shared__ __attribute__((aligned(16))) float rows[kKB];  // V rows' largest magnitudes
   const int t = threadIdx.x;
   const int kb = blockIdx.x, head = blockIdx.y;
   const int64_t seq = blockIdx.z;
@@ -101,7 +117,7 @@ sdpa_pack_kernel(const float* __restrict__ K, int64_t ldk, const float* __restri
   // 4 dims (float4 q4 of a row) of 4 keys each: K's keys 8 i + r, V's 4 r + i
   const int q4 = t & 31, r = t >> 5;
   float4 a[4];
-  float v[4][4], mk = 0.f, mv = 0.f;
+  float v[4][4], mk = 0.f, mv[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int64_t kr = (int64_t)kb * kKB + 8 * i + r, vr = (int64_t)kb * kKB + 4 * r + i;
@@ -115,18 +131,38 @@ sdpa_pack_kernel(const float* __restrict__ K, int64_t ldk, const float* __restri
   for (int i = 0; i < 4; i++) {
     mk = amax_finite(amax_finite(mk, a[i].x), a[i].y);
     mk = amax_finite(amax_finite(mk, a[i].z), a[i].w);
+    mv[i] = 0.f;
 #pragma unroll
-    for (int c = 0; c < 4; c++) mv = amax_finite(mv, v[i][c]);
+    for (int c = 0; c < 4; c++) mv[i] = amax_finite(mv[i], v[i][c]);
   }
+  // the four V rows' maxima over 32 lanes: each lane goes on with two, then
+  // with one of them (row 2 (lane & 1) + (lane >> 1 & 1))
+  const bool b0 = t & 1, b1 = t & 2;
+  float m0 = fmaxf(b0 ? mv[2] : mv[0], __shfl_xor(b0 ? mv[0] : mv[2], 1));
+  const float m1 = fmaxf(b0 ? mv[3] : mv[1], __shfl_xor(b0 ? mv[1] : mv[3], 1));
+  m0 = fmaxf(b1 ? m1 : m0, __shfl_xor(b1 ? m0 : m1, 2));
 #pragma unroll
-  for (int d = 1; d < 64; d *= 2)
-    mk = fmaxf(mk, __shfl_xor(mk, d)), mv = fmaxf(mv, __shfl_xor(mv, d));
-  if ((t & 63) == 0) red[0][t >> 6] = mk, red[1][t >> 6] = mv;
+  for (int d = 4; d < 32; d *= 2) m0 = fmaxf(m0, __shfl_xor(m0, d));
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) mk = fmaxf(mk, __shfl_xor(mk, d));
+  if ((t & 63) == 0) red[t >> 6] = mk;
+  if ((t & 31) < 4) rows[4 * r + 2 * (t & 1) + (t >> 1 & 1)] = m0;
   __syncthreads();
-  mk = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
-  mv = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
-  const int ek = top_exp(mk), ev = top_exp(mv) < kMinV ? kMinV : top_exp(mv);
-  if (t == 0) exps[rec] = int2{ek, mv == 0.f ? kZeroV : ev};
+  mk = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  float top = 0.f;
+#pragma unroll
+  for (int i = 0; i < kKB; i++) top = fmaxf(top, rows[i]);
+  auto v_exp = [](float m) { return top_exp(m) < kMinV ? kMinV : top_exp(m); };
+  const int ek = top_exp(mk), ev = v_exp(top);
+  auto row_shift = [&](float m) { return m > 0.f ? (ev - v_exp(m)) & -kShift : 0; };
+  int sh[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) sh[i] = row_shift(rows[4 * r + i]);
+  if (q4 == 0) shifts[rec * (kKB / 4) + r] = sh[0] | sh[1] << 8 | sh[2] << 16 | sh[3] << 24;
+  if (t < 64) {
+    const bool uneven = __ballot(row_shift(rows[t & 31]) > 0) != 0;
+    if (t == 0) exps[rec] = int2{ek, top == 0.f ? kZeroV : 2 * ev + (uneven ? 1 : 0)};
+  }
   auto put = [&](char* p, const float y0, const float y1, const float y2, const float y3) {
     const v4h hi = {(_Float16)y0, (_Float16)y1, (_Float16)y2, (_Float16)y3};
     const v4h lo = {(_Float16)(y0 - (float)hi.x), (_Float16)(y1 - (float)hi.y),
@@ -149,8 +185,9 @@ sdpa_pack_kernel(const float* __restrict__ K, int64_t ldk, const float* __restri
 #pragma unroll
   for (int c = 0; c < 4; c++) {
     const int d = 4 * q4 + c;
-    put(buf + kRecV + swz(d >> 4, (r & 3) * 16 + (d & 15)) + (r >> 2) * 8, ldexpf(v[0][c], -ev),
-        ldexpf(v[1][c], -ev), ldexpf(v[2][c], -ev), ldexpf(v[3][c], -ev));
+    put(buf + kRecV + swz(d >> 4, (r & 3) * 16 + (d & 15)) + (r >> 2) * 8,
+        ldexpf(v[0][c], sh[0] - ev), ldexpf(v[1][c], sh[1] - ev), ldexpf(v[2][c], sh[2] - ev),
+        ldexpf(v[3][c], sh[3] - ev));
   }
   __syncthreads();
   char* dst = packed + rec * kRec;
@@ -184,6 +221,13 @@ struct Inv {
   __device__ __forceinline__ float operator()(float o) const { return ldexpf(o * r, e); }
 };
 
+// l 2^d: for d below -100 in two steps, since the exponential's 2^d becomes 0
+// below the normal numbers, which l 2^d need not be
+__device__ __forceinline__ float scale_l(float l, float d) {
+  const float half = __builtin_amdgcn_exp2f(0.5f * d);
+  return d < -100.f ? l * half * half : l * __builtin_amdgcn_exp2f(d);
+}
+
 // Keeps a value's computation where it is written (the compiler would sink it
 // past the barrier to its use).
 template <class T>
@@ -205,8 +249,9 @@ __device__ __forceinline__ void split_pair(float a, float b, float neg1, uint32_
 
 __global__ void __launch_bounds__(kWaves * 64)
 sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restrict__ packed,
-                   const int2* __restrict__ exps, float* __restrict__ O, int64_t ldo, int64_t Lq,
-                   int64_t Lk, Plan plan, float scale_log2e, Parts parts) {
+                   const int2* __restrict__ exps, const uint32_t* __restrict__ shifts,
+                   float* __restrict__ O, int64_t ldo, int64_t Lq, int64_t Lk, Plan plan,
+                   float scale_log2e, Parts parts) {
   constexpr int QT = 2;            // 16-query tiles per wave
   constexpr int LD = 16 / kWaves;  // a wave's DMAs of one K or V block
   __shared__ __attribute__((aligned(16))) char lds[kRing * kRec];
@@ -247,7 +292,7 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
   const int64_t rec0 = (seq * (plan.items / plan.qgroups) + head) * nkb;
   const int2* ex = exps + rec0;
 
-  // This wave's DMAs: LD of the 16 KB-chunks of K(i) or V(i) (block kb0 + i)
+  // This wave's DMAs: LD of the 16 1 KB-chunks of K(i) or V(i) (block kb0 + i)
   // into ring slot i % kRing; blocks past the range repeat the last one
   // (never used).
   const dev::v4u rs = dev::raw_rsrc(packed + rec0 * kRec, (uint32_t)nkb * (uint32_t)kRec);
@@ -271,7 +316,7 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
   // and the first DMAs; the other DMAs follow the queries' conversion, whose
   // wait would cover them too.
   int2 ev = ex[kb0 + lane < nkb ? kb0 + lane : nkb - 1];
-  int vmin = ex[lane < nkb ? lane : nkb - 1].y;
+  const int ev0 = ex[lane < nkb ? lane : nkb - 1].y;
   // The query rows, lane (j, h): dims 32 d + 8 h + 0..7 of query 16 t + j,
   // scaled by 2^-eq and split into fp16 parts
   v8h qh[QT][4], ql[QT][4];
@@ -309,17 +354,41 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
     }
   }
   issue_v(1), issue_k(2), issue_v(2), issue_k(3);
-  // a V block of zeros takes the smallest exponent of the others
-  for (int k = lane + 64; k < nkb; k += 64) vmin = min(vmin, ex[k].y);
+  // the largest and smallest V exponents of the head's blocks (16 bits each,
+  // the smallest negated); a block of zeros takes the smallest
+  auto range = [](int y) {
+    return y == kZeroV ? v2s{-1000, -1000} : v2s{(short)(y >> 1), (short)-(y >> 1)};
+  };
+  v2s vr = range(ev0);
+  for (int k = lane + 64; k < nkb; k += 64) vr = __builtin_elementwise_max(vr, range(ex[k].y));
 #pragma unroll
-  for (int d = 1; d < 64; d *= 2) vmin = min(vmin, __shfl_xor(vmin, d));
-  vmin = vmin == kZeroV ? 0 : vmin;
-  if (ev.y == kZeroV) ev.y = vmin;
+  for (int d = 1; d < 64; d *= 2)
+    vr = __builtin_elementwise_max(
+        vr, __builtin_bit_cast(v2s, __shfl_xor(__builtin_bit_cast(int, vr), d)));
+  const int vmin = vr.x == -1000 ? 0 : -vr.y, vfar = vr.x - kFar;
+  const int n = kb1 - kb0;
+  // the partial block, if this range ends with it (else never reached)
+  const int rem = (int)(Lk % kKB);
+  const int last = rem && kb1 == nkb ? n - 1 : -1;
+  // 64 blocks' exponents, which of them are uneven or far below, and at which
+  // the loop's common path ends: those, the partial block, and the next 64's
+  // first
+  uint64_t odd, stops;
+  auto decode_ev = [&](int i) {
+    const bool zero = ev.y == kZeroV, uneven = !zero && (ev.y & 1);
+    ev.y = zero ? vmin : ev.y >> 1;
+    odd = __ballot(uneven || ev.y < vfar);
+    stops = odd | 1 | (last >= i && last < i + 64 ? (uint64_t)1 << (last & 63) : 0);
+  };
   auto load_ev = [&](int i) {
     const int k = kb0 + i + lane;
     ev = ex[k < nkb ? k : nkb - 1];
-    if (ev.y == kZeroV) ev.y = vmin;
+    decode_ev(i);
   };
+  decode_ev(0);
+  auto is_odd = [&](int i) { return (odd >> (i & 63) & 1) != 0; };
+  // keys 16 kt + 4 h .. + 3 of block i, a byte each
+  auto key_shifts = [&](int i, int kt) { return shifts[(rec0 + kb0 + i) * (kKB / 4) + 4 * kt + h]; };
   auto kfrag = [&](int i, int c) {
     const char* p = ldsp + (i & (kRing - 1)) * kRecV + c * 1024;
     return Frag{*reinterpret_cast<const uint4*>(p), *reinterpret_cast<const uint4*>(p + kPart)};
@@ -338,18 +407,16 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
 #pragma unroll
     for (int t = 0; t < QT; t++) acc[d][t] = v4f{};
   // R: the reference exponent of a query; P = 2^(s + e_v - R) with the base-2
-  // logit s and V's block exponent e_v, so that P V~ (V~ = V 2^-e_v) sums to
-  // 2^-R sum 2^s V, and l = 2^-R sum 2^s. R follows max(s + e_v), kept in
+  // logit s and V's exponent e_v (its block's, less the key's shift), so that
+  // P V~ (V~ = V 2^-e_v) sums to 2^-R sum 2^s V. R follows max(s + e_v), kept in
   // [R + 7, R + 15]: P is then at most 2^15, its fp16 parts keep 22 bits down
-  // to 2^-10 of the largest P V~ so far (and an absolute 2^-32 of it below),
-  // and the accumulators are rarely rescaled.
+  // to 2^-10 of the largest so far (and an absolute 2^-32 of it below), and the
+  // accumulators are rarely rescaled. l = 2^(-R - kSumExp) sum 2^s: the sum of a
+  // block's P with its e_v taken out, but from the logits again where keys of
+  // a block differ in e_v or P may have become 0 beside V larger elsewhere.
   float R[QT], lsum[QT], sq[QT], off[QT];
 #pragma unroll
   for (int t = 0; t < QT; t++) R[t] = -INFINITY, lsum[t] = 0.f;
-  const int n = kb1 - kb0;
-  // the partial block, if this range ends with it (else never reached)
-  const int rem = (int)(Lk % kKB);
-  const int last = rem && kb1 == nkb ? n - 1 : -1;
   auto mask = [&](Scores& sc) {
 #pragma unroll
     for (int kt = 0; kt < 2; kt++)
@@ -369,11 +436,45 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
       const bool u = mb[t] > R[t] + 15.f;
       const float rn = u ? mb[t] - 7.f : R[t];
       const float alpha = u ? __builtin_amdgcn_exp2f(R[t] - rn) : 1.f;
+      lsum[t] = u ? scale_l(lsum[t], R[t] - rn) : lsum[t];
       R[t] = rn;
       off[t] = e - rn;
-      lsum[t] *= alpha;
 #pragma unroll
       for (int d = 0; d < 8; d++) acc[d][t] *= alpha;
+    }
+  };
+
+  // the scale of q.k in base 2
+  auto logit_scale = [&](int t, int kx) {
+    return ldexpf(scale_log2e, max(eq[t] + kx, kMinLogit));
+  };
+  // An odd block's scores, down by its keys' shifts
+  auto shift_keys = [&](Scores& sc, int i) {
+    const int kx = __builtin_amdgcn_readlane(ev.x, i & 63);
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      const uint32_t u = key_shifts(i, kt);
+#pragma unroll
+      for (int t = 0; t < QT; t++) {
+        const float up = -1.f / logit_scale(t, kx);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          sc.s[kt][t][r] = fmaf((float)(u >> 8 * r & 255), up, sc.s[kt][t][r]);
+      }
+    }
+  };
+  // An odd block's part of l, from its shifted scores (whose sq and off are set)
+  auto add_l = [&](const Scores& sc, int i) {
+    const int e_v = __builtin_amdgcn_readlane(ev.y, i & 63);
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      const uint32_t u = key_shifts(i, kt);
+#pragma unroll
+      for (int t = 0; t < QT; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          lsum[t] += __builtin_amdgcn_exp2f(fmaf(sc.s[kt][t][r], sq[t], off[t]) +
+                                            (float)((int)(u >> 8 * r & 255) - e_v - kSumExp));
     }
   };
 
@@ -394,15 +495,17 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
     for (int t = 0; t < QT; t++) st.s[kt][t] = mfma_h(f.lo, qh[t][d], st.s[kt][t]);
   }
   if (last == 0) mask(st);
+  if (is_odd(0)) shift_keys(st, 0);
   {
     float mb[QT];
 #pragma unroll
     for (int t = 0; t < QT; t++) {
-      sq[t] = ldexpf(scale_log2e, eq[t] + __builtin_amdgcn_readlane(ev.x, 0));
+      sq[t] = logit_scale(t, __builtin_amdgcn_readlane(ev.x, 0));
       mb[t] = fmaf(quad16_max(max4(max4(-INFINITY, st.s[0][t]), st.s[1][t])), sq[t],
                    (float)__builtin_amdgcn_readlane(ev.y, 0));
     }
     raise(mb, (float)__builtin_amdgcn_readlane(ev.y, 0));
+    if (is_odd(0)) add_l(st, 0);
   }
   __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(4 * LD) & ~(15 << 8));
   asm volatile("s_barrier" ::: "memory");
@@ -423,6 +526,9 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
 #pragma unroll
     for (int t = 0; t < QT; t++) ps[t] = 0.f;
     const int e_v = __builtin_amdgcn_readlane(ev.y, i & 63);
+    const int i1 = i + 1;
+    const bool special = stops >> (i1 & 63) & 1;
+    const int e_l = is_odd(i) ? -1000 : -kSumExp - e_v;  // odd: add_l has been there
     // pair u of step c: elements 2 e, 2 e + 1 (of 8) of query tile t
     auto elem = [&](int c, int u, int k, int& t, int& e) {
       const int pi = c * (QT / 2) + u;
@@ -469,9 +575,11 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
     // everyone's have, and K(i+1), V(i-1) have been read by all
     __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(3 * LD));
     asm volatile("s_barrier" ::: "memory");
-    if (i + 1 == last) mask(nx);
-    const int i1 = i + 1;
-    if ((i1 & 63) == 0) load_ev(i1);
+    if (special) {
+      if ((i1 & 63) == 0) load_ev(i1);
+      if (i1 == last) mask(nx);
+      if (i1 < n && is_odd(i1)) shift_keys(nx, i1);
+    }
     const uint32_t sv = soff(i + 3) + kRecV, sk = soff(i + 5);
     const uint32_t dv = slot_v(i + 3), dk = slot_k(i + 5);
     float ml[QT], vx = 0.f;
@@ -505,7 +613,7 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
       if (c == 1) {
 #pragma unroll
         for (int t = 0; t < QT; t++) {
-          lsum[t] += ldexpf(ps[t], -kSumExp - e_v);
+          lsum[t] += ldexpf(ps[t], e_l);
           pin(lsum[t]);
         }
       }
@@ -514,7 +622,7 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
         vx = (float)__builtin_amdgcn_readlane(ev.y, i1 & 63);
 #pragma unroll
         for (int t = 0; t < QT; t++) {
-          sq[t] = ldexpf(scale_log2e, eq[t] + kx);
+          sq[t] = logit_scale(t, kx);
           pin(sq[t]);
         }
       }
@@ -538,7 +646,10 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (i1 < n && __any(up)) raise(ml, vx);  // (past the end: a repeated block)
+    if (i1 < n && (__ballot(up) | (odd >> (i1 & 63) & 1))) {  // (past the end: a repeated block)
+      raise(ml, vx);
+      if (is_odd(i1)) add_l(nx, i1);
+    }
   };
   for (int i = 0;;) {
     step(i, st, st2);
@@ -586,8 +697,8 @@ sdpa_combine_kernel(Plan plan, Parts parts, int64_t Lq, float* __restrict__ O, i
   const int64_t row = (seq * (plan.items - plan.nfull) + it) * S * kQ + q;
   const float2* ml = parts.ml + row;
   const float* op = parts.o + row * kHd + d;
-  float mx = -INFINITY;
-  for (int s = 0; s < S; s++) mx = fmaxf(mx, ml[s * kQ].x);
+  float mx = -INFINITY, mn = INFINITY;
+  for (int s = 0; s < S; s++) mx = fmaxf(mx, ml[s * kQ].x), mn = fminf(mn, ml[s * kQ].x);
   float lt = 0.f;
   float4 o = {0.f, 0.f, 0.f, 0.f};
   for (int s = 0; s < S; s++) {
@@ -599,6 +710,10 @@ sdpa_combine_kernel(Plan plan, Parts parts, int64_t Lq, float* __restrict__ O, i
     o.y += wt * v.y;
     o.z += wt * v.z;
     o.w += wt * v.w;
+  }
+  if (mx - mn > 100.f) {
+    lt = 0.f;
+    for (int s = 0; s < S; s++) lt += scale_l(ml[s * kQ].y, ml[s * kQ].x - mx);
   }
   const Inv inv(lt);
   *reinterpret_cast<float4*>(O + (seq * Lq + qi) * ldo + (int64_t)head * kHd + d) =
@@ -629,6 +744,7 @@ hipError_t launch_sdpa_packed(const float* q, int64_t ldq, const float* k, int64
       const sdpa::Layout l = sdpa::layout(p, nh, nb);
       if (l.bytes > scratch_bytes) return hipErrorInvalidValue;
       int2* exps = reinterpret_cast<int2*>(packed + l.exps);
+      uint32_t* shifts = reinterpret_cast<uint32_t*>(packed + l.shifts);
       const Parts parts{reinterpret_cast<float*>(packed + l.o),
                         reinterpret_cast<float2*>(packed + l.ml)};
       const int64_t col = (int64_t)h0 * kHd;
@@ -636,11 +752,11 @@ hipError_t launch_sdpa_packed(const float* q, int64_t ldq, const float* k, int64
       float* ob = out + b0 * Lq * ldo + col;
       hipLaunchKernelGGL(sdpa_pack_kernel, dim3((unsigned)p.nkb, (unsigned)nh, (unsigned)nb),
                          dim3(256), 0, s, k + b0 * Lk * ldk + col, ldk, v + b0 * Lk * ldv + col,
-                         ldv, Lk, p.nkb, packed, exps);
+                         ldv, Lk, p.nkb, packed, exps, shifts);
       const int64_t shares = (int64_t)(p.items - p.nfull) * p.splits;
       hipLaunchKernelGGL(sdpa_packed_kernel, dim3((unsigned)(p.nfull + shares), (unsigned)nb),
-                         dim3(kWaves * 64), 0, s, qb, ldq, packed, exps, ob, ldo, Lq, Lk, p,
-                         scale_log2e, parts);
+                         dim3(kWaves * 64), 0, s, qb, ldq, packed, exps, shifts, ob, ldo, Lq, Lk,
+                         p, scale_log2e, parts);
       if (p.splits > 1)
         hipLaunchKernelGGL(sdpa_combine_kernel,
                            dim3((unsigned)(p.items - p.nfull), kQ / 8, (unsigned)nb), dim3(256),

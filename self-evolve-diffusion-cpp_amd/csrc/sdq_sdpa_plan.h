@@ -33,9 +33,9 @@ struct Plan {
   int kbs;
 };
 // Scratch of a launch: at most this, whatever the call (a head's 2^21 keys are
-// 2 GiB of records; their exponents come on top).
+// 2 GiB of records; their exponents and shifts come on top).
 constexpr int64_t kMaxRecs = int64_t(1) << 31;
-constexpr int64_t kMaxScratch = kMaxRecs + (1 << 20);
+constexpr int64_t kMaxScratch = kMaxRecs + (3 << 20);
 constexpr int64_t kShareBytes = kQ * (kHd * 4 + 8);  // a share's partial output
 
 // `most`: bytes that the partial outputs of one sequence may take. Depends on
@@ -70,7 +70,9 @@ inline Plan make_plan(int64_t Lq, int64_t Lk, int heads, int cu_count, int64_t m
 
 // Scratch of one launch over `heads` heads of `batch` sequences.
 struct Layout {
-  int64_t exps, o, ml, bytes;  // offsets of its parts (the records lie at 0)
+  // offsets of its parts (the records lie at 0): the records' exponents, their
+  // keys' shifts, the shares' outputs and sums
+  int64_t exps, shifts, o, ml, bytes;
 };
 inline Layout layout(const Plan& p, int64_t heads, int64_t batch) {
   const int64_t recs = batch * heads * p.nkb;
@@ -78,7 +80,8 @@ inline Layout layout(const Plan& p, int64_t heads, int64_t batch) {
       p.splits > 1 ? batch * (p.items - p.nfull) * p.splits * (int64_t)kQ : 0;
   Layout l;
   l.exps = recs * kRec;
-  l.o = l.exps + pad256(recs * 8);
+  l.shifts = l.exps + pad256(recs * 8);
+  l.o = l.shifts + pad256(recs * kKB);
   l.ml = l.o + rows * kHd * 4;
   l.bytes = l.ml + rows * 8;
   return l;
@@ -87,8 +90,10 @@ inline Layout layout(const Plan& p, int64_t heads, int64_t batch) {
 // The plan of a launch over `heads` heads, its partial outputs within what the
 // records leave of kMaxScratch.
 inline Plan launch_plan(int64_t Lq, int64_t Lk, int heads, int cu_count) {
-  const int64_t recs = heads * div_up(Lk, kKB);
-  return make_plan(Lq, Lk, heads, cu_count, kMaxScratch - recs * kRec - pad256(recs * 8));
+  Plan p{};
+  p.nkb = (int)div_up(Lk, kKB);
+  p.splits = 1;
+  return make_plan(Lq, Lk, heads, cu_count, kMaxScratch - layout(p, heads, 1).bytes);
 }
 
 // A call runs in launches of as many sequences, or of equal numbers of heads

@@ -1,8 +1,8 @@
 """sdq_sdpa's packed form at the edges of its key blocks (32), query groups
 (256) and key shares, over V's element range, in chunks, and the form without
 scratch under graph capture. Bound: 2e-5 of the output scale (the parity bound
-of the attention against the oracle), or per output dimension where V's
-magnitudes differ."""
+of the attention against the oracle), of each output dimension's own scale
+where V's magnitudes differ from dimension to dimension or key to key."""
 import numpy as np
 import pytest
 
@@ -96,6 +96,54 @@ def test_value_range(sdq_dev, case):
     err = float((got - want).abs().max() / scale)
     print(f"  max err {err:.3e}", flush=True)
     assert err <= bound
+
+
+@pytest.mark.parametrize("Lk", [300, 1024, 5000])
+@pytest.mark.parametrize("cut", [True, False])
+@pytest.mark.parametrize("case", ["falling", "rising", "far_rows", "light_keys", "ignored",
+                                  "outlier_dim", "outlier_element"])
+def test_value_magnitudes(sdq_dev, monkeypatch, case, cut, Lk):
+    """V of 2^40 and 2^-90, by halves with blocks of zeros in either order and
+    row by row (the small keys count in the softmax's sum all the same); keys
+    of 2^-20 of the weight whose V is 2^20 times larger; keys of no weight whose
+    V is 2^100; a dimension 2^16 and an element 2^12 above the others. Every
+    output dimension to its own scale, with the keys cut into shares and not."""
+    import torch
+
+    print(f"[sdpa-packed] magnitudes {case} Lk={Lk} cut={cut}", flush=True)
+    if not cut:
+        monkeypatch.setenv("SDQ_SDPA_SPLIT", "1")
+    g = torch.Generator(device=sdq_dev)
+    g.manual_seed(9)
+    Lq, heads = 70, 2
+    C = heads * 128
+    q = torch.randn((Lq, C), generator=g, device=sdq_dev)
+    kv = torch.randn((Lk, 2 * C), generator=g, device=sdq_dev)
+    v = kv[:, C:]
+    if case in ("falling", "rising"):
+        first, second = (40, -90) if case == "falling" else (-90, 40)
+        v[:Lk // 2] *= 2.0 ** first
+        v[Lk // 2:] *= 2.0 ** second
+        v[32:96] = 0.0
+    elif case == "far_rows":
+        v[0::2] *= 2.0 ** 40
+        v[1::2] *= 2.0 ** -90
+    elif case in ("light_keys", "ignored"):
+        e = -20 if case == "light_keys" else -2000
+        q[:, ::128] = 8.0
+        kv[:, 0:C:128] = 0.0
+        kv[1::3, 0:C:128] = e * np.log(2.0) * 128 ** 0.5 / 8
+        v[1::3] *= 2.0 ** (20 if case == "light_keys" else 100)
+    elif case == "outlier_dim":
+        v[:, 7] *= 2.0 ** 16
+    else:
+        v[17, 5] *= 2.0 ** 12
+    want = _want64(q, kv, heads)
+    got = _run(sdq_dev, q, kv, heads).double()
+    assert torch.isfinite(got).all()
+    err = ((got - want).abs().amax(0) / want.abs().amax(0)).max()
+    print(f"  max err of a dimension {float(err):.3e}", flush=True)
+    assert err <= 2e-5
 
 
 def test_chunks(sdq_dev):
