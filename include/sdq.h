@@ -319,10 +319,11 @@ int sdq_add(float* x, const float* y, int64_t n, void* stream);
  * h*head_dim .. h*head_dim+head_dim-1; head_dim = 128. Every fp32 product as
  * three split fp16 MFMA products of power-of-two-scaled parts (taken back out
  * exactly), an online softmax: within 2e-5 of the reference's output scale
- * (its serial sums are not reproduced), whatever V's magnitudes. An output
+ * (its serial sums are not reproduced), whatever the magnitudes of keys and
+ * values. An output
  * dimension far below its head's largest loses low bits: it is within 2e-5 of
  * its own scale at 2^-12 of the largest, within 4e-4 at 2^-20. K and V are
- * packed once into scratch of the stream's workspace (at most 2 GiB and 3 MiB,
+ * packed once into scratch of the stream's workspace (at most 2 GiB and 5 MiB,
  * grown and kept like the others); where that cannot be had (a stream capturing
  * a graph before it has grown, no device memory) a slower form without scratch
  * runs, to the same bound.

@@ -44,15 +44,15 @@ constexpr int kRing = 4;             // blocks of K and of V in LDS
 // Operands are scaled by powers of two so that the largest element of a key
 // block's K, of its V, and of a query row lies in [2^14, 2^15). hi + lo then
 // hold 22 bits of an element down to 2^-18 of that largest one and an absolute
-// 2^-40 of it below: a key 2^18 smaller than the largest of its 32 loses low
-// bits of its logits, a V element those of its own dimension.
+// 2^-40 of it below.
 constexpr int kTop = 15;
-// A V row whose largest element lies 2^kShift or more below its block's is
-// scaled up by 2^(a multiple of kShift), its P down by the same, so that no
-// key's P v is lost beside another's: a block with such rows is uneven. (Of the
-// output's scale, before and with it: weights of 2^-20 on V 2^20 larger 1e-3,
-// 6e-6; V of 2^40 and 2^-90 130%, 4e-6. Ordinary blocks keep their values; 27280
-// tokens 0.9% longer, 157 x 768 34.6 -> 35.4 us.)
+// A row of K or V whose largest element lies 2^kShift or more below its block's
+// is scaled up by 2^(a multiple of kShift), its scores or P down by the same, so
+// that no key's logits or P v are lost beside another's: a block with such rows
+// is uneven. (Errors of the output's scale without and with it: weights of 2^-20
+// on V 2^20 larger 1e-3, 6e-6; V of 2^40 and 2^-90 130%, 4e-6; all the weight on
+// keys 2^30 shorter than their neighbours 8e-3, 4e-6. Ordinary blocks keep their
+// values; 27280 tokens 1% longer, 157 x 768 34.6 -> 35.7 us.)
 constexpr int kShift = 8;
 // Blocks whose V lies this far below the head's largest are treated like
 // uneven ones (their P may be 0 where their weights are not).
@@ -98,16 +98,16 @@ __device__ __forceinline__ float quad16_sum(float v) {
 //     dims 32 d + 8 (lane / 16) + 0..7
 //   V [part][16-dim tile dt][lane]: dim 16 dt + lane % 16, keys
 //     16 (m / 4) + 4 (lane / 16) + m % 4, m = 0..7
-// Keys past Lk are zeros. exps: K's exponent e and 2 e + (uneven) of V (kZeroV:
-// zeros); shifts: the keys' of V, a byte each. HBM-bound: 8 bytes read and 8
+// Keys past Lk are zeros. exps: K's exponent and 2 e + (uneven) with V's e
+// (kZeroV in the place of 2 e: zeros); shifts: V's keys', then K's, in units of
+// kShift, a byte each. HBM-bound: 8 bytes read and 8
 // written per (key, dim) pair of K and V.
 __global__ void __launch_bounds__(256)
 sdpa_pack_kernel(const float* __restrict__ K, int64_t ldk, const float* __restrict__ V,
                  int64_t ldv, int64_t Lk, int nkb, char* __restrict__ packed,
-                 int2* __restrict__ exps, uint32_t* __restrict__ shifts) {
+                 int2* __restrict__ exps, uint8_t* __restrict__ shifts) {
   __shared__ __attribute__((aligned(16))) char buf[kRec];
-  __shared__ float red[4];
-  __shared__ __attribute__((aligned(16))) float rows[kKB];  // V rows' largest magnitudes
+  __shared__ __attribute__((aligned(16))) float rows[2][kKB];  // V's, K's largest magnitudes
   const int t = threadIdx.x;
   const int kb = blockIdx.x, head = blockIdx.y;
   const int64_t seq = blockIdx.z;
@@ -117,7 +117,7 @@ sdpa_pack_kernel(const float* __restrict__ K, int64_t ldk, const float* __restri
   // 4 dims (float4 q4 of a row) of 4 keys each: K's keys 8 i + r, V's 4 r + i
   const int q4 = t & 31, r = t >> 5;
   float4 a[4];
-  float v[4][4], mk = 0.f, mv[4];
+  float v[4][4], mk[4], mv[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     const int64_t kr = (int64_t)kb * kKB + 8 * i + r, vr = (int64_t)kb * kKB + 4 * r + i;
@@ -129,39 +129,44 @@ sdpa_pack_kernel(const float* __restrict__ K, int64_t ldk, const float* __restri
   }
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    mk = amax_finite(amax_finite(mk, a[i].x), a[i].y);
-    mk = amax_finite(amax_finite(mk, a[i].z), a[i].w);
+    mk[i] = amax_finite(amax_finite(0.f, a[i].x), a[i].y);
+    mk[i] = amax_finite(amax_finite(mk[i], a[i].z), a[i].w);
     mv[i] = 0.f;
 #pragma unroll
     for (int c = 0; c < 4; c++) mv[i] = amax_finite(mv[i], v[i][c]);
   }
-  // the four V rows' maxima over 32 lanes: each lane goes on with two, then
-  // with one of them (row 2 (lane & 1) + (lane >> 1 & 1))
+  // four rows' maxima over 32 lanes: each lane goes on with two, then with one
+  // of them, row mine
   const bool b0 = t & 1, b1 = t & 2;
-  float m0 = fmaxf(b0 ? mv[2] : mv[0], __shfl_xor(b0 ? mv[0] : mv[2], 1));
-  const float m1 = fmaxf(b0 ? mv[3] : mv[1], __shfl_xor(b0 ? mv[1] : mv[3], 1));
-  m0 = fmaxf(b1 ? m1 : m0, __shfl_xor(b1 ? m0 : m1, 2));
+  const int mine = 2 * (t & 1) + (t >> 1 & 1);
+  auto row_max = [&](const float (&m)[4]) {
+    float m0 = fmaxf(b0 ? m[2] : m[0], __shfl_xor(b0 ? m[0] : m[2], 1));
+    const float m1 = fmaxf(b0 ? m[3] : m[1], __shfl_xor(b0 ? m[1] : m[3], 1));
+    m0 = fmaxf(b1 ? m1 : m0, __shfl_xor(b1 ? m0 : m1, 2));
 #pragma unroll
-  for (int d = 4; d < 32; d *= 2) m0 = fmaxf(m0, __shfl_xor(m0, d));
-#pragma unroll
-  for (int d = 1; d < 64; d *= 2) mk = fmaxf(mk, __shfl_xor(mk, d));
-  if ((t & 63) == 0) red[t >> 6] = mk;
-  if ((t & 31) < 4) rows[4 * r + 2 * (t & 1) + (t >> 1 & 1)] = m0;
+    for (int d = 4; d < 32; d *= 2) m0 = fmaxf(m0, __shfl_xor(m0, d));
+    return m0;
+  };
+  const float rv = row_max(mv), rk = row_max(mk);
+  if (q4 < 4) rows[0][4 * r + mine] = rv, rows[1][8 * mine + r] = rk;
   __syncthreads();
-  mk = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  float top = 0.f;
+  float top = 0.f, topk = 0.f;
 #pragma unroll
-  for (int i = 0; i < kKB; i++) top = fmaxf(top, rows[i]);
+  for (int i = 0; i < kKB; i++) top = fmaxf(top, rows[0][i]), topk = fmaxf(topk, rows[1][i]);
   auto v_exp = [](float m) { return top_exp(m) < kMinV ? kMinV : top_exp(m); };
-  const int ek = top_exp(mk), ev = v_exp(top);
-  auto row_shift = [&](float m) { return m > 0.f ? (ev - v_exp(m)) & -kShift : 0; };
-  int sh[4];
+  const int ek = top_exp(topk), ev = v_exp(top);
+  auto v_shift = [&](float m) { return m > 0.f ? (ev - v_exp(m)) & -kShift : 0; };
+  auto k_shift = [&](float m) { return m > 0.f ? (ek - top_exp(m)) & -kShift : 0; };
+  int sh[4], shk[4];
 #pragma unroll
-  for (int i = 0; i < 4; i++) sh[i] = row_shift(rows[4 * r + i]);
-  if (q4 == 0) shifts[rec * (kKB / 4) + r] = sh[0] | sh[1] << 8 | sh[2] << 16 | sh[3] << 24;
+  for (int i = 0; i < 4; i++)
+    sh[i] = v_shift(rows[0][4 * r + i]), shk[i] = k_shift(rows[1][8 * i + r]);
   if (t < 64) {
-    const bool uneven = __ballot(row_shift(rows[t & 31]) > 0) != 0;
-    if (t == 0) exps[rec] = int2{ek, top == 0.f ? kZeroV : 2 * ev + (uneven ? 1 : 0)};
+    const float m = rows[t >> 5][t & 31];
+    const int sm = t < 32 ? v_shift(m) : k_shift(m);
+    shifts[rec * 2 * kKB + t] = (uint8_t)(sm / kShift);
+    const int uneven = __ballot(sm > 0) != 0;
+    if (t == 0) exps[rec] = int2{ek, (top == 0.f ? kZeroV : 2 * ev) + uneven};
   }
   auto put = [&](char* p, const float y0, const float y1, const float y2, const float y3) {
     const v4h hi = {(_Float16)y0, (_Float16)y1, (_Float16)y2, (_Float16)y3};
@@ -180,7 +185,8 @@ sdpa_pack_kernel(const float* __restrict__ K, int64_t ldk, const float* __restri
   for (int i = 0; i < 4; i++) {
     const int key = 8 * i + r;
     put(buf + swz((q4 >> 3) * 2 + (key >> 4), (q4 >> 1 & 3) * 16 + (key & 15)) + (q4 & 1) * 8,
-        ldexpf(a[i].x, -ek), ldexpf(a[i].y, -ek), ldexpf(a[i].z, -ek), ldexpf(a[i].w, -ek));
+        ldexpf(a[i].x, shk[i] - ek), ldexpf(a[i].y, shk[i] - ek), ldexpf(a[i].z, shk[i] - ek),
+        ldexpf(a[i].w, shk[i] - ek));
   }
 #pragma unroll
   for (int c = 0; c < 4; c++) {
@@ -357,7 +363,7 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
   // the largest and smallest V exponents of the head's blocks (16 bits each,
   // the smallest negated); a block of zeros takes the smallest
   auto range = [](int y) {
-    return y == kZeroV ? v2s{-1000, -1000} : v2s{(short)(y >> 1), (short)-(y >> 1)};
+    return y >= kZeroV ? v2s{-1000, -1000} : v2s{(short)(y >> 1), (short)-(y >> 1)};
   };
   v2s vr = range(ev0);
   for (int k = lane + 64; k < nkb; k += 64) vr = __builtin_elementwise_max(vr, range(ex[k].y));
@@ -375,7 +381,7 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
   // first
   uint64_t odd, stops;
   auto decode_ev = [&](int i) {
-    const bool zero = ev.y == kZeroV, uneven = !zero && (ev.y & 1);
+    const bool zero = ev.y >= kZeroV, uneven = ev.y & 1;
     ev.y = zero ? vmin : ev.y >> 1;
     odd = __ballot(uneven || ev.y < vfar);
     stops = odd | 1 | (last >= i && last < i + 64 ? (uint64_t)1 << (last & 63) : 0);
@@ -387,8 +393,11 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
   };
   decode_ev(0);
   auto is_odd = [&](int i) { return (odd >> (i & 63) & 1) != 0; };
-  // keys 16 kt + 4 h .. + 3 of block i, a byte each
-  auto key_shifts = [&](int i, int kt) { return shifts[(rec0 + kb0 + i) * (kKB / 4) + 4 * kt + h]; };
+  // the V (v = 0) or K shifts of keys 16 kt + 4 h .. + 3 of block i, a byte each
+  auto key_shifts = [&](int i, int v, int kt) {
+    return shifts[(rec0 + kb0 + i) * (2 * kKB / 4) + 8 * v + 4 * kt + h];
+  };
+  auto shift_of = [](uint32_t u, int r) { return (int)(u >> 8 * r & 255) * kShift; };
   auto kfrag = [&](int i, int c) {
     const char* p = ldsp + (i & (kRing - 1)) * kRecV + c * 1024;
     return Frag{*reinterpret_cast<const uint4*>(p), *reinterpret_cast<const uint4*>(p + kPart)};
@@ -453,13 +462,14 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
     const int kx = __builtin_amdgcn_readlane(ev.x, i & 63);
 #pragma unroll
     for (int kt = 0; kt < 2; kt++) {
-      const uint32_t u = key_shifts(i, kt);
+      const uint32_t u = key_shifts(i, 0, kt), uk = key_shifts(i, 1, kt);
 #pragma unroll
       for (int t = 0; t < QT; t++) {
         const float up = -1.f / logit_scale(t, kx);
 #pragma unroll
         for (int r = 0; r < 4; r++)
-          sc.s[kt][t][r] = fmaf((float)(u >> 8 * r & 255), up, sc.s[kt][t][r]);
+          sc.s[kt][t][r] =
+              fmaf((float)shift_of(u, r), up, ldexpf(sc.s[kt][t][r], -shift_of(uk, r)));
       }
     }
   };
@@ -468,13 +478,13 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
     const int e_v = __builtin_amdgcn_readlane(ev.y, i & 63);
 #pragma unroll
     for (int kt = 0; kt < 2; kt++) {
-      const uint32_t u = key_shifts(i, kt);
+      const uint32_t u = key_shifts(i, 0, kt);
 #pragma unroll
       for (int t = 0; t < QT; t++)
 #pragma unroll
         for (int r = 0; r < 4; r++)
           lsum[t] += __builtin_amdgcn_exp2f(fmaf(sc.s[kt][t][r], sq[t], off[t]) +
-                                            (float)((int)(u >> 8 * r & 255) - e_v - kSumExp));
+                                            (float)(shift_of(u, r) - e_v - kSumExp));
     }
   };
 
@@ -744,7 +754,7 @@ hipError_t launch_sdpa_packed(const float* q, int64_t ldq, const float* k, int64
       const sdpa::Layout l = sdpa::layout(p, nh, nb);
       if (l.bytes > scratch_bytes) return hipErrorInvalidValue;
       int2* exps = reinterpret_cast<int2*>(packed + l.exps);
-      uint32_t* shifts = reinterpret_cast<uint32_t*>(packed + l.shifts);
+      uint8_t* shifts = reinterpret_cast<uint8_t*>(packed + l.shifts);
       const Parts parts{reinterpret_cast<float*>(packed + l.o),
                         reinterpret_cast<float2*>(packed + l.ml)};
       const int64_t col = (int64_t)h0 * kHd;
@@ -755,7 +765,8 @@ hipError_t launch_sdpa_packed(const float* q, int64_t ldq, const float* k, int64
                          ldv, Lk, p.nkb, packed, exps, shifts);
       const int64_t shares = (int64_t)(p.items - p.nfull) * p.splits;
       hipLaunchKernelGGL(sdpa_packed_kernel, dim3((unsigned)(p.nfull + shares), (unsigned)nb),
-                         dim3(kWaves * 64), 0, s, qb, ldq, packed, exps, shifts, ob, ldo, Lq, Lk,
+                         dim3(kWaves * 64), 0, s, qb, ldq, packed, exps,
+                         reinterpret_cast<const uint32_t*>(shifts), ob, ldo, Lq, Lk,
                          p, scale_log2e, parts);
       if (p.splits > 1)
         hipLaunchKernelGGL(sdpa_combine_kernel,

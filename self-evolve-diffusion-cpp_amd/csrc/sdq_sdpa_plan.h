@@ -35,7 +35,7 @@ struct Plan {
 // Scratch of a launch: at most this, whatever the call (a head's 2^21 keys are
 // 2 GiB of records; their exponents and shifts come on top).
 constexpr int64_t kMaxRecs = int64_t(1) << 31;
-constexpr int64_t kMaxScratch = kMaxRecs + (3 << 20);
+constexpr int64_t kMaxScratch = kMaxRecs + (5 << 20);
 constexpr int64_t kShareBytes = kQ * (kHd * 4 + 8);  // a share's partial output
 
 // `most`: bytes that the partial outputs of one sequence may take. Depends on
@@ -71,7 +71,7 @@ inline Plan make_plan(int64_t Lq, int64_t Lk, int heads, int cu_count, int64_t m
 // Scratch of one launch over `heads` heads of `batch` sequences.
 struct Layout {
   // offsets of its parts (the records lie at 0): the records' exponents, their
-  // keys' shifts, the shares' outputs and sums
+  // keys' shifts (V's, K's), the shares' outputs and sums
   int64_t exps, shifts, o, ml, bytes;
 };
 inline Layout layout(const Plan& p, int64_t heads, int64_t batch) {
@@ -81,7 +81,7 @@ inline Layout layout(const Plan& p, int64_t heads, int64_t batch) {
   Layout l;
   l.exps = recs * kRec;
   l.shifts = l.exps + pad256(recs * 8);
-  l.o = l.shifts + pad256(recs * kKB);
+  l.o = l.shifts + pad256(recs * 2 * kKB);
   l.ml = l.o + rows * kHd * 4;
   l.bytes = l.ml + rows * 8;
   return l;

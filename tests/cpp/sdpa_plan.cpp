@@ -21,7 +21,7 @@ bool check(int64_t Lq, int64_t Lk, int heads, int batch, int cus) {
     return false;
   };
   const sd::Chunk c = sd::chunk(Lq, Lk, heads, batch, cus);
-  if (have > (int64_t(1) << 31) + (3 << 20)) return bad("more than 2 GiB", have, c.seqs);
+  if (have > (int64_t(1) << 31) + (5 << 20)) return bad("more than 2 GiB", have, c.seqs);
   if (c.heads < 1 || c.seqs < 1) return bad("empty chunk", c.heads, c.seqs);
   if (c.heads < heads && c.seqs != 1) return bad("chunk of heads and sequences", c.heads, c.seqs);
   for (int h : {c.heads, heads % c.heads})

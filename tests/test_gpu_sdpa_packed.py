@@ -101,13 +101,14 @@ def test_value_range(sdq_dev, case):
 @pytest.mark.parametrize("Lk", [300, 1024, 5000])
 @pytest.mark.parametrize("cut", [True, False])
 @pytest.mark.parametrize("case", ["falling", "rising", "far_rows", "light_keys", "ignored",
-                                  "outlier_dim", "outlier_element"])
+                                  "outlier_dim", "outlier_element", "short_keys"])
 def test_value_magnitudes(sdq_dev, monkeypatch, case, cut, Lk):
     """V of 2^40 and 2^-90, by halves with blocks of zeros in either order and
     row by row (the small keys count in the softmax's sum all the same); keys
     of 2^-20 of the weight whose V is 2^20 times larger; keys of no weight whose
-    V is 2^100; a dimension 2^16 and an element 2^12 above the others. Every
-    output dimension to its own scale, with the keys cut into shares and not."""
+    V is 2^100; a dimension 2^16 and an element 2^12 above the others; keys 2^30
+    shorter than their neighbours, of all the weight. Every output dimension to
+    its own scale, with the keys cut into shares and not."""
     import torch
 
     print(f"[sdpa-packed] magnitudes {case} Lk={Lk} cut={cut}", flush=True)
@@ -136,6 +137,10 @@ def test_value_magnitudes(sdq_dev, monkeypatch, case, cut, Lk):
         v[1::3] *= 2.0 ** (20 if case == "light_keys" else 100)
     elif case == "outlier_dim":
         v[:, 7] *= 2.0 ** 16
+    elif case == "short_keys":
+        q.abs_()
+        kv[1::2, :C] = -kv[1::2, :C].abs() * 2.0 ** 30
+        v[32:64] = 0.0
     else:
         v[17, 5] *= 2.0 ** 12
     want = _want64(q, kv, heads)
