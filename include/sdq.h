@@ -161,7 +161,11 @@ int sdq_weight_export_host(const sdq_weight* w, int8_t* q, float* scale);
  * stream and allocates. Under HIP-graph capture such a call is refused with
  * SDQ_ERR_INVALID before anything is queued (the capture stays usable); one
  * call of the same shape on the stream before the capture makes the captured
- * call allocation-free, and its graph replays bit-identical results.
+ * call allocation-free, and its graph replays bit-identical results. A buffer
+ * that a captured call uses is kept when the workspace grows later, so the
+ * graph stays valid (every entry point with a workspace, attention included).
+ * Its replays use the capture stream's workspace: run them on that stream, or
+ * ordered with its other work by events, one at a time.
  * Replaces: sd::qgemm (src/core/tensor.h:52) + mlin's bias pass
  * (src/model/ovi_dit.cpp:66-84) + the consumer named by epi->kind. */
 int sdq_qlinear(const sdq_weight* w, const float* A, int64_t M, int64_t K, const sdq_epilogue* epi,

@@ -143,6 +143,20 @@ int ensure_device(int dev) {
   return SDQ_OK;
 }
 
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+// Workspace buffers handed out under capture: a graph may be replayed at any
+// time with their addresses, so they are kept when a larger one takes their
+// place (until the process ends; nothing says when the last graph is gone).
+std::set<void*> g_captured;
+
 // Grows (never shrinks) the workspace of (dev, stream). A buffer that is
 // replaced may still be read by work queued on `stream`, so the stream is
 // drained before the old buffer is freed. A stream that is capturing a graph
@@ -150,7 +164,16 @@ int ensure_device(int dev) {
 // error that leaves the capture intact (a call of the same size or larger on
 // the stream before the capture grows it in advance).
 int grow(hipStream_t s, void** p, size_t* have, size_t need) {
-  if (*have >= need) return SDQ_OK;
+  if (*have >= need) {
+    if (*p && capturing(s)) {
+      try {
+        g_captured.insert(*p);
+      } catch (...) {
+        return set_error(SDQ_ERR_NOMEM, "host allocation failed");
+      }
+    }
+    return SDQ_OK;
+  }
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   hipError_t e = hipStreamIsCapturing(s, &st);
   if (e != hipSuccess) return hip_error(e, "hipStreamIsCapturing");
@@ -160,7 +183,7 @@ int grow(hipStream_t s, void** p, size_t* have, size_t need) {
                      "graph: make the same call once on this stream before the capture");
   e = hipStreamSynchronize(s);
   if (e != hipSuccess) return hip_error(e, "hipStreamSynchronize");
-  if (*p) (void)hipFree(*p);
+  if (*p && !g_captured.count(*p)) (void)hipFree(*p);
   *p = nullptr;
   *have = 0;
   e = hipMalloc(p, need);
@@ -180,14 +203,10 @@ int workspace(int dev, hipStream_t s, size_t at_bytes, size_t as_bytes, size_t c
   int rc = grow(s, reinterpret_cast<void**>(&w.at), &w.at_bytes, at_bytes);
   if (!rc) rc = grow(s, reinterpret_cast<void**>(&w.as), &w.as_bytes, as_bytes);
   size_t cb = w.col_cap * 2 * sizeof(float);
-  if (!rc && cb < col_cap * 2 * sizeof(float)) {
-    rc = grow(s, reinterpret_cast<void**>(&w.cols), &cb, col_cap * 2 * sizeof(float));
-    if (!rc) w.col_cap = col_cap;
-  }
-  if (!rc && !w.sink) {
-    size_t have = 0;
-    rc = grow(s, reinterpret_cast<void**>(&w.sink), &have, 4096);
-  }
+  if (!rc) rc = grow(s, reinterpret_cast<void**>(&w.cols), &cb, col_cap * 2 * sizeof(float));
+  if (!rc) w.col_cap = cb / (2 * sizeof(float));
+  size_t sb = w.sink ? 4096 : 0;  // never replaced
+  if (!rc) rc = grow(s, reinterpret_cast<void**>(&w.sink), &sb, 4096);
   if (!rc && part_bytes) rc = grow(s, reinterpret_cast<void**>(&w.part), &w.part_bytes, part_bytes);
   if (!rc && pmax_bytes) rc = grow(s, reinterpret_cast<void**>(&w.pmax), &w.pmax_bytes, pmax_bytes);
   if (rc) return rc;

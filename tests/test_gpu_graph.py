@@ -124,6 +124,65 @@ def test_growth_under_capture_is_refused(sdq_dev, oracle):
     _replays(sdq_dev, oracle, sdq.qlinear, M, K, N, "none", 300, warm=True)
     w.free()
 
+
+
+@pytest.mark.parametrize("entry", ["sdpa", "qlinear"])
+def test_graph_outlives_workspace_growth(sdq_dev, oracle, entry):
+    """A graph captured on a warmed-up stream, then a larger eager call on that
+    stream, whose workspace takes new buffers, then memory of the old buffers'
+    sizes overwritten: the replays still give the eager results."""
+    import torch
+
+    import sdq
+
+    print(f"[graph] growth after capture {entry}", flush=True)
+    s = torch.cuda.Stream()
+    g = torch.Generator(device=sdq_dev)
+    g.manual_seed(11)
+
+    def rand(*shape):
+        return torch.randn(shape, generator=g, device=sdq_dev)
+
+    if entry == "sdpa":
+        make = lambda n: (rand(n, 3 * 256), torch.zeros((n, 256), device=sdq_dev))  # noqa: E731
+        call = lambda x, y: sdq.sdpa(x, x, x, y, 2, qcol=0, kcol=256, vcol=512)  # noqa: E731
+        sizes = (70001, 90001)  # beyond any other test's, whatever stream torch hands out
+    else:
+        W = oracle.randn(512 * 256, 400).reshape(512, 256) * np.float32(0.02)
+        w = sdq.Weight.from_host(*oracle.quant_rows(W))
+        make = lambda n: (rand(n, 256), torch.zeros((n, 512), device=sdq_dev))  # noqa: E731
+        call = lambda x, y: sdq.qlinear(w, x, y)  # noqa: E731
+        sizes = (300000, 400000)
+    (x, y), (x2, y2) = make(sizes[0]), make(sizes[1])
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        call(x, y)
+    s.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        call(x, y)
+    with torch.cuda.stream(s):
+        call(x2, y2)  # grows
+    s.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    junk = [torch.full((2 ** 26,), float("nan"), device=sdq_dev)
+            for _ in range(min(24, free // 2 ** 29))]
+    want = torch.zeros_like(y)
+    for rep in range(3):
+        x.copy_(rand(*x.shape))
+        y.fill_(-1.0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(s):
+            graph.replay()
+        s.synchronize()
+        with torch.cuda.stream(s):
+            call(x, want)
+        s.synchronize()
+        assert torch.equal(y, want), f"{entry} replay {rep}"
+    assert all(bool(j.isnan().all()) for j in junk)
+    del graph
+
+
 _BLOCK_NAMES = ("q", "k", "v", "o", "cq", "ck", "cv", "co", "kf", "vf", "fc1", "fc2")
 
 
