@@ -196,6 +196,15 @@ int grow(hipStream_t s, void** p, size_t* have, size_t need) {
   return SDQ_OK;
 }
 
+// The same for a buffer that the call can do without: a failure leaves no
+// error text behind.
+bool try_grow(hipStream_t s, void** p, size_t* have, size_t need) {
+  const std::string before = t_err;
+  if (grow(s, p, have, need) == SDQ_OK) return true;
+  t_err = before;
+  return false;
+}
+
 int workspace(int dev, hipStream_t s, size_t at_bytes, size_t as_bytes, size_t col_cap,
               size_t part_bytes, size_t pmax_bytes, Workspace** out) {
   std::lock_guard<std::mutex> lk(g_mu);
@@ -492,8 +501,8 @@ int qlinear_device(const sdq_weight* w, const float* A, int64_t M, int64_t K,
     tail_splitk = rmax_out ? 1 : choose_splitk(kCfg128x128, M - Ma, N, w->KFp, cu_count);
     if (tail_splitk > 1) {
       std::lock_guard<std::mutex> lk(g_mu);
-      if (grow(s, reinterpret_cast<void**>(&ws->part), &ws->part_bytes,
-               (size_t)tail_splitk * (size_t)(M - Ma) * (size_t)N * 4) == SDQ_OK)
+      if (try_grow(s, reinterpret_cast<void**>(&ws->part), &ws->part_bytes,
+                   (size_t)tail_splitk * (size_t)(M - Ma) * (size_t)N * 4))
         tail_part = ws->part;
     }
   }
@@ -1873,9 +1882,12 @@ int sdq_sdpa_batched(const float* q, int64_t ldq, const float* k, int64_t ldk, c
   // not refused for want of memory, under graph capture either.
   float* scratch = nullptr;
   const int64_t need = sdpa_packed_bytes(Lq, Lk, heads, batch, cu_count);
-  if (need > 0 && ws_floats(dev, s, &Workspace::sdpa, &Workspace::sdpa_bytes, (size_t)need,
-                            &scratch) != SDQ_OK)
-    scratch = nullptr;
+  if (need > 0) {
+    std::lock_guard<std::mutex> lk(g_mu);
+    Workspace& ws = g_ws[{dev, s}];
+    if (try_grow(s, reinterpret_cast<void**>(&ws.sdpa), &ws.sdpa_bytes, (size_t)need))
+      scratch = ws.sdpa;
+  }
   hipEvent_t p0 = t_prof ? prof_mark(s) : nullptr;
   const hipError_t e =
       scratch ? launch_sdpa_packed(q, ldq, k, ldk, v, ldv, out, ldo, Lq, Lk, heads, s, batch,

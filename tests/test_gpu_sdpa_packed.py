@@ -210,3 +210,25 @@ def test_capture_without_warm_up(sdq_dev):
         torch.cuda.synchronize()
         want = _want64(q, kv, 2)
         assert float((out.double() - want).abs().max() / want.abs().max()) <= 2e-5
+
+
+def test_fallback_leaves_no_error_text(sdq_dev):
+    """A call that does without its scratch (a capture whose workspace would
+    have to grow) succeeds, and the thread's last error stays the one before."""
+    import torch
+
+    import sdq
+
+    print("[sdpa-packed] error text", flush=True)
+    q = torch.zeros((40, 384), device=sdq_dev)
+    kv = torch.zeros((120_000, 768), device=sdq_dev)  # more than any stream has had
+    out = torch.empty((40, 384), device=sdq_dev)
+    torch.cuda.synchronize()
+    lib = sdq.load_library()
+    assert lib.sdq_add(None, None, -1, None) != 0
+    before = lib.sdq_last_error()
+    assert before
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        sdq.sdpa(q, kv, kv, out, 3, kcol=0, vcol=384)
+    assert lib.sdq_last_error() == before
