@@ -1742,10 +1742,10 @@ int sdq_rmsnorm_rope_batch(const sdq_rms_seg* segs, int nseg, int64_t C, int hea
   if ((rc = ensure_device(dev))) return rc;
   const hipStream_t s = static_cast<hipStream_t>(stream);
   float* inv = nullptr;
-  if (rows_w > 0 &&
+  if (rows_w > 0 && !rms_rows_fits(g, n, C, heads) &&
       (rc = ws_floats(dev, s, &Workspace::rinv, &Workspace::rinv_bytes, (size_t)rows_w * 4, &inv)))
     return rc;
-  for (int i = 0; i < n; i++)
+  for (int i = 0; i < n && inv; i++)
     if (g[i].w) {
       g[i].inv = inv;
       inv += g[i].L;

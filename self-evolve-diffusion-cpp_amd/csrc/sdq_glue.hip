@@ -219,17 +219,27 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 }  // namespace
 
+bool rms_rows_fits(const RmsSeg* segs, int nseg, int64_t C, int heads) {
+  bool rows = C % 4 == 0 && C <= rowblock::kMaxCols && C / heads % 4 == 0;
+  for (int i = 0; i < nseg; i++) {
+    const RmsSeg& g = segs[i];
+    rows = rows && aligned16(g.x) && g.ld % 4 == 0 && (g.L == 0 || (g.w && aligned16(g.w)));
+  }
+  return rows;
+}
+
 hipError_t launch_rmsnorm_rope_segs(const RmsSeg* segs, int nseg, int64_t C, int heads, float eps,
                                     hipStream_t s) {
   if (nseg < 1 || nseg > kMaxRmsSegs || C <= 0 || heads <= 0 || C % heads || (C / heads) % 2)
     return hipErrorInvalidValue;
   RmsSegs st{};
   st.n = nseg;
-  bool vec = C % 4 == 0, few = true, any_w = false, all_w = true, full = C % 32 == 0;
+  const bool rows = rms_rows_fits(segs, nseg, C, heads);
+  bool vec = C % 4 == 0, few = true, any_w = false, full = C % 32 == 0;
   for (int i = 0; i < nseg; i++) {
     const RmsSeg& g = segs[i];
     if (g.L < 0 || g.ld < C || g.nr < 0 || g.nr > C / heads / 2 || (!g.w && !g.cs) ||
-        (g.w && !g.inv) || (g.L > 0 && !g.x))
+        (g.w && !g.inv && !rows) || (g.L > 0 && !g.x))
       return hipErrorInvalidValue;
     st.s[i] = g;
     st.blk0[i + 1] = st.blk0[i] + (g.w ? ceil_div(g.L, 8) : 0);
@@ -237,12 +247,9 @@ hipError_t launch_rmsnorm_rope_segs(const RmsSeg* segs, int nseg, int64_t C, int
     vec = vec && aligned16(g.x) && g.ld % 4 == 0;
     few = few && g.L <= 4096;
     any_w = any_w || (g.w && g.L > 0);
-    all_w = all_w && (g.w || g.L == 0);
     full = full && (g.L == 0 || seg_span_bytes(g, C) <= kFullMaxBytes);
   }
   full = full && vec;
-  bool rows = vec && all_w && C <= rowblock::kMaxCols && C / heads % 4 == 0;
-  for (int i = 0; i < nseg; i++) rows = rows && (segs[i].L == 0 || aligned16(segs[i].w));
   if (rows) {
     for (int i = 0; i < nseg; i++)
       st.blk0[i + 1] = st.blk0[i] + ceil_div(segs[i].L, rowblock::kRows);

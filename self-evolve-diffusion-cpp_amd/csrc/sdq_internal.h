@@ -126,7 +126,7 @@ hipError_t launch_act_quant_frags_lnmod_rows(const float* A, int64_t M, int64_t 
 // table cs [L][nr] (cs == nullptr: no RoPE). inv: [L] scratch.
 // One column block of strided rows for launch_rmsnorm_rope_segs: L rows of
 // stride ld at x; w NULL = rotation only; cs NULL / nr 0 = no rotation; inv
-// [L] floats of scratch when w is set.
+// [L] floats of scratch when w is set and rms_rows_fits does not hold.
 struct RmsSeg {
   float* x;
   int64_t L, ld;
@@ -136,6 +136,9 @@ struct RmsSeg {
   float* inv;
 };
 constexpr int kMaxRmsSegs = 4;
+// Segments that one pass takes, without scratch (every one weighted, up to 3072
+// columns, 16-byte aligned rows and weights).
+bool rms_rows_fits(const RmsSeg* segs, int nseg, int64_t C, int heads);
 hipError_t launch_rmsnorm_rope_segs(const RmsSeg* segs, int nseg, int64_t C, int heads, float eps,
                                     hipStream_t s);
 hipError_t launch_rmsnorm_rope(float* x, int64_t L, int64_t C, int64_t ld, const float* w,

@@ -99,3 +99,34 @@ def test_quantizer_rounding(sdq_dev, oracle, v):
     torch.cuda.synchronize()
     codes, _ = oracle.act_quant(x)
     assert_bitexact(Y.cpu().numpy(), np.tile(codes[:, :N].astype(np.int32), (12, 1)), "codes")
+
+
+def test_rmsnorm_rope_captures_without_warm_up(sdq_dev, oracle):
+    """One pass needs no scratch: more rows than any stream has had are
+    captured with no call before, and every replay equals the eager call."""
+    import torch
+
+    import sdq
+
+    L, C, heads = 300_000, 256, 2
+    print(f"[rowblock] capture L={L} C={C}", flush=True)
+    g = torch.Generator(device=sdq_dev)
+    g.manual_seed(3)
+    src = torch.randn((L, C), generator=g, device=sdq_dev)
+    w = torch.randn(C, generator=g, device=sdq_dev)
+    cs = torch.randn((L, 64, 2), generator=g, device=sdq_dev)
+    x = src.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        sdq.rmsnorm_rope_batch([(x, 0, w, cs)], C, heads)
+    for rep in range(3):
+        src.normal_(generator=g)
+        x.copy_(src)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = src.clone()
+        sdq.rmsnorm_rope_batch([(want, 0, w, cs)], C, heads)
+        torch.cuda.synchronize()
+        assert torch.equal(x, want), rep
