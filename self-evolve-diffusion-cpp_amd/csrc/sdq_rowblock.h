@@ -34,6 +34,9 @@ constexpr int kThreads = 64 * (kWaves + 1);
 constexpr int kChunk = 256;    // columns per chunk
 constexpr int kMaxChunks = 12;
 constexpr int64_t kMaxCols = kMaxChunks * kChunk;
+// Workgroups of one launch: a grid holds fewer than 2^32 threads. (The two-kernel
+// form, 8 threads per row, goes on beyond.)
+constexpr int64_t kMaxBlocks = ((int64_t(1) << 32) - 1) / kThreads;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 

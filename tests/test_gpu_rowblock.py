@@ -130,3 +130,29 @@ def test_rmsnorm_rope_captures_without_warm_up(sdq_dev, oracle):
         sdq.rmsnorm_rope_batch([(want, 0, w, cs)], C, heads)
         torch.cuda.synchronize()
         assert torch.equal(x, want), rep
+
+
+def test_more_rows_than_one_grid_holds(sdq_dev):
+    """Rows beyond one launch of 14-row workgroups still run: the last ones
+    equal a call on them alone."""
+    import torch
+
+    import sdq
+
+    M, K = 117_440_512 + 5, 4
+    print(f"[rowblock] rows M={M} K={K}", flush=True)
+    x = torch.randn((M, K), device=sdq_dev)
+    w, b = torch.randn(K, device=sdq_dev), torch.randn(K, device=sdq_dev)
+    cs = torch.randn((1, 2, 2), device=sdq_dev).expand(M, 2, 2).contiguous()
+    y = torch.empty_like(x)
+    sdq.layernorm(x, y, w, b)
+    for r in (slice(0, 99), slice(M - 99, M)):
+        want = torch.empty((99, K), device=sdq_dev)
+        sdq.layernorm(x[r].contiguous(), want, w, b)
+        assert torch.equal(y[r], want)
+    y.copy_(x)
+    sdq.rmsnorm_rope_batch([(y, 0, w, cs)], K, 1)
+    for r in (slice(0, 99), slice(M - 99, M)):
+        want = x[r].contiguous()
+        sdq.rmsnorm_rope_batch([(want, 0, w, cs[:99].contiguous())], K, 1)
+        assert torch.equal(y[r], want)
