@@ -83,6 +83,7 @@ struct Workspace {
   size_t grp_bytes = 0;
   float* sdpa = nullptr;  // attention: packed K and V, shares' partial outputs
   size_t sdpa_bytes = 0;
+  std::mutex sdpa_mu;  // held from its lookup to the last launch that uses it
 };
 std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
 
@@ -1880,11 +1881,17 @@ int sdq_sdpa_batched(const float* q, int64_t ldq, const float* k, int64_t ldk, c
   // The packed form when its scratch can be had (at most
   // sdpa::kMaxScratch bytes), else the form without scratch: an attention call is
   // not refused for want of memory, under graph capture either.
+  // Threads that share the stream queue their calls' launches one after the
+  // other, so that each call's scratch is its own until the next begins.
   float* scratch = nullptr;
+  std::unique_lock<std::mutex> turn;
   const int64_t need = sdpa_packed_bytes(Lq, Lk, heads, batch, cu_count);
   if (need > 0) {
-    std::lock_guard<std::mutex> lk(g_mu);
+    std::unique_lock<std::mutex> lk(g_mu);
     Workspace& ws = g_ws[{dev, s}];
+    lk.unlock();
+    turn = std::unique_lock<std::mutex>(ws.sdpa_mu);
+    lk.lock();
     if (try_grow(s, reinterpret_cast<void**>(&ws.sdpa), &ws.sdpa_bytes, (size_t)need))
       scratch = ws.sdpa;
   }

@@ -232,3 +232,45 @@ def test_fallback_leaves_no_error_text(sdq_dev):
     with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
         sdq.sdpa(q, kv, kv, out, 3, kcol=0, vcol=384)
     assert lib.sdq_last_error() == before
+
+
+def test_threads_on_one_stream(sdq_dev):
+    """Four threads with their own inputs on one stream, sizes that grow the
+    workspace among them: every result equals the call alone."""
+    import threading
+
+    import torch
+
+    import sdq
+
+    print("[sdpa-packed] threads", flush=True)
+    g = torch.Generator(device=sdq_dev)
+    g.manual_seed(12)
+    heads, C = 3, 384
+    sizes = [1100, 1500, 2300, 150_000]
+    xs = [torch.randn((min(n, 1500), C), generator=g, device=sdq_dev) for n in sizes]
+    kvs = [torch.randn((n, 2 * C), generator=g, device=sdq_dev) for n in sizes]
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    outs = [[torch.zeros_like(x) for _ in range(8)] for x in xs]
+    torch.cuda.synchronize()
+    go = threading.Barrier(len(sizes))
+
+    def run(i):
+        sdq.init(0)
+        go.wait()
+        for out in outs[i]:
+            sdq.sdpa(xs[i], kvs[i], kvs[i], out, heads, kcol=0, vcol=C, stream=s)
+
+    threads = [threading.Thread(target=run, args=(i,)) for i in range(len(sizes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    s.synchronize()
+    for i, x in enumerate(xs):
+        want = torch.zeros_like(x)
+        sdq.sdpa(x, kvs[i], kvs[i], want, heads, kcol=0, vcol=C, stream=s)
+        s.synchronize()
+        for out in outs[i]:
+            assert torch.equal(out, want), sizes[i]
