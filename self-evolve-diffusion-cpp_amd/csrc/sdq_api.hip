@@ -87,6 +87,13 @@ struct Workspace {
 };
 std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
 
+// The workspace of (device, stream), under g_mu. hipStreamPerThread is another
+// stream in every thread: the thread's own address stands for it.
+Workspace& ws_of(int dev, hipStream_t s) {
+  thread_local char self;
+  return g_ws[{dev, s == hipStreamPerThread ? reinterpret_cast<hipStream_t>(&self) : s}];
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // ---- optional per-kernel event timing (sdq_profile_begin/end) ----
@@ -209,7 +216,7 @@ bool try_grow(hipStream_t s, void** p, size_t* have, size_t need) {
 int workspace(int dev, hipStream_t s, size_t at_bytes, size_t as_bytes, size_t col_cap,
               size_t part_bytes, size_t pmax_bytes, Workspace** out) {
   std::lock_guard<std::mutex> lk(g_mu);
-  Workspace& w = g_ws[{dev, s}];
+  Workspace& w = ws_of(dev, s);
   int rc = grow(s, reinterpret_cast<void**>(&w.at), &w.at_bytes, at_bytes);
   if (!rc) rc = grow(s, reinterpret_cast<void**>(&w.as), &w.as_bytes, as_bytes);
   size_t cb = w.col_cap * 2 * sizeof(float);
@@ -229,7 +236,7 @@ int workspace(int dev, hipStream_t s, size_t at_bytes, size_t as_bytes, size_t c
 int ws_floats(int dev, hipStream_t s, float* Workspace::*buf, size_t Workspace::*have,
               size_t bytes, float** out) {
   std::lock_guard<std::mutex> lk(g_mu);
-  Workspace& w = g_ws[{dev, s}];
+  Workspace& w = ws_of(dev, s);
   int rc = grow(s, reinterpret_cast<void**>(&(w.*buf)), &(w.*have), bytes);
   if (rc) return rc;
   *out = w.*buf;
@@ -1255,7 +1262,7 @@ int sdq_qlinear_group(const sdq_group_item* items, int n, void* stream) {
     char* base = nullptr;
     {
       std::lock_guard<std::mutex> lk(g_mu);
-      Workspace& ws = g_ws[{dev, s}];
+      Workspace& ws = ws_of(dev, s);
       if ((rc = grow(s, reinterpret_cast<void**>(&ws.grp), &ws.grp_bytes, off))) return rc;
       base = ws.grp;
     }
@@ -1532,7 +1539,7 @@ int sdq_qlinear_stack(const sdq_group_item* items, int n, int ngroup, const sdq_
   char* base = nullptr;
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    Workspace& ws = g_ws[{dev, s}];
+    Workspace& ws = ws_of(dev, s);
     if ((rc = grow(s, reinterpret_cast<void**>(&ws.grp), &ws.grp_bytes, off))) return rc;
     base = ws.grp;
   }
@@ -1789,7 +1796,7 @@ int sdq_layernorm(const float* x, int64_t M, int64_t K, const float* w, const fl
   float2* st = nullptr;
   if (!rows) {
     std::lock_guard<std::mutex> lk(g_mu);
-    Workspace& ws = g_ws[{dev, s}];
+    Workspace& ws = ws_of(dev, s);
     if ((rc = grow(s, reinterpret_cast<void**>(&ws.st), &ws.st_bytes, (size_t)M * sizeof(float2))))
       return rc;
     st = ws.st;
@@ -1888,7 +1895,7 @@ int sdq_sdpa_batched(const float* q, int64_t ldq, const float* k, int64_t ldk, c
   const int64_t need = sdpa_packed_bytes(Lq, Lk, heads, batch, cu_count);
   if (need > 0) {
     std::unique_lock<std::mutex> lk(g_mu);
-    Workspace& ws = g_ws[{dev, s}];
+    Workspace& ws = ws_of(dev, s);
     lk.unlock();
     turn = std::unique_lock<std::mutex>(ws.sdpa_mu);
     lk.lock();

@@ -234,23 +234,26 @@ def test_fallback_leaves_no_error_text(sdq_dev):
     assert lib.sdq_last_error() == before
 
 
-def test_threads_on_one_stream(sdq_dev):
+@pytest.mark.parametrize("shared", [True, False])
+def test_threads_on_one_stream(sdq_dev, shared):
     """Four threads with their own inputs on one stream, sizes that grow the
-    workspace among them: every result equals the call alone."""
+    workspace among them: every result equals the call alone. The same on the
+    per-thread stream, one handle for a stream of each thread."""
     import threading
 
     import torch
 
     import sdq
 
-    print("[sdpa-packed] threads", flush=True)
+    print(f"[sdpa-packed] threads shared={shared}", flush=True)
     g = torch.Generator(device=sdq_dev)
     g.manual_seed(12)
     heads, C = 3, 384
     sizes = [1100, 1500, 2300, 150_000]
     xs = [torch.randn((min(n, 1500), C), generator=g, device=sdq_dev) for n in sizes]
     kvs = [torch.randn((n, 2 * C), generator=g, device=sdq_dev) for n in sizes]
-    s = torch.cuda.Stream()
+    own = torch.cuda.Stream()
+    s = own if shared else 2  # hipStreamPerThread
     torch.cuda.synchronize()
     outs = [[torch.zeros_like(x) for _ in range(8)] for x in xs]
     torch.cuda.synchronize()
@@ -267,10 +270,10 @@ def test_threads_on_one_stream(sdq_dev):
         t.start()
     for t in threads:
         t.join()
-    s.synchronize()
+    torch.cuda.synchronize()
     for i, x in enumerate(xs):
         want = torch.zeros_like(x)
-        sdq.sdpa(x, kvs[i], kvs[i], want, heads, kcol=0, vcol=C, stream=s)
-        s.synchronize()
+        sdq.sdpa(x, kvs[i], kvs[i], want, heads, kcol=0, vcol=C, stream=own)
+        own.synchronize()
         for out in outs[i]:
             assert torch.equal(out, want), sizes[i]
