@@ -51,8 +51,17 @@ inline Plan make_plan(int64_t Lq, int64_t Lk, int heads, int cu_count, int64_t m
   const int cus = cu_count > 0 ? cu_count : 256;
   p.nfull = p.items / cus * cus;
   const int rest = p.items - p.nfull;
-  if (rest == 0 || std::getenv("SDQ_SDPA_SPLIT")) {  // the variable: comparisons without shares
+  // for comparisons: a factor (2 to 16, where the shares fit), below 2 no cut
+  const char* forced = std::getenv("SDQ_SDPA_SPLIT");
+  int f = forced ? std::atoi(forced) : 0;
+  if (rest == 0 || (forced && f < 2)) {
     p.nfull = p.items;
+    return p;
+  }
+  if (forced) {
+    for (f = f < 16 ? f : 16; f > 1 && rest * f * kShareBytes > most;) f--;
+    p.kbs = (p.nkb + f - 1) / f;
+    p.splits = (p.nkb + p.kbs - 1) / p.kbs;  // no empty share
     return p;
   }
   // The cut that ends first, in key-block times: rounds of shares, each with

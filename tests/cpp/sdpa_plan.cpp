@@ -1,7 +1,8 @@
 // Sweeps the packed attention's host plan (csrc/sdq_sdpa_plan.h): every launch
 // of a call must lie inside the scratch that is asked for the call, that
 // scratch inside 2 GiB (and its records' exponents), and every item's keys must
-// be covered once. Prints the first call that breaks a rule.
+// be covered once. Prints the first call that breaks a rule. With an argument:
+// prints one call's cut.
 #include <cmath>
 #include <cstdio>
 #include <random>
@@ -40,7 +41,12 @@ bool check(int64_t Lq, int64_t Lk, int heads, int batch, int cus) {
 
 }  // namespace
 
-int main() {
+int main(int argc, char**) {
+  if (argc > 1) {  // the cut of 157 queries x 768 keys x 24 heads
+    const sd::Plan p = sd::launch_plan(157, 768, 24, 256);
+    std::printf("%d shares of %d blocks\n", p.splits, p.kbs);
+    return 0;
+  }
   // shares' outputs beyond the records: 2.7, 3.0 and 49 GiB without a bound of
   // their own; then ragged last chunks of heads
   bool ok = check(27280, 1 << 20, 1, 1, 256) && check(1024, 1024, 24, 64, 256) &&
