@@ -419,7 +419,8 @@ int sdq_profile_end(sdq_kernel_time* out, int max_records, int* n_records);
  * operands, N % 4 == 0): one, or two when a 256x256 launch hands its last
  * rows to a 128x128 launch; for each, the record name sdq_profile_end uses
  * and the activation rows [row0, row0 + rows) it covers, so a caller can
- * price each kernel's own work. No GPU work is done.
+ * price each kernel's own work ("..._splitk": with the sum of its k-ranges).
+ * No GPU work is done.
  * Replaces: nothing in the reference (measurement support). */
 typedef struct sdq_gemm_plan {
   int nlaunch;

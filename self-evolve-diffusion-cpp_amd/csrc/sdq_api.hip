@@ -505,7 +505,8 @@ int qlinear_device(const sdq_weight* w, const float* A, int64_t M, int64_t K,
   int tail_splitk = 1;
   int* tail_part = nullptr;
   if (const int64_t Ma = cfg == kCfg256x256 && !fixed ? tail_split_rows(M, N, cu_count) : 0) {
-    // row maxima come from the unsplit launch only
+    // row maxima come from the unsplit launch only (sdq_qlinear_plan names the
+    // rest by the same rule)
     tail_splitk = rmax_out ? 1 : choose_splitk(kCfg128x128, M - Ma, N, w->KFp, cu_count);
     if (tail_splitk > 1) {
       std::lock_guard<std::mutex> lk(g_mu);
@@ -530,9 +531,9 @@ int qlinear_device(const sdq_weight* w, const float* A, int64_t M, int64_t K,
       const std::string g = std::string("qgemm_") + gemm_cfg_name(cfg) + (splitk > 1 ? "_splitk" : "");
       if (tail) {
         // the 256x256 launch over the full rounds' rows, then the 128x128
-        // launch over the remaining rows: one record each
+        // launch (its split and sum) over the remaining rows: one record each
         t_recs.push_back({g, p1, pmid});
-        t_recs.push_back({"qgemm_tail128", pmid, p2});
+        t_recs.push_back({tail_part ? "qgemm_tail128_splitk" : "qgemm_tail128", pmid, p2});
         pmid = nullptr;
       } else {
         t_recs.push_back({g, p1, p2});
@@ -2165,7 +2166,8 @@ int sdq_qlinear_plan(const sdq_weight* w, int64_t M, int epi_kind, sdq_gemm_plan
   const int64_t Ma = (cfg == kCfg256x256 && w->K > 0) ? tail_split_rows(M, w->N, cu) : 0;
   if (Ma > 0) {
     put(g, 0, Ma);
-    put("qgemm_tail128", Ma, M - Ma);
+    const bool split = choose_splitk(kCfg128x128, M - Ma, w->N, w->KFp, cu) > 1;
+    put(split ? "qgemm_tail128_splitk" : "qgemm_tail128", Ma, M - Ma);
   } else {
     put(g, 0, M);
   }

@@ -25,7 +25,7 @@ def test_tail_splitk_bitexact(sdq_dev, oracle, M, kind):
     bias, gate = oracle.randn(N, 4), oracle.randn(N, 5)
     w = sdq.Weight.from_host(q, s)
     plan = sdq.qlinear_plan(w, M, kind)
-    assert plan[1] == ("qgemm_tail128", 10752, M - 10752), plan
+    assert plan[1] == ("qgemm_tail128_splitk", 10752, M - 10752), plan
     t = lambda a: torch.from_numpy(a).to(sdq_dev)  # noqa: E731
     resid = torch.randn((M, N), generator=g, device=sdq_dev)
     kw = {}
@@ -37,8 +37,10 @@ def test_tail_splitk_bitexact(sdq_dev, oracle, M, kind):
     else:
         Y = resid.clone()
         kw = dict(bias=t(bias), resid=Y, gate=t(gate) if kind == "gated" else None)
+    sdq.profile_begin()
     sdq.qlinear(w, A, Y, kind=kind, **kw)
     torch.cuda.synchronize()
+    assert "qgemm_tail128_splitk" in sdq.profile_end()
     rows = np.r_[0:3, 10749:10756, M // 2, max(10752, M - 5):M]
     rows = np.unique(rows[rows < M])
     a = A[torch.from_numpy(rows).to(sdq_dev)].cpu().numpy()
