@@ -315,6 +315,24 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
     for (int c = 0; c < LD; c++)
       dev::dma16<0>(rs, voff, soff(i) + kRecV + c * 1024u, slot_v(i) + c * 1024u);
   };
+  const int n = kb1 - kb0;
+  // A wave past the queries moves its share of the blocks and no more (the
+  // same waits and barriers as below).
+  if (q0 >= Lq) {
+    issue_k(0), issue_v(0), issue_k(1), issue_v(1), issue_k(2), issue_v(2), issue_k(3);
+    __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(6 * LD));
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(4 * LD));
+    asm volatile("s_barrier" ::: "memory");
+    issue_k(4);
+    for (int i = 0; i < n; i++) {
+      __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(3 * LD));
+      asm volatile("s_barrier" ::: "memory");
+      issue_v(i + 3), issue_k(i + 5);
+    }
+    __builtin_amdgcn_s_waitcnt(dev::waitcnt_vm(0));
+    return;
+  }
   float neg1 = -1.f;  // for split_pair
   asm volatile("" : "+s"(neg1));
   // Everything the first scores need is asked for at once: block exponents
@@ -372,7 +390,6 @@ sdpa_packed_kernel(const float* __restrict__ Q, int64_t ldq, const char* __restr
     vr = __builtin_elementwise_max(
         vr, __builtin_bit_cast(v2s, __shfl_xor(__builtin_bit_cast(int, vr), d)));
   const int vmin = vr.x == -1000 ? 0 : -vr.y, vfar = vr.x - kFar;
-  const int n = kb1 - kb0;
   // the partial block, if this range ends with it (else never reached)
   const int rem = (int)(Lk % kKB);
   const int last = rem && kb1 == nkb ? n - 1 : -1;
