@@ -328,9 +328,10 @@ int sdq_add(float* x, const float* y, int64_t n, void* stream);
  * dimension far below its head's largest loses low bits: it is within 2e-5 of
  * its own scale at 2^-12 of the largest, within 4e-4 at 2^-20. K and V are
  * packed once into scratch of the stream's workspace (at most 2 GiB and 5 MiB,
- * grown and kept like the others); where that cannot be had (a stream capturing
- * a graph before it has grown, no device memory) a slower form without scratch
- * runs, to the same bound.
+ * grown and kept like the others); at most 64 queries over more than 4096 keys
+ * run in one pass over K and V instead, with scratch for partial outputs. Where
+ * scratch cannot be had (a stream capturing a graph before it has grown, no
+ * device memory) a slower form without it runs, to the same bound.
  * 16-byte aligned rows. Stream-ordered. */
 int sdq_sdpa(const float* q, int64_t ldq, const float* k, int64_t ldk, const float* v, int64_t ldv,
              float* out, int64_t ldo, int64_t Lq, int64_t Lk, int heads, int head_dim,

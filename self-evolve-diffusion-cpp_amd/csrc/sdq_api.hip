@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "sdq_internal.h"
+#include "sdq_sdpa_plan.h"
 
 // Scratch memory of sdq_qlinear_noalloc: a file-scope device array, one copy
 // per GPU (each holds it until the process ends). In host code this name is
@@ -1893,7 +1894,9 @@ int sdq_sdpa_batched(const float* q, int64_t ldq, const float* k, int64_t ldk, c
   // other, so that each call's scratch is its own until the next begins.
   float* scratch = nullptr;
   std::unique_lock<std::mutex> turn;
-  const int64_t need = sdpa_packed_bytes(Lq, Lk, heads, batch, cu_count);
+  const int splits = sdpa::few_splits(Lq, Lk, heads, cu_count);
+  const int64_t few = splits > 1 ? sdpa::few_scratch(Lq, heads, splits, batch) : 0;
+  const int64_t need = few ? few : sdpa_packed_bytes(Lq, Lk, heads, batch, cu_count);
   if (need > 0) {
     std::unique_lock<std::mutex> lk(g_mu);
     Workspace& ws = ws_of(dev, s);
@@ -1905,7 +1908,10 @@ int sdq_sdpa_batched(const float* q, int64_t ldq, const float* k, int64_t ldk, c
   }
   hipEvent_t p0 = t_prof ? prof_mark(s) : nullptr;
   const hipError_t e =
-      scratch ? launch_sdpa_packed(q, ldq, k, ldk, v, ldv, out, ldo, Lq, Lk, heads, s, batch,
+      scratch && few
+          ? launch_sdpa_few(q, ldq, k, ldk, v, ldv, out, ldo, Lq, Lk, heads, s, batch, scratch, few,
+                            splits)
+      : scratch ? launch_sdpa_packed(q, ldq, k, ldk, v, ldv, out, ldo, Lq, Lk, heads, s, batch,
                                    scratch, need, cu_count)
               : launch_sdpa(q, ldq, k, ldk, v, ldv, out, ldo, Lq, Lk, heads, s, batch);
   if (e != hipSuccess) {

@@ -15,6 +15,7 @@
 #include <type_traits>
 #include "sdq_rowblock.h"
 #include "sdq_rowsum.h"
+#include "sdq_sdpa_plan.h"
 
 #pragma clang fp contract(off)
 
@@ -473,9 +474,11 @@ hipError_t launch_resid2(float* x, int64_t M, int64_t N, const ResidStep& a, con
 
 // ---------------------------------------------------------------------------
 // Scaled dot-product attention (src/model/blocks.cpp:112-199, non-causal)
-// without scratch memory: what sdq_sdpa runs where the packed form of
-// sdq_sdpa.hip cannot have its own (a stream that captures a graph before
-// its workspace has grown, no device memory left).
+// without packed keys and values: what sdq_sdpa runs for few queries over many
+// keys (SPLIT: one pass over K and V costs less than packing them first; see
+// sdpa::few_splits) and where the packed form of sdq_sdpa.hip cannot have its
+// scratch (a stream that captures a graph before its workspace has grown, no
+// device memory left).
 // out[i, head] = softmax_j(q_i . k_j / sqrt(hd)) v_j, head_dim 128: the
 // scores as three fp16 products per fp32 product on v_mfma_f32_32x32x16_f16
 // (the softmax's exponential would amplify any error in them: each q and k
@@ -483,7 +486,9 @@ hipError_t launch_resid2(float* x, int64_t M, int64_t N, const ResidStep& a, con
 // split as x = hi + lo, hi = fp16(x), lo = fp16(x - hi), and q.k taken as
 // hi.hi + hi.lo + lo.hi, ~2^-22 relative per product; the powers of two come
 // back out exactly in fp32), P.V as three bf16 products per fp32 product on
-// v_mfma_f32_32x32x16_bf16 (~2^-17 relative, P in [0, 1]), an online softmax
+// v_mfma_f32_32x32x16_bf16 (~2^-17 relative, P in [0, 1]; SPLIT: as six
+// products of three parts each, ~2^-26, in the time of its waits for memory), an
+// online softmax
 // (running max and sum per query, the accumulator rescaled when the max
 // moves), fp32 accumulation. The reference sums in a fixed serial order, so
 // results agree within 2e-5 of the output scale, not bit for bit.
@@ -565,11 +570,24 @@ __device__ __forceinline__ float half_wave_max(float v) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-template <int NW>
+// SPLIT: workgroup z of the grid takes key blocks [z kbs, (z + 1) kbs) and
+// leaves its unnormalized output and its (max, sum) state;
+// sdpa_merge_kernel combines them.
+struct SdpaPart {
+  float* o;      // [splits][rows][heads * 128]: sum of p v
+  float2* ml;    // [splits][rows][heads]: (running max, sum of p), base 2
+  int64_t rows;  // batch * Lq
+  int heads;
+  int kbs;
+};
+
+template <int NW, bool SPLIT>
 __global__ void __launch_bounds__(NW * 64)
 sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ K, int64_t ldk,
             const float* __restrict__ V, int64_t ldv, float* __restrict__ O, int64_t ldo,
-            int64_t Lq, int64_t Lk, int qgroups, float scale_log2e) {
+            int64_t Lq, int64_t Lk, int qgroups, float scale_log2e, SdpaPart part) {
+  constexpr int VP = SPLIT ? 3 : 2;  // parts of P and V
+  constexpr int VB = SPLIT ? 1 : 2;  // V buffers (three parts, twice: one workgroup per CU)
   // Sequence blockIdx.y of a batch: its Lq query rows and Lk key rows follow
   // the previous sequence's (stacked rows, attention stays inside each).
   Q += (int64_t)blockIdx.y * Lq * ldq;
@@ -582,17 +600,17 @@ sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ 
   __shared__ __attribute__((aligned(16))) _Float16 ksh[2][kKB][kKPadH];
   __shared__ __attribute__((aligned(16))) _Float16 ksl[2][kKB][kKPadH];
   __shared__ __attribute__((aligned(16))) float kexp[3][kKB];
-  // V^T as bf16 hi and lo parts, two keys per dword, keys of each 16-key
+  // V^T as bf16 parts, two keys per dword, keys of each 16-key
   // group stored in the order 0-3, 8-11, 4-7, 12-15 (lane half h then reads
   // its 8 keys of a PV step as one 16-byte run)
-  __shared__ __attribute__((aligned(16))) uint32_t vth[2][kHd][kVPd];
-  __shared__ __attribute__((aligned(16))) uint32_t vtl[2][kHd][kVPd];
+  __shared__ __attribute__((aligned(16))) uint32_t vt[VP][VB][kHd][kVPd];
   constexpr int NT = NW * 64;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int head = blockIdx.x / qgroups, qg = blockIdx.x - head * qgroups;
   const int64_t q0 = ((int64_t)qg * NW + w) * 32;
   const int j = lane & 31, h = lane >> 5;
   const int64_t col = (int64_t)head * kHd;
+  const int64_t kb0 = SPLIT ? (int64_t)blockIdx.z * part.kbs : 0;
 
   // this lane's query row, dims 64h .. 64h+63, scaled by 2^-e (the row's
   // largest element in [0.5, 1)) and split into fp16 parts for the 8 MFMA
@@ -644,7 +662,7 @@ sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ 
 #pragma unroll
     for (int c = 0; c < PER; c++) {
       const int f = tid + c * NT;
-      const int64_t kr = kb * kKB + (f >> 5);
+      const int64_t kr = (kb0 + kb) * kKB + (f >> 5);
       pk[c] = f < kKB * kHd / 4 && kr < Lk
                   ? *reinterpret_cast<const float4*>(K + kr * ldk + col + 4 * (f & 31))
                   : float4{0.f, 0.f, 0.f, 0.f};
@@ -655,7 +673,8 @@ sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ 
     for (int c = 0; c < PERV; c++) {
       const int f = tid + c * NT;
       const int kp = f & 15, d4 = 2 * (f >> 5) + ((f >> 4) & 1);
-      const int64_t k0 = kb * kKB + pos_key(2 * kp), k1 = kb * kKB + pos_key(2 * kp + 1);
+      const int64_t k0 = (kb0 + kb) * kKB + pos_key(2 * kp);
+      const int64_t k1 = (kb0 + kb) * kKB + pos_key(2 * kp + 1);
       const bool okf = f < kKB / 2 * kHd / 4;
       pv0[c] = okf && k0 < Lk ? *reinterpret_cast<const float4*>(V + k0 * ldv + col + 4 * d4)
                               : float4{0.f, 0.f, 0.f, 0.f};
@@ -682,12 +701,12 @@ sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ 
       if ((f & 31) == 0) kexp[slot][f >> 5] = ldexpf(1.f, ek);
     }
   };
-  // x -> (bf16(x), bf16(x - bf16(x))) for the two keys of a dword
-  auto split2 = [](float x0, float x1, uint32_t& hi, uint32_t& lo) {
+  // the next bf16 part of the two keys of a dword, taken off x0 and x1
+  auto part2 = [](float& x0, float& x1) {
     const __bf16 h0 = (__bf16)x0, h1 = (__bf16)x1;
-    const __bf16 l0 = (__bf16)(x0 - (float)h0), l1 = (__bf16)(x1 - (float)h1);
-    hi = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-    lo = (uint32_t)__builtin_bit_cast(uint16_t, l0) | ((uint32_t)__builtin_bit_cast(uint16_t, l1) << 16);
+    x0 -= (float)h0, x1 -= (float)h1;
+    return (uint32_t)__builtin_bit_cast(uint16_t, h0) |
+           ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
   };
   auto stash_v = [&](int b) {
 #pragma unroll
@@ -695,15 +714,12 @@ sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ 
       const int f = tid + c * NT;
       if (f < kKB / 2 * kHd / 4) {
         const int kp = f & 15, d = 4 * (2 * (f >> 5) + ((f >> 4) & 1));
-        const float a0[4] = {pv0[c].x, pv0[c].y, pv0[c].z, pv0[c].w};
-        const float a1[4] = {pv1[c].x, pv1[c].y, pv1[c].z, pv1[c].w};
+        float a0[4] = {pv0[c].x, pv0[c].y, pv0[c].z, pv0[c].w};
+        float a1[4] = {pv1[c].x, pv1[c].y, pv1[c].z, pv1[c].w};
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          uint32_t hi, lo;
-          split2(a0[e], a1[e], hi, lo);
-          vth[b][d + e][kp] = hi;
-          vtl[b][d + e][kp] = lo;
-        }
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int p = 0; p < VP; p++) vt[p][b % VB][d + e][kp] = part2(a0[e], a1[e]);
       }
     }
   };
@@ -728,7 +744,8 @@ sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ 
 #pragma unroll
   for (int t = 0; t < 4; t++) acc[t] = v16f{};
   float m = -INFINITY, lsum = 0.f;
-  const int64_t nkb = (Lk + kKB - 1) / kKB;
+  int64_t nkb = (Lk + kKB - 1) / kKB - kb0;
+  if (SPLIT && nkb > part.kbs) nkb = part.kbs;
   // prologue: K(0) -> scores; then K(1) and V(0) staged
   fetch_k(0);
   stash_k(0, 0);
@@ -750,7 +767,8 @@ sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ 
     // 2^-e_k, put back here); keys past Lk are -inf.
     // v_exp_f32 flushes results below 2^-126 to 0, which moves a row sum
     // that holds a 1 (the max) by less than 2^-121.
-    const int rem = Lk - kb * kKB < kKB ? (int)(Lk - kb * kKB) : kKB;
+    const int64_t left = Lk - (kb0 + kb) * kKB;
+    const int rem = left < kKB ? (int)left : kKB;
     float t[16];
     float mloc = -INFINITY;
     const float* kf = kexp[(int)(kb % 3)];
@@ -788,33 +806,40 @@ sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ 
     // O^T += V^T . P^T on the bf16 MFMA (32x32x16), each product split as
     // V_hi.P_hi + V_hi.P_lo + V_lo.P_hi (x_hi = bf16(x), x_lo = bf16(x - x_hi):
     // ~2^-17 relative per product, fp32 accumulation; P is in [0, 1], so no
-    // exponential amplifies it). Step s2 takes keys 16 s2 + 8(m/4) + 4h + m%4,
+    // exponential amplifies it), with three parts the three products of 2^-18
+    // as well. Step s2 takes keys 16 s2 + 8(m/4) + 4h + m%4,
     // m = 0..7, exactly the lane's P registers t[8 s2 + m] and its two V^T
     // float4s at keys 16 s2 + 4h and 16 s2 + 8 + 4h.
 #pragma unroll
     for (int s2 = 0; s2 < 2; s2++) {
-      v8bf ph, pl;
+      v8bf p[VP];
 #pragma unroll
       for (int m = 0; m < 8; m++) {
-        const float x = t[8 * s2 + m];
-        const __bf16 hb = (__bf16)x;
-        ph[m] = hb;
-        pl[m] = (__bf16)(x - (float)hb);
+        float x = t[8 * s2 + m];
+#pragma unroll
+        for (int i = 0; i < VP; i++) {
+          p[i][m] = (__bf16)x;
+          x -= (float)p[i][m];
+        }
       }
 #pragma unroll
       for (int tt = 0; tt < 4; tt++) {
         const int dq = 8 * s2 + 4 * h;  // dword of stored position 16 s2 + 8h
-        const v8bf vh = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4*>(&vth[b][32 * tt + j][dq]));
-        const v8bf vl = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4*>(&vtl[b][32 * tt + j][dq]));
-        acc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, ph, acc[tt], 0, 0, 0);
-        acc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, pl, acc[tt], 0, 0, 0);
-        acc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vl, ph, acc[tt], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < VP; i++) {
+          const v8bf v = __builtin_bit_cast(
+              v8bf, *reinterpret_cast<const uint4*>(&vt[i][b % VB][32 * tt + j][dq]));
+#pragma unroll
+          for (int k = 0; k + i < VP; k++)
+            acc[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v, p[k], acc[tt], 0, 0, 0);
+        }
       }
     }
     // K(kb+2) into the buffer K(kb) left before the last barrier; V(kb+1)
     // into the one V(kb-1) left. Kept after the P.V MFMAs: hoisted into the
     // softmax, the stash's work would wait there for this iteration's loads.
     __builtin_amdgcn_sched_barrier(0);
+    if (VB == 1) __syncthreads();  // V(kb) has been read by all
     stash_k(b, (int)((kb + 2) % 3));
     stash_v(b ^ 1);
     st = sn;
@@ -823,6 +848,20 @@ sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ 
   // out[query][dim]: lane holds dims 32tt + 8(r/4) + 4h + r%4 of query j
   const float ltot = pair32_sum(lsum);
   const int64_t qi = q0 + j;
+  if constexpr (SPLIT) {
+    if (qi < Lq) {
+      const int64_t row = (int64_t)blockIdx.z * part.rows + (int64_t)blockIdx.y * Lq + qi;
+      float* dst = part.o + row * part.heads * kHd + col;
+#pragma unroll
+      for (int tt = 0; tt < 4; tt++)
+#pragma unroll
+        for (int g = 0; g < 4; g++)
+          *reinterpret_cast<float4*>(dst + 32 * tt + 8 * g + 4 * h) =
+              float4{acc[tt][4 * g], acc[tt][4 * g + 1], acc[tt][4 * g + 2], acc[tt][4 * g + 3]};
+      if (h == 0) part.ml[row * part.heads + head] = float2{m, ltot};
+    }
+    return;
+  }
   const float inv = 1.f / ltot;
   if (qi < Lq) {
     float* dst = O + qi * ldo + col;
@@ -837,7 +876,66 @@ sdpa_kernel(const float* __restrict__ Q, int64_t ldq, const float* __restrict__ 
   }
 }
 
+// out[row][head dims] = sum_s w_s o_s / sum_s w_s l_s, w_s = 2^(m_s - max m).
+// One thread per 4 dims.
+__global__ void __launch_bounds__(256)
+sdpa_merge_kernel(SdpaPart part, int splits, float* __restrict__ O, int64_t ldo) {
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t per_row = (int64_t)part.heads * (kHd / 4);
+  if (idx >= part.rows * per_row) return;
+  const int64_t row = idx / per_row;
+  const int rem = (int)(idx - row * per_row);
+  const int head = rem / (kHd / 4), d4 = rem - head * (kHd / 4);
+  const float2* ml = part.ml + row * part.heads + head;
+  const int64_t step = part.rows * part.heads;  // between two splits' states
+  float mx = -INFINITY;
+  for (int s = 0; s < splits; s++) mx = fmaxf(mx, ml[s * step].x);
+  float lt = 0.f;
+  float4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int s = 0; s < splits; s++) {
+    const float2 x = ml[s * step];
+    const float w = __builtin_amdgcn_exp2f(x.x - mx);
+    lt += w * x.y;
+    const float4 v = *reinterpret_cast<const float4*>(
+        part.o + ((s * part.rows + row) * part.heads + head) * kHd + 4 * d4);
+    o.x += w * v.x;
+    o.y += w * v.y;
+    o.z += w * v.z;
+    o.w += w * v.w;
+  }
+  const float inv = 1.f / lt;
+  *reinterpret_cast<float4*>(O + row * ldo + (int64_t)head * kHd + 4 * d4) =
+      float4{o.x * inv, o.y * inv, o.z * inv, o.w * inv};
+}
+
 }  // namespace
+
+hipError_t launch_sdpa_few(const float* q, int64_t ldq, const float* k, int64_t ldk,
+                           const float* v, int64_t ldv, float* out, int64_t ldo, int64_t Lq,
+                           int64_t Lk, int heads, hipStream_t s, int batch, void* scratch,
+                           int64_t scratch_bytes, int splits) {
+  const int64_t one = sdpa::few_bytes(Lq, heads, splits);
+  if (Lq <= 0 || Lq > 64 || Lk <= 0 || heads <= 0 || batch <= 0 || splits < 2 || !scratch ||
+      one > scratch_bytes)
+    return hipErrorInvalidValue;
+  const float scale_log2e = (1.f / sqrtf((float)kHd)) * 1.4426950408889634f;
+  const int64_t chunk = std::min<int64_t>(std::min<int64_t>(scratch_bytes / one, batch), 65535);
+  for (int64_t b = 0; b < batch; b += chunk) {
+    const int n = (int)std::min<int64_t>(chunk, batch - b);
+    SdpaPart p{static_cast<float*>(scratch), nullptr, n * Lq, heads,
+               (int)ceil_div(ceil_div(Lk, kKB), splits)};
+    p.ml = reinterpret_cast<float2*>(p.o + splits * p.rows * heads * kHd);
+    float* ob = out + b * Lq * ldo;
+    hipLaunchKernelGGL((sdpa_kernel<2, true>), dim3((unsigned)heads, (unsigned)n, (unsigned)splits),
+                       dim3(128), 0, s, q + b * Lq * ldq, ldq, k + b * Lk * ldk, ldk,
+                       v + b * Lk * ldv, ldv, ob, ldo, Lq, Lk, 1, scale_log2e, p);
+    hipLaunchKernelGGL(sdpa_merge_kernel, dim3((unsigned)ceil_div(p.rows * heads * (kHd / 4), 256)),
+                       dim3(256), 0, s, p, splits, ob, ldo);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
 
 hipError_t launch_sdpa(const float* q, int64_t ldq, const float* k, int64_t ldk, const float* v,
                        int64_t ldv, float* out, int64_t ldo, int64_t Lq, int64_t Lk, int heads,
@@ -850,11 +948,11 @@ hipError_t launch_sdpa(const float* q, int64_t ldq, const float* k, int64_t ldk,
   const int qgroups = (int)ceil_div(Lq, 32 * nw);
   const dim3 grid((unsigned)(qgroups * heads), (unsigned)batch);
   if (nw == 8)
-    hipLaunchKernelGGL((sdpa_kernel<8>), grid, dim3(512), 0, s, q, ldq, k, ldk, v, ldv, out, ldo,
-                       Lq, Lk, qgroups, scale_log2e);
+    hipLaunchKernelGGL((sdpa_kernel<8, false>), grid, dim3(512), 0, s, q, ldq, k, ldk, v, ldv, out,
+                       ldo, Lq, Lk, qgroups, scale_log2e, SdpaPart{});
   else
-    hipLaunchKernelGGL((sdpa_kernel<2>), grid, dim3(128), 0, s, q, ldq, k, ldk, v, ldv, out, ldo,
-                       Lq, Lk, qgroups, scale_log2e);
+    hipLaunchKernelGGL((sdpa_kernel<2, false>), grid, dim3(128), 0, s, q, ldq, k, ldk, v, ldv, out,
+                       ldo, Lq, Lk, qgroups, scale_log2e, SdpaPart{});
   return hipGetLastError();
 }
 

@@ -187,6 +187,12 @@ hipError_t launch_linear_f32(const float* x, int64_t M, int64_t K, const float* 
 hipError_t launch_sdpa(const float* q, int64_t ldq, const float* k, int64_t ldk, const float* v,
                        int64_t ldv, float* out, int64_t ldo, int64_t Lq, int64_t Lk, int heads,
                        hipStream_t s, int batch);
+// The same for at most 64 queries (few_splits > 1 in sdq_sdpa_plan.h), keys cut
+// into `splits` ranges; scratch for one sequence's partial outputs at least.
+hipError_t launch_sdpa_few(const float* q, int64_t ldq, const float* k, int64_t ldk,
+                           const float* v, int64_t ldv, float* out, int64_t ldo, int64_t Lq,
+                           int64_t Lk, int heads, hipStream_t s, int batch, void* scratch,
+                           int64_t scratch_bytes, int splits);
 // The same attention with scratch memory of sdpa_packed_bytes bytes (0: the
 // shape is outside that form): K and V split and packed once, then read by
 // every workgroup as they are. cu_count: the device's CUs.

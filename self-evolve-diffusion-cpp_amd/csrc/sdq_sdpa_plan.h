@@ -144,5 +144,42 @@ inline int64_t scratch_bytes(int64_t Lq, int64_t Lk, int heads, int batch, int c
   return most;
 }
 
+// Few queries over many keys (at most 64 over more than kFewKeys): packing K and
+// V moves them three times where one pass reads them once, so that pass takes
+// less, cut into this many key ranges (1: the packed form). us, 24 heads, 64
+// queries, packed / one pass: 4096 keys 64 / 67, 8192 116-126 / 101, 20000 303 /
+// 197, 27280 450-470 / 258. More queries need a pass per 64: 157 queries over 8192
+// keys 133 / 195.
+constexpr int64_t kFewKeys = 4096;
+inline int few_splits(int64_t Lq, int64_t Lk, int heads, int cu_count) {
+  if (Lq > 64 || Lk <= kFewKeys || heads > 65535) return 1;
+  const int64_t nkb = div_up(Lk, kKB);
+  if (const char* forced = std::getenv("SDQ_SDPA_SPLIT")) {  // for comparisons
+    const int f = std::atoi(forced);
+    return f < 2 ? 1 : (int)div_up(nkb, div_up(nkb, f < 16 ? f : 16));
+  }
+  // the fewest rounds of workgroups (two per CU) per unit of work, no empty range
+  const int64_t slots = 2 * (int64_t)(cu_count > 0 ? cu_count : 256);
+  int best = 1;
+  double best_cost = 0.9 * (double)div_up(heads, slots);
+  for (int S = 2; S <= 32; S++) {
+    if (div_up(nkb, div_up(nkb, S)) != S) continue;
+    const double cost = (double)div_up((int64_t)heads * S, slots) / S;
+    if (cost < best_cost) best_cost = cost, best = S;
+  }
+  return best;
+}
+// Scratch of one sequence's partial outputs, and of a call's: sequences run in
+// turns of as many as fit kMaxScratch.
+inline int64_t few_bytes(int64_t Lq, int heads, int splits) {
+  return splits * Lq * heads * (kHd + 2) * 4;
+}
+inline int64_t few_scratch(int64_t Lq, int heads, int splits, int batch) {
+  const int64_t one = few_bytes(Lq, heads, splits);
+  if (one > kMaxScratch) return 0;
+  const int64_t n = kMaxScratch / one;
+  return one * (n < batch ? n : batch);
+}
+
 }  // namespace sdpa
 }  // namespace sdq

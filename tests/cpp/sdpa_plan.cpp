@@ -14,6 +14,15 @@ namespace sd = sdq::sdpa;
 namespace {
 
 bool check(int64_t Lq, int64_t Lk, int heads, int batch, int cus) {
+  if (const int S = sd::few_splits(Lq, Lk, heads, cus); S > 1) {
+    const int64_t nkb = sd::div_up(Lk, sd::kKB), b = sd::few_scratch(Lq, heads, S, batch);
+    if (S > 32 || sd::div_up(nkb, sd::div_up(nkb, S)) != S || b > sd::kMaxScratch ||
+        (b && b < sd::few_bytes(Lq, heads, S))) {
+      std::printf("few queries: Lq=%lld Lk=%lld heads=%d: %d ranges, %lld bytes\n", (long long)Lq,
+                  (long long)Lk, heads, S, (long long)b);
+      return false;
+    }
+  }
   const int64_t have = sd::scratch_bytes(Lq, Lk, heads, batch, cus);
   if (have == 0) return true;
   auto bad = [&](const char* what, int64_t a, int64_t b) {

@@ -98,11 +98,11 @@ def test_value_range(sdq_dev, case):
     assert err <= bound
 
 
-@pytest.mark.parametrize("Lk", [300, 1024, 5000])
+@pytest.mark.parametrize("Lq,Lk", [(70, 300), (70, 1024), (70, 5000), (60, 5000)])
 @pytest.mark.parametrize("cut", [True, False])
 @pytest.mark.parametrize("case", ["falling", "rising", "far_rows", "light_keys", "ignored",
                                   "outlier_dim", "outlier_element", "short_keys"])
-def test_value_magnitudes(sdq_dev, monkeypatch, case, cut, Lk):
+def test_value_magnitudes(sdq_dev, monkeypatch, case, cut, Lq, Lk):
     """V of 2^40 and 2^-90, by halves with blocks of zeros in either order and
     row by row (the small keys count in the softmax's sum all the same); keys
     of 2^-20 of the weight whose V is 2^20 times larger; keys of no weight whose
@@ -111,12 +111,12 @@ def test_value_magnitudes(sdq_dev, monkeypatch, case, cut, Lk):
     its own scale, with the keys cut into shares and not."""
     import torch
 
-    print(f"[sdpa-packed] magnitudes {case} Lk={Lk} cut={cut}", flush=True)
+    print(f"[sdpa-packed] magnitudes {case} Lq={Lq} Lk={Lk} cut={cut}", flush=True)
     if not cut:
         monkeypatch.setenv("SDQ_SDPA_SPLIT", "1")
     g = torch.Generator(device=sdq_dev)
     g.manual_seed(9)
-    Lq, heads = 70, 2
+    heads = 2
     C = heads * 128
     q = torch.randn((Lq, C), generator=g, device=sdq_dev)
     kv = torch.randn((Lk, 2 * C), generator=g, device=sdq_dev)
@@ -149,6 +149,31 @@ def test_value_magnitudes(sdq_dev, monkeypatch, case, cut, Lk):
     err = ((got - want).abs().amax(0) / want.abs().amax(0)).max()
     print(f"  max err of a dimension {float(err):.3e}", flush=True)
     assert err <= 2e-5
+
+
+@pytest.mark.parametrize("Lq,Lk,heads", [(1, 4097, 1), (31, 4128, 5), (33, 8191, 3),
+                                         (64, 4129, 24), (64, 20001, 2), (65, 4129, 2),
+                                         (64, 4096, 2)])
+def test_few_queries(sdq_dev, Lq, Lk, heads):
+    """At most 64 queries over more than 4096 keys: key ranges that end in a
+    partial block, partial and whole query groups, and two stacked sequences
+    with the bits of two separate calls. To the packed form's precision."""
+    import torch
+
+    print(f"[sdpa-packed] few Lq={Lq} Lk={Lk} heads={heads}", flush=True)
+    g = torch.Generator(device=sdq_dev)
+    g.manual_seed(Lq + Lk)
+    q = torch.randn((2 * Lq, 128 * heads), generator=g, device=sdq_dev)
+    kv = torch.randn((2 * Lk, 256 * heads), generator=g, device=sdq_dev)
+    both = _run(sdq_dev, q, kv, heads, batch=2)
+    for b in range(2):
+        qs, ks = q[b * Lq:(b + 1) * Lq], kv[b * Lk:(b + 1) * Lk]
+        one = _run(sdq_dev, qs, ks, heads)
+        assert torch.equal(both[b * Lq:(b + 1) * Lq], one)
+        want = _want64(qs, ks, heads)
+        err = float((one.double() - want).norm() / want.norm())
+        print(f"  err {err:.3e}", flush=True)
+        assert err <= 2e-6  # float sums of up to 20001 terms; the two-part products alone 4e-6
 
 
 def test_chunks(sdq_dev):
