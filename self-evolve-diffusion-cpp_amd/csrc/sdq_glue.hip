@@ -222,13 +222,14 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 bool rms_rows_fits(const RmsSeg* segs, int nseg, int64_t C, int heads) {
   bool rows = C % 4 == 0 && C <= rowblock::kMaxCols && C / heads % 4 == 0;
-  int64_t blocks = 0;
+  int64_t blocks = 0, total = 0;
   for (int i = 0; i < nseg; i++) {
     const RmsSeg& g = segs[i];
-    blocks += ceil_div(g.L, rowblock::kRows);
+    blocks += ceil_div(g.L, rowblock::kRows), total += g.L;
     rows = rows && aligned16(g.x) && g.ld % 4 == 0 && (g.L == 0 || (g.w && aligned16(g.w)));
   }
-  return rows && blocks <= rowblock::kMaxBlocks;
+  return rows && blocks <= rowblock::kMaxBlocks &&
+         (C >= rowblock::kNarrowRms || total <= rowblock::kManyRows);
 }
 
 hipError_t launch_rmsnorm_rope_segs(const RmsSeg* segs, int nseg, int64_t C, int heads, float eps,
@@ -420,6 +421,7 @@ bus_copy_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, uint32_t
 bool ln_rows_fits(const float* x, int64_t M, int64_t K, const float* w, const float* b,
                   const float* y) {
   return K % 4 == 0 && K <= rowblock::kMaxCols &&
+         (K >= rowblock::kNarrowLn || M <= rowblock::kManyRows) &&
          ceil_div(M, rowblock::kRows) <= rowblock::kMaxBlocks && aligned16(x) && aligned16(y) &&
          aligned16(w) && aligned16(b);
 }

@@ -37,6 +37,13 @@ constexpr int64_t kMaxCols = kMaxChunks * kChunk;
 // Workgroups of one launch: a grid holds fewer than 2^32 threads. (The two-kernel
 // form, 8 threads per row, goes on beyond.)
 constexpr int64_t kMaxBlocks = ((int64_t(1) << 32) - 1) / kThreads;
+// Many narrow rows stay with the two-kernel form: a workgroup adds 512 columns
+// whatever the row's width. us, two kernels / one pass, 200000 rows: layernorm
+// of 4 columns 62 / 97, of 20 80 / 99, of 28 102 / 100; rmsnorm + RoPE of 4
+// columns 35 / 75, of 48 65 / 79, of 64 94 / 79. 60000 rows of 4: 25 / 34 and
+// 19 / 26; 27280: 19 / 18 and 18 / 15.
+constexpr int64_t kManyRows = 32768;
+constexpr int64_t kNarrowLn = 28, kNarrowRms = 64;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 

@@ -156,3 +156,26 @@ def test_more_rows_than_one_grid_holds(sdq_dev):
         want = x[r].contiguous()
         sdq.rmsnorm_rope_batch([(want, 0, w, cs[:99].contiguous())], K, 1)
         assert torch.equal(y[r], want)
+
+
+@pytest.mark.parametrize("M,K", [(32768, 4), (32769, 4), (32769, 24), (32769, 28), (32769, 60),
+                                 (32769, 64)])
+def test_many_narrow_rows(sdq_dev, oracle, M, K):
+    """Both sides of the row count and widths where the two-kernel form takes
+    over, bit-exact against the oracle."""
+    import torch
+
+    import sdq
+
+    print(f"[rowblock] narrow M={M} K={K}", flush=True)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(sdq_dev)  # noqa: E731
+    x = _x(oracle, M, K, K)
+    w, b = oracle.randn(K, 11), oracle.randn(K, 12)
+    y = torch.empty((M, K), device=sdq_dev)
+    sdq.layernorm(t(x), y, t(w), t(b), 1e-6)
+    d = t(x)
+    cs = oracle.rope_cs(np.random.default_rng(5).uniform(-3, 3, (M, 2)).astype(np.float32))
+    sdq.rmsnorm_rope_batch([(d, 0, t(w), t(cs))], K, 1)
+    torch.cuda.synchronize()
+    assert_bitexact(y.cpu().numpy(), oracle.layernorm(x, 1e-6, w, b), "layernorm")
+    assert_bitexact(d.cpu().numpy(), oracle.rope(oracle.rmsnorm(x, w, 1e-6), cs, 1), "rms + rope")
