@@ -371,11 +371,13 @@ int sdq_qgemm(const sdq_weight* w, const float* A, int64_t M, int64_t K, float* 
 /* Host-pointer synchronous variant of sdq_qlinear: copies A (and bias /
  * gate / resid) in, runs, copies Y out. Replaces sd::qgemm's host-tensor
  * contract (tensor.h:52) for callers that hold CPU tensors. Each calling
- * thread keeps, per device, a stream of its own, two 16 MiB pinned bounce
- * buffers and a device buffer that grows to the largest call's inputs and
- * output; they are reused by its later calls (no allocation once grown) and
- * are not released when the thread exits, so call it from long-lived
- * threads. */
+ * thread keeps, per device, up to four slots, each an 8 MiB pinned buffer and
+ * a device block that grows with the calls, on two streams of its own with a
+ * workspace each; a call goes through them in pieces of rows. Rows too long for
+ * a slot, and an output that lies on an input, go whole: the first device block
+ * then grows to the call's inputs and output. Slots are reused by later calls
+ * (no allocation once grown) and are not released when the thread exits, so
+ * call it from long-lived threads. */
 int sdq_qlinear_host(const sdq_weight* w, const float* A, int64_t M, int64_t K,
                      const sdq_epilogue* epi, void* Y);
 

@@ -14,7 +14,7 @@
 // queries, a third of its VALU work; here one pass does it once, in the order
 // the MFMAs read, so that LDS-DMAs move the blocks as they are and the loop
 // holds MFMAs, LDS reads and the softmax only. 27280^2, 24 heads: 30.2 ms
-// without, 19.3-19.7 ms with it (0.24 ms of that the packing); MFMAs 16x16x32:
+// without, 19.5-20.3 ms with it (0.25 ms of that the packing); MFMAs 16x16x32:
 // 32x32x16 ones took 20.7 ms (fewer accumulator bits switch, a higher clock).
 #include "sdq_internal.h"
 #include "sdq_device.h"
