@@ -11,6 +11,7 @@
 // std::cos / std::sin of float angles).
 #include "sdq_internal.h"
 
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 #include "sdq_rowblock.h"
@@ -222,14 +223,13 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 bool rms_rows_fits(const RmsSeg* segs, int nseg, int64_t C, int heads) {
   bool rows = C % 4 == 0 && C <= rowblock::kMaxCols && C / heads % 4 == 0;
-  int64_t blocks = 0, total = 0;
+  int64_t total = 0;
   for (int i = 0; i < nseg; i++) {
     const RmsSeg& g = segs[i];
-    blocks += ceil_div(g.L, rowblock::kRows), total += g.L;
+    total += g.L;
     rows = rows && aligned16(g.x) && g.ld % 4 == 0 && (g.L == 0 || (g.w && aligned16(g.w)));
   }
-  return rows && blocks <= rowblock::kMaxBlocks &&
-         (C >= rowblock::kNarrowRms || total <= rowblock::kManyRows);
+  return rows && !rowblock::narrow(total, C, rowblock::kNarrowRms, total * C / 2);
 }
 
 hipError_t launch_rmsnorm_rope_segs(const RmsSeg* segs, int nseg, int64_t C, int heads, float eps,
@@ -255,12 +255,24 @@ hipError_t launch_rmsnorm_rope_segs(const RmsSeg* segs, int nseg, int64_t C, int
   }
   full = full && vec;
   if (rows) {
-    for (int i = 0; i < nseg; i++)
-      st.blk0[i + 1] = st.blk0[i] + ceil_div(segs[i].L, rowblock::kRows);
-    if (st.blk0[nseg] == 0) return hipSuccess;
+    // in turns of as many rows of each segment as one grid holds of all
+    const int64_t turn = rowblock::kMaxRows / kMaxRmsSegs / rowblock::kRows * rowblock::kRows;
+    int64_t most = 0;
+    for (int i = 0; i < nseg; i++) most = std::max(most, segs[i].L);
+    if (most == 0) return hipSuccess;
     return rowblock::for_cols(C, [&](auto nc) {
-      hipLaunchKernelGGL((rms_rope_rows_kernel<decltype(nc)::value>), dim3((unsigned)st.blk0[nseg]),
-                         dim3(rowblock::kThreads), 0, s, st, (int)C, (int)(C / heads), eps);
+      for (int64_t r = 0; r < most; r += turn) {
+        for (int i = 0; i < nseg; i++) {
+          const RmsSeg& g = segs[i];
+          const int64_t n = std::max<int64_t>(0, std::min(g.L - r, turn));
+          st.s[i] = RmsSeg{n ? g.x + r * g.ld : g.x, n, g.ld, g.w,
+                           n && g.cs ? g.cs + r * g.nr * 2 : g.cs, g.nr, nullptr};
+          st.blk0[i + 1] = st.blk0[i] + ceil_div(n, rowblock::kRows);
+        }
+        hipLaunchKernelGGL((rms_rope_rows_kernel<decltype(nc)::value>),
+                           dim3((unsigned)st.blk0[nseg]), dim3(rowblock::kThreads), 0, s, st,
+                           (int)C, (int)(C / heads), eps);
+      }
       return hipGetLastError();
     });
   }
@@ -421,8 +433,7 @@ bus_copy_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, uint32_t
 bool ln_rows_fits(const float* x, int64_t M, int64_t K, const float* w, const float* b,
                   const float* y) {
   return K % 4 == 0 && K <= rowblock::kMaxCols &&
-         (K >= rowblock::kNarrowLn || M <= rowblock::kManyRows) &&
-         ceil_div(M, rowblock::kRows) <= rowblock::kMaxBlocks && aligned16(x) && aligned16(y) &&
+         !rowblock::narrow(M, K, rowblock::kNarrowLn, M * K) && aligned16(x) && aligned16(y) &&
          aligned16(w) && aligned16(b);
 }
 
@@ -430,9 +441,12 @@ hipError_t launch_ln_rows(const float* x, int64_t M, int64_t K, const float* w, 
                           float eps, float* y, hipStream_t s) {
   if (M <= 0 || K <= 0) return hipSuccess;
   return rowblock::for_cols(K, [&](auto nc) {
-    hipLaunchKernelGGL((ln_rows_kernel<decltype(nc)::value>),
-                       dim3((unsigned)ceil_div(M, rowblock::kRows)), dim3(rowblock::kThreads), 0, s,
-                       x, M, (int)K, w, b, eps, y);
+    for (int64_t r = 0; r < M; r += rowblock::kMaxRows) {
+      const int64_t n = std::min(M - r, rowblock::kMaxRows);
+      hipLaunchKernelGGL((ln_rows_kernel<decltype(nc)::value>),
+                         dim3((unsigned)ceil_div(n, rowblock::kRows)), dim3(rowblock::kThreads), 0,
+                         s, x + r * K, n, (int)K, w, b, eps, y + r * K);
+    }
     return hipGetLastError();
   });
 }

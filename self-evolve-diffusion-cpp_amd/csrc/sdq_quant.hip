@@ -16,6 +16,7 @@
 // row-major kernel (parity API) on 32-row blocks. Few long rows take a
 // split form instead (per-chunk maxima, then reduce + quantize), so that
 // the whole GPU walks them.
+#include <algorithm>
 #include <cstdlib>
 
 #include "sdq_internal.h"
@@ -714,9 +715,14 @@ hipError_t launch_act_quant_frags_lnmod_rows(const float* A, int64_t M, int64_t 
                                              const float* scale, float eps, hipStream_t s) {
   if (!shift || !scale || K <= 0) return hipErrorInvalidValue;
   return rowblock::for_cols(KFp * 32, [&](auto nc) {
-    hipLaunchKernelGGL((lnmod_quant_rows_kernel<decltype(nc)::value>),
-                       dim3((unsigned)ceil_div(Mp, rowblock::kRows)), dim3(rowblock::kThreads), 0,
-                       s, A, M, Mp, (int)K, (int)KFp, shift, scale, eps, at, as, cc);
+    for (int64_t r = 0; r < Mp; r += rowblock::kMaxRows) {
+      const int64_t n = std::min(Mp - r, rowblock::kMaxRows);
+      const int64_t m = std::max<int64_t>(0, std::min(M - r, n));  // the rest is tile padding
+      hipLaunchKernelGGL((lnmod_quant_rows_kernel<decltype(nc)::value>),
+                         dim3((unsigned)ceil_div(n, rowblock::kRows)), dim3(rowblock::kThreads), 0,
+                         s, m ? A + r * K : A, m, n, (int)K, (int)KFp, shift, scale, eps,
+                         at + r / kFragRows * KFp * kFragBytes, as + r, r ? ColCopy{} : cc);
+    }
     return hipGetLastError();
   });
 }

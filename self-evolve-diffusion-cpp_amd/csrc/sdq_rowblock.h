@@ -34,9 +34,9 @@ constexpr int kThreads = 64 * (kWaves + 1);
 constexpr int kChunk = 256;    // columns per chunk
 constexpr int kMaxChunks = 12;
 constexpr int64_t kMaxCols = kMaxChunks * kChunk;
-// Workgroups of one launch: a grid holds fewer than 2^32 threads. (The two-kernel
-// form, 8 threads per row, goes on beyond.)
-constexpr int64_t kMaxBlocks = ((int64_t(1) << 32) - 1) / kThreads;
+// Rows of one launch (of 32-row fragments); more run as several. A grid of 2^32
+// threads or more wraps without an error.
+constexpr int64_t kMaxRows = ((int64_t(1) << 32) - 1) / kThreads * kRows / 32 * 32;
 // Many narrow rows stay with the two-kernel form: a workgroup adds 512 columns
 // whatever the row's width. us, two kernels / one pass, 200000 rows: layernorm
 // of 4 columns 62 / 97, of 20 80 / 99, of 28 102 / 100; rmsnorm + RoPE of 4
@@ -44,6 +44,11 @@ constexpr int64_t kMaxBlocks = ((int64_t(1) << 32) - 1) / kThreads;
 // 19 / 26; 27280: 19 / 18 and 18 / 15.
 constexpr int64_t kManyRows = 32768;
 constexpr int64_t kNarrowLn = 28, kNarrowRms = 64;
+// (that form: 8 threads per row, then one per value or pair, in one grid each)
+inline bool narrow(int64_t rows, int64_t cols, int64_t below, int64_t threads) {
+  return cols < below && rows > kManyRows && 8 * rows < int64_t(1) << 32 &&
+         threads < int64_t(1) << 32;
+}
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 

@@ -132,29 +132,39 @@ def test_rmsnorm_rope_captures_without_warm_up(sdq_dev, oracle):
         assert torch.equal(x, want), rep
 
 
-def test_more_rows_than_one_grid_holds(sdq_dev):
-    """Rows beyond one launch of 14-row workgroups still run: the last ones
-    equal a call on them alone."""
+@pytest.mark.parametrize("K", [4, 64])
+def test_more_rows_than_one_grid_holds(sdq_dev, oracle, K):
+    """Rows beyond one grid of 14-row workgroups: the first, those at its end and
+    the last equal a call on them alone (4 columns: the two-kernel form)."""
     import torch
 
     import sdq
 
-    M, K = 117_440_512 + 5, 4
+    M, n = 117_440_480 + 45, 99  # one launch's rows (whole 32-row fragments) and some
     print(f"[rowblock] rows M={M} K={K}", flush=True)
+    parts = [slice(0, n), slice(117_440_480 - 60, 117_440_480 - 60 + n), slice(M - n, M)]
     x = torch.randn((M, K), device=sdq_dev)
     w, b = torch.randn(K, device=sdq_dev), torch.randn(K, device=sdq_dev)
+    q, s = oracle.quant_rows(oracle.randn(4 * K, 13).reshape(4, K))
+    lin = sdq.Weight.from_host(q, s)
+    Y, Yn = torch.empty((M, 4), device=sdq_dev), torch.empty((n, 4), device=sdq_dev)
+    sdq.qlinear_lnmod(lin, x, Y, w, b, 1e-6)
+    for r in parts:
+        sdq.qlinear_lnmod(lin, x[r].contiguous(), Yn, w, b, 1e-6)
+        assert torch.equal(Y[r], Yn)
+    del Y
     cs = torch.randn((1, 2, 2), device=sdq_dev).expand(M, 2, 2).contiguous()
     y = torch.empty_like(x)
     sdq.layernorm(x, y, w, b)
-    for r in (slice(0, 99), slice(M - 99, M)):
-        want = torch.empty((99, K), device=sdq_dev)
+    for r in parts:
+        want = torch.empty((n, K), device=sdq_dev)
         sdq.layernorm(x[r].contiguous(), want, w, b)
         assert torch.equal(y[r], want)
     y.copy_(x)
     sdq.rmsnorm_rope_batch([(y, 0, w, cs)], K, 1)
-    for r in (slice(0, 99), slice(M - 99, M)):
-        want = x[r].contiguous()
-        sdq.rmsnorm_rope_batch([(want, 0, w, cs[:99].contiguous())], K, 1)
+    for r in parts:
+        want = x[r].clone()
+        sdq.rmsnorm_rope_batch([(want, 0, w, cs[:n].contiguous())], K, 1)
         assert torch.equal(y[r], want)
 
 
